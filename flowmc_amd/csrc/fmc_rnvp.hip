@@ -3,19 +3,18 @@
 // ([d, hidden, d], ReLU; common.py:68-112, 171-208) read the conditioning
 // dims and drive the transformed dims:
 //   s = tanh(MLP_s(c)) dt,  t = MLP_t(c) dt,  y = (x + t) e^s,  log-det = sum s.
-// The model is FP32 end to end. Its GEMMs are small (d x hidden per sample and
-// layer), and on CDNA4 the FP32 vector FMA rate equals the FP32 MFMA rate, so
-// the products are FP32 FMA register tiles (4 outputs x 4 samples per thread)
-// over LDS-resident activations, with weights read as aligned float4 rows of
-// an L2-resident packed copy. Products with few outputs (the d_t scale / shift
-// rows, the d_c conditioning gradients) split their reduction over the lanes
-// of a wavefront and combine them with xor shuffles.
-//
-// Work mapping: a workgroup of 256 threads owns RN_TS = 16 samples for the
-// whole pass (all layers), activations in LDS (~42 KB at d=32, hidden 256, so
-// three workgroups share a CU). The adjoint runs one layer per launch and
-// writes per-tile weight-gradient partials; a second kernel sums them over
-// tiles in a fixed order and scatters them into the gradient vector.
+// The model is FP32 end to end. The passes run on the FP32 matrix cores
+// (v_mfma_f32_16x16x4: the FP32 vector rate without packed forms is half of
+// it): 409,600 samples at d = 32, 8 layers, hidden 256 drawn in 1.10 ms, 98
+// TFLOP/s, where FMA register tiles over LDS took 4.05 ms; 10,000 in 67 us
+// (213 us). Training (forward with saved inputs, adjoint) uses FP32 FMA
+// register tiles (4 outputs x 4 samples per thread) over LDS-resident
+// activations, with weights read as aligned float4 rows of an L2-resident
+// packed copy; products with few outputs split their reduction over the lanes
+// of a wavefront and combine them with xor shuffles. Its workgroups of 256
+// threads own RN_TS = 16 samples; the adjoint runs one layer per launch and
+// writes per-tile weight-gradient partials, which a second kernel sums over
+// tiles in a fixed order and scatters into the gradient vector.
 #include "fmc_common.h"
 
 namespace fmc {
@@ -64,6 +63,43 @@ struct RnPk {
     W2c = base + 3 * s;
     b1 = base + 4 * s;
     b2c = b1 + h4;
+  }
+};
+// ---- MFMA fragment images, per (layer, p), after the images above. Blocks of
+// 16 conditioning dims (kg < KC), 16 transformed dims (r < R) and 16 hidden
+// features (hb < HB); one 16 x 16 weight block is 64 lanes x float4, lane l
+// (c = l % 16, q = l / 16) holding four k-steps of v_mfma_f32_16x16x4:
+//   W1f [hb][kg]: W1[16 hb + c][cond(16 kg + 4q + e)]
+//   W2f [hb][r]:  W2[trans(16 r + c)][16 hb + 4q + e]
+// (k = 4q + e is also the row a lane's accumulator e holds, so the output
+// block of the first product is the second product's operand as it lies),
+// then b1 [16 HB], b2 [16 R], and the index words {n_cond, n_trans, 0, 0,
+// cond [16 KC], trans [16 R]} (padding entries 0). A slot has a fixed size:
+// KC + R <= ceil(d / 16) + 1 whatever the mask.
+__host__ __device__ inline int rn_b16(int v) { return (v + 15) >> 4; }
+__host__ __device__ inline int64_t rn_fr_slot(int d, int h) {
+  const int kr = rn_b16(d) + 1, hb = rn_b16(h);
+  return 256LL * hb * kr + 16LL * hb + 16LL * rn_b16(d) + 4 + 16LL * kr;
+}
+__host__ __device__ inline int64_t rn_fr_base(int d, int h, int L) { return (2LL * L * rn_pk_mlp(d, h) + 15) & ~15LL; }
+__host__ __device__ inline int64_t rn_packed_size(int d, int h, int L) {
+  return rn_fr_base(d, h, L) + 2LL * L * ((rn_fr_slot(d, h) + 15) & ~15LL);
+}
+struct RnFr {
+  int KC, R, HB;
+  const float *W1f, *W2f, *b1, *b2;
+  const int32_t *nct, *cond, *trans;  // {n_cond, n_trans}, index lists
+  __device__ RnFr(const float* packed, int d, int h, int L, int l, int p, int dc, int dtr) {
+    KC = rn_b16(dc);
+    R = rn_b16(dtr);
+    HB = rn_b16(h);
+    W1f = packed + rn_fr_base(d, h, L) + (2LL * l + p) * ((rn_fr_slot(d, h) + 15) & ~15LL);
+    W2f = W1f + 256LL * HB * KC;
+    b1 = W2f + 256LL * HB * R;
+    b2 = b1 + 16 * HB;
+    nct = reinterpret_cast<const int32_t*>(b2 + 16 * R);
+    cond = nct + 4;
+    trans = cond + 16 * KC;
   }
 };
 // ---- layout: per layer [n_cond, n_trans, cond[d], trans[d]]
@@ -253,6 +289,55 @@ __global__ void __launch_bounds__(256) rnvp_pack_kernel(RnvpDev f, float* packed
   }
 }
 
+// The fragment images of one (layer, p) slot (RnFr): one thread per word.
+__global__ void __launch_bounds__(256) rnvp_pack_frag_kernel(RnvpDev f, float* packed) {
+  const int d = f.d, h = f.h;
+  const int lp = blockIdx.y, l = lp >> 1, p = lp & 1;
+  const int32_t* lay = rn_lay(f, l);
+  const int dc = lay[0], dtr = lay[1];
+  const int32_t* cond = lay + 2;
+  const int32_t* trans = lay + 2 + d;
+  const RnFr fr(packed, d, h, f.L, l, p, dc, dtr);
+  const float* W1 = f.theta + rn_mlp(d, h, l, p);
+  const float* b1 = W1 + (int64_t)h * d;
+  const float* W2 = b1 + h;
+  const float* b2 = W2 + (int64_t)d * h;
+  float* dst = const_cast<float*>(fr.W1f);
+  const int64_t n1 = 256LL * fr.HB * fr.KC, n2 = n1 + 256LL * fr.HB * fr.R, n3 = n2 + 16 * fr.HB, n4 = n3 + 16 * fr.R;
+  const int64_t n5 = n4 + 4, n6 = n5 + 16 * fr.KC, n = n6 + 16 * fr.R;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
+    float v = 0.f;
+    if (e < n2) {
+      const bool first = e < n1;
+      const int64_t r = first ? e : e - n1;
+      const int nb = first ? fr.KC : fr.R;
+      const int hb = (int)(r / (256 * nb)), w = (int)(r - (int64_t)hb * 256 * nb);
+      const int b = w >> 8, lane = (w >> 2) & 63, el = w & 3, c = lane & 15, k = 4 * (lane >> 4) + el;
+      if (first) {
+        const int j = 16 * hb + c, i = 16 * b + k;
+        if (j < h && i < dc) v = W1[(int64_t)j * d + cond[i]];
+      } else {
+        const int i = 16 * b + c, j = 16 * hb + k;
+        if (j < h && i < dtr) v = W2[(int64_t)trans[i] * h + j];
+      }
+    } else if (e < n3) {
+      if (e - n2 < h) v = b1[e - n2];
+    } else if (e < n4) {
+      if (e - n3 < dtr) v = b2[trans[e - n3]];
+    } else {
+      int w = 0;
+      if (e < n5)
+        w = e == n4 ? dc : (e == n4 + 1 ? dtr : 0);
+      else if (e < n6)
+        w = e - n5 < dc ? cond[e - n5] : 0;
+      else
+        w = e - n6 < dtr ? trans[e - n6] : 0;
+      v = __int_as_float(w);
+    }
+    dst[e] = v;
+  }
+}
+
 // -------------------------------------------------------------- passes ---
 struct RnPassArgs {
   int dir;    // 0 forward (realNVP.py:163-180), 1 inverse (:182-198)
@@ -270,7 +355,22 @@ struct RnPassArgs {
 
 enum { RN_STD = 1, RN_BASE = 2, RN_SAMPLE = 4 };
 
-__global__ void __launch_bounds__(RN_THREADS) rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
+template <class K>
+static int rn_set_lds(K kernel, size_t shm) {
+  const hipError_t e =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+  if (e != hipSuccess) {
+    set_error(FMC_ERR_HIP, "hipFuncSetAttribute(%zu bytes of LDS): %s", shm, hipGetErrorString(e));
+    return FMC_ERR_HIP;
+  }
+  return FMC_OK;
+}
+
+// The forward pass of a training step (saved layer inputs), on FMA register
+// tiles: the adjoint recomputes the hidden layers with the same sums, and a
+// ReLU mask that rounds differently in the two changes a weight gradient by a
+// whole sample's share.
+__global__ void __launch_bounds__(RN_THREADS) rnvp_train_pass_kernel(RnvpDev f, RnPassArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int d = f.d, h = f.h;
   const RnSmem sm(d, h, false);
@@ -286,40 +386,24 @@ __global__ void __launch_bounds__(RN_THREADS) rnvp_pass_kernel(RnvpDev f, RnPass
   const int64_t st = rn_stats(d, h, f.L);
   const float* dmean = th + st;
   const float* dcov = dmean + d;
-  const float* bmean = dcov + (int64_t)d * d;
-  const float* bcov = bmean + d;
 
   for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
     const int m = o / d, j = o - m * d;
     const int64_t row = m0 + m;
     float v = 0.f;
     if (row < a.n) {
-      if ((a.flags & RN_SAMPLE) && a.x_in == nullptr) {
-        const float4 z = philox_normal4(a.key0, a.key1, (uint32_t)(j >> 2), (uint32_t)(a.sample0 + row), 0u,
-                                        RNG_FLOW_BASE);
-        const int e = j & 3;
-        v = (e == 0) ? z.x : (e == 1) ? z.y : (e == 2) ? z.z : z.w;
-      } else {
-        v = a.x_in[row * d + j];
-      }
-      if (a.dir == 0 && (a.flags & RN_STD)) {
-        v = (v - dmean[j]) / sqrtf(dcov[(int64_t)j * d + j]);
-      } else if (a.dir != 0 && (a.flags & RN_SAMPLE)) {
-        v = bmean[j] + sqrtf(bcov[(int64_t)j * d + j]) * v;
-      }
+      v = a.x_in[row * d + j];
+      if (a.flags & RN_STD) v = (v - dmean[j]) / sqrtf(dcov[(int64_t)j * d + j]);
     }
     xs[m * ldx + j] = v;
   }
   for (int m = tid; m < RN_TS; m += RN_THREADS) ldr[m] = 0.f;
   __syncthreads();
 
-  for (int step = 0; step < f.L; ++step) {
-    const int l = (a.dir == 0) ? step : f.L - 1 - step;
-    if (a.saved) {
-      for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
-        const int m = o / d, j = o - m * d;
-        if (m0 + m < a.n) a.saved[((int64_t)l * a.n + m0 + m) * d + j] = xs[m * ldx + j];
-      }
+  for (int l = 0; l < f.L; ++l) {
+    for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
+      const int m = o / d, j = o - m * d;
+      if (m0 + m < a.n) a.saved[((int64_t)l * a.n + m0 + m) * d + j] = xs[m * ldx + j];
     }
     const int32_t* lay = rn_lay(f, l);
     const int dc = lay[0], dtr = lay[1];
@@ -341,14 +425,14 @@ __global__ void __launch_bounds__(RN_THREADS) rnvp_pass_kernel(RnvpDev f, RnPass
       const float s = tanhf(sT[o]) * f.dt;
       const float t = tT[o] * f.dt;
       const float x = xs[m * ldx + j];
-      xs[m * ldx + j] = (a.dir == 0) ? (x + t) * expf(s) : x * expf(-s) - t;
+      xs[m * ldx + j] = (x + t) * expf(s);
       sT[o] = s;
     }
     __syncthreads();
     for (int m = tid; m < RN_TS; m += RN_THREADS) {
       float s = 0.f;
       for (int i = 0; i < dtr; ++i) s += sT[i * RN_TS + m];
-      ldr[m] += (a.dir == 0) ? s : -s;
+      ldr[m] += s;
     }
     __syncthreads();
   }
@@ -357,7 +441,7 @@ __global__ void __launch_bounds__(RN_THREADS) rnvp_pass_kernel(RnvpDev f, RnPass
     const int64_t row = m0 + m;
     if (row >= a.n) continue;
     float ld = ldr[m];
-    if (a.dir == 0 && (a.flags & RN_BASE)) {
+    if (a.flags & RN_BASE) {
       // log N(y; 0, I) (realNVP.py:211-213: the standard normal, not base_dist)
       float q = 0.f;
       for (int j = 0; j < d; ++j) {
@@ -374,10 +458,304 @@ __global__ void __launch_bounds__(RN_THREADS) rnvp_pass_kernel(RnvpDev f, RnPass
       const int m = o / d, j = o - m * d;
       const int64_t row = m0 + m;
       if (row >= a.n) continue;
-      float v = xs[m * ldx + j];
-      if (a.dir != 0 && (a.flags & RN_STD)) v = v * sqrtf(dcov[(int64_t)j * d + j]) + dmean[j];
-      a.x_out[row * d + j] = v;
+      a.x_out[row * d + j] = xs[m * ldx + j];
     }
+  }
+}
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4_t rn_mfma(float a, float b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t rn_ld4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
+
+// One hidden block's weight fragments (a lane's share), requested one block
+// ahead of their use. Block indices past the end repeat the last block, so
+// every block issues the same loads and the waits cover them exactly.
+template <int NB>
+struct RnFrag {
+  f32x4_t w1[NB], w2[NB], b;
+  __device__ __forceinline__ void load(const RnFr& f, int hb, int r0, int lane) {
+    const int kc = f.KC > 0 ? f.KC : 1;  // (without conditioning dims any block of the slot serves)
+#pragma unroll
+    for (int k = 0; k < NB; ++k) w1[k] = rn_ld4(f.W1f + ((int64_t)hb * kc + (k < kc ? k : kc - 1)) * 256 + 4 * lane);
+#pragma unroll
+    for (int r = 0; r < NB; ++r)
+      w2[r] = rn_ld4(f.W2f + ((int64_t)hb * f.R + (r0 + r < f.R ? r0 + r : f.R - 1)) * 256 + 4 * lane);
+    b = rn_ld4(f.b1 + 16 * hb + 4 * (lane >> 4));
+  }
+};
+
+// out[r][m] += W2 relu(W1 c + b1) over the hidden blocks hb0, hb0 + hs, ..,
+// for the row blocks r0 .. r0 + NB - 1. The hidden block (16 features x 16
+// samples) never leaves the registers: a lane's four accumulators are the
+// second product's four k-steps.
+template <int NB, int MB>
+__device__ __forceinline__ void rn_mlp(const RnFr& f, int r0, int hb0, int hs, int dc, const f32x4_t (&c)[NB][MB],
+                                       const float* xs, int ldx, f32x4_t (&out)[NB][MB], int lane) {
+  if (hb0 >= f.HB) return;
+  RnFrag<NB> cur, nxt;
+  cur.load(f, hb0, r0, lane);
+  for (int hb = hb0; hb < f.HB; hb += hs) {
+    nxt.load(f, hb + hs < f.HB ? hb + hs : hb, r0, lane);
+    f32x4_t a[MB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m) a[m] = cur.b;
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+      if (k < f.KC) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int m = 0; m < MB; ++m) a[m] = rn_mfma(cur.w1[k][e], c[k][m][e], a[m]);
+      }
+    for (int k = NB; k < f.KC; ++k) {  // more conditioning dims than the registers hold
+      const f32x4_t w = rn_ld4(f.W1f + ((int64_t)hb * f.KC + k) * 256 + 4 * lane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * k + 4 * (lane >> 4) + e;
+        const int j = f.cond[i];
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+          a[m] = rn_mfma(w[e], i < dc ? xs[(16 * m + (lane & 15)) * ldx + j] : 0.f, a[m]);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[m][e] = __builtin_amdgcn_fmed3f(a[m][e], 0.f, INFINITY);
+#pragma unroll
+    for (int r = 0; r < NB; ++r)
+      if (r0 + r < f.R) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int m = 0; m < MB; ++m) out[r][m] = rn_mfma(cur.w2[r][e], a[m][e], out[r][m]);
+      }
+    cur = nxt;
+  }
+}
+
+// All layers of a pass for 16 MB samples on the FP32 matrix cores, which bound
+// it at large n (65 % of a large FP32 product's rate at 409,600 samples, the
+// rest tails, tanh / exp and weight reads); small batches are bound by the
+// serial chain of hidden blocks and layers.
+// SPLIT = false: every wavefront owns 16 MB samples and runs alone (no
+// barrier); SPLIT = true: the eight wavefronts of a workgroup share one
+// 16-sample tile, each taking one MLP (wave & 1) and every fourth hidden
+// block, their partial outputs summed in LDS in a fixed order. NB: blocks of
+// 16 conditioning / transformed dims held in registers; masks that leave more
+// on one side take the loops over the rest.
+template <int NB, int MB, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 512 : 256) __attribute__((amdgpu_waves_per_eu(NB <= 1 ? 4 : 2)))
+rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
+  static_assert(!SPLIT || MB == 1, "a shared tile holds 16 samples");
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int S = 16 * MB, NT = SPLIT ? 512 : 64;
+  const int d = f.d, h = f.h, ldx = d + 1;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, q = lane >> 4, t = SPLIT ? (int)threadIdx.x : lane;
+  const int xsz = rn_rup16(S * ldx * 4) / 4;
+  float* xs = reinterpret_cast<float*>(smem) + (SPLIT ? 0 : wave * xsz);
+  float* red = reinterpret_cast<float*>(smem) + xsz;  // SPLIT: [8 waves][NB][64] float4, then [8][16] log-dets
+  float* ldp = red + 8 * NB * 256;
+  const int64_t m0 = ((int64_t)blockIdx.x * (SPLIT ? 1 : 4) + (SPLIT ? 0 : wave)) * S;
+  if (m0 >= a.n) return;  // (a whole wavefront; a whole workgroup when the tile is shared)
+  auto sync = [] {
+    if constexpr (SPLIT) {
+      __syncthreads();
+    } else {  // LDS of this wavefront only: order its accesses
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  const float* th = f.theta;
+  const int64_t st = rn_stats(d, h, f.L);
+  const float* dmean = th + st;
+  const float* dcov = dmean + d;
+  const float* bmean = dcov + (int64_t)d * d;
+  const float* bcov = bmean + d;
+
+  if ((a.flags & RN_SAMPLE) && a.x_in == nullptr) {  // base noise: one Philox block per four dims
+    const int ch = (d + 3) >> 2;
+    for (int o = t; o < S * ch; o += NT) {
+      const int m = o / ch, k = o - m * ch;
+      const float4 z = philox_normal4(a.key0, a.key1, (uint32_t)k, (uint32_t)(a.sample0 + m0 + m), 0u, RNG_FLOW_BASE);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = 4 * k + e;
+        if (j < d) xs[m * ldx + j] = m0 + m < a.n ? bmean[j] + sqrtf(bcov[(int64_t)j * d + j]) * f4c(z, e) : 0.f;
+      }
+    }
+  } else {
+    for (int o = t; o < S * d; o += NT) {
+      const int m = o / d, j = o - m * d;
+      float v = 0.f;
+      if (m0 + m < a.n) {
+        v = a.x_in[m0 * d + o];
+        if (a.dir == 0 && (a.flags & RN_STD))
+          v = (v - dmean[j]) / sqrtf(dcov[(int64_t)j * d + j]);
+        else if (a.dir != 0 && (a.flags & RN_SAMPLE))
+          v = bmean[j] + sqrtf(bcov[(int64_t)j * d + j]) * v;
+      }
+      xs[m * ldx + j] = v;
+    }
+  }
+  sync();
+
+  float ldacc[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) ldacc[m] = 0.f;
+  for (int step = 0; step < f.L; ++step) {
+    const int l = (a.dir == 0) ? step : f.L - 1 - step;
+    const int32_t* lay = rn_lay(f, l);
+    const int dc = lay[0], dtr = lay[1];
+    const RnFr fs(f.packed, d, h, f.L, l, 0, dc, dtr), ft(f.packed, d, h, f.L, l, 1, dc, dtr);
+    f32x4_t c[NB][MB];  // conditioning inputs as MFMA operands
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+      if (k < fs.KC) {
+        const int4 ci = *reinterpret_cast<const int4*>(fs.cond + 16 * k + 4 * q);
+        const int i0 = 16 * k + 4 * q;
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          const float* xr = xs + (16 * m + col) * ldx;
+          c[k][m] = f32x4_t{i0 < dc ? xr[ci.x] : 0.f, i0 + 1 < dc ? xr[ci.y] : 0.f, i0 + 2 < dc ? xr[ci.z] : 0.f,
+                            i0 + 3 < dc ? xr[ci.w] : 0.f};
+        }
+      }
+    for (int r0 = 0; r0 < fs.R; r0 += NB) {
+      f32x4_t os[NB][MB], ot[NB][MB];
+#pragma unroll
+      for (int r = 0; r < NB; ++r)
+#pragma unroll
+        for (int m = 0; m < MB; ++m) os[r][m] = ot[r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (SPLIT) {
+        rn_mlp<NB, MB>((wave & 1) ? ft : fs, r0, wave >> 1, 4, dc, c, xs, ldx, os, lane);
+#pragma unroll
+        for (int r = 0; r < NB; ++r) *reinterpret_cast<f32x4_t*>(red + ((wave * NB + r) * 64 + lane) * 4) = os[r][0];
+        __syncthreads();
+      } else {
+        rn_mlp<NB, MB>(fs, r0, 0, 1, dc, c, xs, ldx, os, lane);
+        rn_mlp<NB, MB>(ft, r0, 0, 1, dc, c, xs, ldx, ot, lane);
+      }
+      // coupling on the transformed dims: a lane holds the scale and shift of
+      // dims 16 r + 4 q + e of its sample (SPLIT: row block r by wave r)
+#pragma unroll
+      for (int r = 0; r < NB; ++r) {
+        if (r0 + r >= fs.R || (SPLIT && wave != r)) continue;
+        if constexpr (SPLIT) {
+#pragma unroll
+          for (int w = 0; w < 8; w += 2) {
+            const f32x4_t u = rn_ld4(red + ((w * NB + r) * 64 + lane) * 4);
+            const f32x4_t v = rn_ld4(red + (((w + 1) * NB + r) * 64 + lane) * 4);
+            os[r][0] = w == 0 ? u : os[r][0] + u;
+            ot[r][0] = w == 0 ? v : ot[r][0] + v;
+          }
+        }
+        const int k0 = 16 * (r0 + r) + 4 * q;
+        const f32x4_t bs = rn_ld4(fs.b2 + k0), bt = rn_ld4(ft.b2 + k0);
+        const int4 ti = *reinterpret_cast<const int4*>(fs.trans + k0);
+        const int tj[4] = {ti.x, ti.y, ti.z, ti.w};
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (k0 + e < dtr) {
+              float* xp = xs + (16 * m + col) * ldx + tj[e];
+              const float s = tanhf(os[r][m][e] + bs[e]) * f.dt;
+              const float tt = (ot[r][m][e] + bt[e]) * f.dt;
+              *xp = (a.dir == 0) ? (*xp + tt) * expf(s) : *xp * expf(-s) - tt;
+              ldacc[m] += s;
+            }
+      }
+      sync();
+    }
+  }
+  // ---- log-det of each sample: the four lanes that share it (SPLIT: and the
+  // waves), in a fixed order
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    ldacc[m] += __shfl_xor(ldacc[m], 16, 64);
+    ldacc[m] += __shfl_xor(ldacc[m], 32, 64);
+  }
+  if constexpr (SPLIT) {
+    if (lane < 16) ldp[wave * 16 + lane] = ldacc[0];
+    __syncthreads();
+    ldacc[0] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NB; ++w) ldacc[0] += ldp[w * 16 + col];
+  }
+  // ---- outputs
+  if (q == 0 && (!SPLIT || wave == 0)) {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int64_t row = m0 + 16 * m + col;
+      if (row >= a.n) continue;
+      float ld = (a.dir == 0) ? ldacc[m] : -ldacc[m];
+      if (a.dir == 0 && (a.flags & RN_BASE)) {
+        // log N(y; 0, I) (realNVP.py:211-213: the standard normal, not base_dist)
+        float s2 = 0.f;
+        for (int j = 0; j < d; ++j) {
+          const float y = xs[(16 * m + col) * ldx + j];
+          s2 += y * y;
+        }
+        ld += -0.5f * s2 - 0.91893853320467274f * (float)d;
+      }
+      if (a.logdet) a.logdet[row] = ld;
+    }
+  }
+  if (a.x_out || a.gy_out) {
+    for (int o = t; o < S * d; o += NT) {
+      const int m = o / d, j = o - m * d;
+      if (m0 + m >= a.n) continue;
+      float v = xs[m * ldx + j];
+      if (a.gy_out) a.gy_out[m0 * d + o] = -a.g_logp[m0 + m] * v;
+      if (a.x_out) {
+        if (a.dir != 0 && (a.flags & RN_STD)) v = v * sqrtf(dcov[(int64_t)j * d + j]) + dmean[j];
+        a.x_out[m0 * d + o] = v;
+      }
+    }
+  }
+}
+
+template <int NB, int MB, bool SPLIT>
+static int rn_launch_pass(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) {
+  const int xsz = rn_rup16(16 * MB * (f.d + 1) * 4);
+  const size_t shm = SPLIT ? (size_t)xsz + 8 * NB * 1024 + 512 : 4 * (size_t)xsz;
+  if (const int rc = rn_set_lds(rnvp_pass_kernel<NB, MB, SPLIT>, shm)) return rc;
+  const int64_t per = SPLIT ? 16 : 64 * MB, grid = (a.n + per - 1) / per;
+  FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
+  hipLaunchKernelGGL((rnvp_pass_kernel<NB, MB, SPLIT>), dim3((unsigned)grid), dim3(SPLIT ? 512 : 256), shm, st, f, a);
+  return check_launch("realnvp pass");
+}
+
+// Which pass runs a batch of n samples (measured, sampling, us; d = 32, 8
+// layers, hidden 256 | d = 64, 10 layers, hidden 128 | d = 5, 4 layers, hidden 64):
+//   n         shared tile (8 waves)   16 samples a wave   32 samples a wave
+//   1000        29 |   39 |  14          82 |   95 |  19      129 |  157 |  26
+//   10000       67 |   92 |  22          86 |  101 |  18      131 |  159 |  25
+//   20000      108 |  147 |  32         123 |  151 |  24      135 |  164 |  25
+//   50000      262 |  350 |  75         219 |  291 |  36      211 |  261 |  36
+//   409600    1825 | 2495 | 534        1177 | 1627 | 186     1101 | 1433 | 171
+// A shared tile spreads the serial hidden blocks of a layer over eight waves,
+// which pays until a wave for every 16 samples fills the chip's SIMDs, and
+// less so the fewer hidden blocks there are to spread; 32 samples a wave halve
+// the weight reads once the grid is several waves a SIMD deep. Wide states,
+// whose four tiles would not leave room for two workgroups a CU, share one.
+static int rn_pass_variant(int64_t n, int d, int h) {
+  const int64_t tiles = (n + 15) / 16, split_to = 100 * rn_b16(h);
+  if (4 * rn_rup16(16 * (d + 1) * 4) > 64 * 1024 || tiles <= (split_to < 1280 ? split_to : 1280)) return 0;
+  return tiles <= 2048 ? 1 : 2;
+}
+
+template <int NB>
+static int rn_pass_nb(hipStream_t st, const RnvpDev& f, const RnPassArgs& a, int var) {
+  switch (var) {
+    case 0: return rn_launch_pass<NB, 1, true>(st, f, a);
+    case 1: return rn_launch_pass<NB, 1, false>(st, f, a);
+    default: return rn_launch_pass<NB, 2, false>(st, f, a);
   }
 }
 
@@ -599,17 +977,6 @@ static int check_rnvp(const fmc_rnvp* r, RnvpDev& f, bool need_packed) {
   return FMC_OK;
 }
 
-template <class K>
-static int rn_set_lds(K kernel, size_t shm) {
-  const hipError_t e =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-  if (e != hipSuccess) {
-    set_error(FMC_ERR_HIP, "hipFuncSetAttribute(%zu bytes of LDS): %s", shm, hipGetErrorString(e));
-    return FMC_ERR_HIP;
-  }
-  return FMC_OK;
-}
-
 }  // namespace fmc
 
 using namespace fmc;
@@ -620,7 +987,7 @@ extern "C" int fmc_rnvp_sizes(const fmc_rnvp* r, int64_t* theta_size, int64_t* p
   int rc = check_rnvp(r, f, false);
   if (rc) return rc;
   if (theta_size) *theta_size = rn_theta_size(f.d, f.h, f.L);
-  if (packed_size) *packed_size = 2LL * f.L * rn_pk_mlp(f.d, f.h);
+  if (packed_size) *packed_size = rn_packed_size(f.d, f.h, f.L);
   if (partial_per_tile) *partial_per_tile = rn_layer_size(f.d, f.h);  // rows: tiles + chunk rows
   if (tile) *tile = RN_TS;
   return FMC_OK;
@@ -633,7 +1000,11 @@ extern "C" int fmc_rnvp_pack(void* stream, const fmc_rnvp* r) {
   const int64_t n = rn_pk_mlp(f.d, f.h);
   const unsigned gx = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
   hipLaunchKernelGGL(rnvp_pack_kernel, dim3(gx, 2 * f.L), dim3(256), 0, (hipStream_t)stream, f, r->packed);
-  return check_launch("realnvp pack");
+  if ((rc = check_launch("realnvp pack"))) return rc;
+  const int64_t nf = rn_fr_slot(f.d, f.h);
+  hipLaunchKernelGGL(rnvp_pack_frag_kernel, dim3((unsigned)((nf + 255) / 256 < 4096 ? (nf + 255) / 256 : 4096), 2 * f.L),
+                     dim3(256), 0, (hipStream_t)stream, f, r->packed);
+  return check_launch("realnvp pack (fragments)");
 }
 
 extern "C" int fmc_rnvp_pass(void* stream, const fmc_rnvp* r, int32_t dir, int32_t flags, const float* x_in,
@@ -650,14 +1021,21 @@ extern "C" int fmc_rnvp_pass(void* stream, const fmc_rnvp* r, int32_t dir, int32
   FMC_ARG(saved == nullptr || dir == 0, "saved layer inputs need the forward direction");
   FMC_ARG(gy_out == nullptr || (g_logp != nullptr && (flags & RN_BASE)), "gy_out needs g_logp and BASE_LOGP");
   if (n == 0) return FMC_OK;
-  const RnSmem sm(f.d, f.h, false);
-  if ((rc = rn_set_lds(rnvp_pass_kernel, (size_t)sm.total))) return rc;
   RnPassArgs a{dir, flags, x_in, n, key0, key1, sample0, x_out, logdet, saved, g_logp, gy_out};
-  const int64_t grid = (n + RN_TS - 1) / RN_TS;
-  FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
-  hipLaunchKernelGGL(rnvp_pass_kernel, dim3((unsigned)grid), dim3(RN_THREADS), (size_t)sm.total,
-                     (hipStream_t)stream, f, a);
-  return check_launch("realnvp pass");
+  hipStream_t st = (hipStream_t)stream;
+  if (saved) {
+    const RnSmem sm(f.d, f.h, false);
+    if ((rc = rn_set_lds(rnvp_train_pass_kernel, (size_t)sm.total))) return rc;
+    const int64_t grid = (n + RN_TS - 1) / RN_TS;
+    FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
+    hipLaunchKernelGGL(rnvp_train_pass_kernel, dim3((unsigned)grid), dim3(RN_THREADS), (size_t)sm.total, st, f, a);
+    return check_launch("realnvp training pass");
+  }
+  const int nb = rn_b16((f.d + 1) / 2);  // blocks of a mask that halves the dims
+  const int var = rn_pass_variant(n, f.d, f.h);
+  if (nb <= 1) return rn_pass_nb<1>(st, f, a, var);
+  if (nb <= 2) return rn_pass_nb<2>(st, f, a, var);
+  return rn_pass_nb<4>(st, f, a, var);
 }
 
 extern "C" int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* r, int32_t layer, const float* x_in, int64_t n,
