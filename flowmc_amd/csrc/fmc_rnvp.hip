@@ -3,25 +3,21 @@
 // ([d, hidden, d], ReLU; common.py:68-112, 171-208) read the conditioning
 // dims and drive the transformed dims:
 //   s = tanh(MLP_s(c)) dt,  t = MLP_t(c) dt,  y = (x + t) e^s,  log-det = sum s.
-// The model is FP32 end to end. The passes run on the FP32 matrix cores
-// (v_mfma_f32_16x16x4: the FP32 vector rate without packed forms is half of
-// it): 409,600 samples at d = 32, 8 layers, hidden 256 drawn in 1.10 ms, 98
-// TFLOP/s, where FMA register tiles over LDS took 4.05 ms; 10,000 in 67 us
-// (213 us). Training (forward with saved inputs, adjoint) uses FP32 FMA
-// register tiles (4 outputs x 4 samples per thread) over LDS-resident
-// activations, with weights read as aligned float4 rows of an L2-resident
-// packed copy; products with few outputs split their reduction over the lanes
-// of a wavefront and combine them with xor shuffles. Its workgroups of 256
-// threads own RN_TS = 16 samples; the adjoint runs one layer per launch and
-// writes per-tile weight-gradient partials, which a second kernel sums over
-// tiles in a fixed order and scatters into the gradient vector.
+// The model is FP32 end to end and every product runs on the FP32 matrix
+// cores (v_mfma_f32_16x16x4: the FP32 vector rate without packed forms is half
+// of it; one instruction is four FMAs in k order, bit for bit, so a chain of
+// them sums in the order its operands are laid out in). A hidden block of 16
+// features x 16 samples stays in registers from the first product to the
+// next: a lane's four accumulators are the second product's four k-steps.
+//   passes   409,600 samples at d = 32, 8 layers, hidden 256 drawn in 1.10 ms,
+//            98 TFLOP/s (FMA register tiles over LDS: 4.05 ms)
+//   training one step of 10,000 samples, same flow: 0.32 ms (1.10 ms with FMA
+//            tiles, one adjoint launch a layer and a partial weight gradient
+//            for every 16 samples): forward 72 us, adjoint of all layers 200,
+//            weight-gradient sums 19
 #include "fmc_common.h"
 
 namespace fmc {
-
-constexpr int RN_TS = 16;       // samples per workgroup
-constexpr int RN_THREADS = 256;
-constexpr int RN_Q = RN_TS / 4;  // float4 sample groups
 
 struct RnvpDev {
   int d, L, h;
@@ -43,298 +39,145 @@ __host__ __device__ inline int64_t rn_stats(int d, int h, int L) { return L * rn
 __host__ __device__ inline int64_t rn_theta_size(int d, int h, int L) {
   return rn_stats(d, h, L) + 2LL * d + 2LL * d * d;
 }
-// ---- packed copy, per (layer, p), with d4 / h4 = d / h rounded up to 4 and
-// zero padding: W1T [d4][h4] (W1T[k][j] = W1[j][cond_k]), W1c [h4][d4] (its
-// transpose), W2T [h4][d4] (W2T[j][i] = W2[trans_i][j]), W2c [d4][h4] (its
-// transpose), b1 [h4], b2c [d4] (b2c[i] = b2[trans_i]). Every row starts on a
-// 16-byte boundary.
-__host__ __device__ inline int rn_r4(int v) { return (v + 3) & ~3; }
-__host__ __device__ inline int64_t rn_pk_mlp(int d, int h) {
-  return 4LL * rn_r4(d) * rn_r4(h) + rn_r4(h) + rn_r4(d);
-}
-__host__ __device__ inline int64_t rn_pk(int d, int h, int l, int p) { return (2LL * l + p) * rn_pk_mlp(d, h); }
-struct RnPk {
-  const float *W1T, *W1c, *W2T, *W2c, *b1, *b2c;
-  __device__ RnPk(const float* base, int d4, int h4) {
-    const int64_t s = (int64_t)d4 * h4;
-    W1T = base;
-    W1c = base + s;
-    W2T = base + 2 * s;
-    W2c = base + 3 * s;
-    b1 = base + 4 * s;
-    b2c = b1 + h4;
-  }
-};
-// ---- MFMA fragment images, per (layer, p), after the images above. Blocks of
-// 16 conditioning dims (kg < KC), 16 transformed dims (r < R) and 16 hidden
-// features (hb < HB); one 16 x 16 weight block is 64 lanes x float4, lane l
-// (c = l % 16, q = l / 16) holding four k-steps of v_mfma_f32_16x16x4:
-//   W1f [hb][kg]: W1[16 hb + c][cond(16 kg + 4q + e)]
-//   W2f [hb][r]:  W2[trans(16 r + c)][16 hb + 4q + e]
-// (k = 4q + e is also the row a lane's accumulator e holds, so the output
-// block of the first product is the second product's operand as it lies),
-// then b1 [16 HB], b2 [16 R], and the index words {n_cond, n_trans, 0, 0,
-// cond [16 KC], trans [16 R]} (padding entries 0). A slot has a fixed size:
-// KC + R <= ceil(d / 16) + 1 whatever the mask.
-__host__ __device__ inline int rn_b16(int v) { return (v + 15) >> 4; }
-__host__ __device__ inline int64_t rn_fr_slot(int d, int h) {
-  const int kr = rn_b16(d) + 1, hb = rn_b16(h);
-  return 256LL * hb * kr + 16LL * hb + 16LL * rn_b16(d) + 4 + 16LL * kr;
-}
-__host__ __device__ inline int64_t rn_fr_base(int d, int h, int L) { return (2LL * L * rn_pk_mlp(d, h) + 15) & ~15LL; }
-__host__ __device__ inline int64_t rn_packed_size(int d, int h, int L) {
-  return rn_fr_base(d, h, L) + 2LL * L * ((rn_fr_slot(d, h) + 15) & ~15LL);
-}
-struct RnFr {
-  int KC, R, HB;
-  const float *W1f, *W2f, *b1, *b2;
-  const int32_t *nct, *cond, *trans;  // {n_cond, n_trans}, index lists
-  __device__ RnFr(const float* packed, int d, int h, int L, int l, int p, int dc, int dtr) {
-    KC = rn_b16(dc);
-    R = rn_b16(dtr);
-    HB = rn_b16(h);
-    W1f = packed + rn_fr_base(d, h, L) + (2LL * l + p) * ((rn_fr_slot(d, h) + 15) & ~15LL);
-    W2f = W1f + 256LL * HB * KC;
-    b1 = W2f + 256LL * HB * R;
-    b2 = b1 + 16 * HB;
-    nct = reinterpret_cast<const int32_t*>(b2 + 16 * R);
-    cond = nct + 4;
-    trans = cond + 16 * KC;
-  }
-};
 // ---- layout: per layer [n_cond, n_trans, cond[d], trans[d]]
 __host__ __device__ inline const int32_t* rn_lay(const RnvpDev& f, int l) { return f.layout + (int64_t)l * (2 + 2 * f.d); }
 
 __host__ __device__ inline int rn_rup16(int v) { return (v + 15) & ~15; }
+__host__ __device__ inline int rn_b16(int v) { return (v + 15) >> 4; }
 
-struct RnSmem {
-  int xs, gb, cT, hT, ghT, sT, tT, gcT, ldr, glp, total;
-  int ldx, d4, h4;
-  __host__ __device__ RnSmem(int d, int h, bool bwd) {
-    ldx = d + 1;
-    d4 = (d + 3) & ~3;
-    h4 = (h + 3) & ~3;
-    int o = 0;
-    xs = o;
-    o += rn_rup16(RN_TS * ldx * 4);
-    gb = o;
-    o += bwd ? rn_rup16(RN_TS * ldx * 4) : 0;
-    cT = o;  // [d4][TS] conditioning inputs, sample-contiguous
-    o += d4 * RN_TS * 4;
-    hT = o;  // [h4][TS] hidden activations
-    o += h4 * RN_TS * 4;
-    ghT = o;  // [h4][TS] hidden pre-activation gradients (adjoint)
-    o += bwd ? h4 * RN_TS * 4 : 0;
-    sT = o;  // [d4][TS] scale pre-activations / tanh / their gradients
-    o += d4 * RN_TS * 4;
-    tT = o;  // [d4][TS] shift outputs / their gradients
-    o += d4 * RN_TS * 4;
-    gcT = o;  // [d4][TS] conditioning-input gradients of one MLP (adjoint)
-    o += bwd ? d4 * RN_TS * 4 : 0;
-    ldr = o;
-    o += RN_TS * 4;
-    glp = o;
-    o += RN_TS * 4;
-    total = o;
+// ---- packed copy: MFMA fragment images per (layer, p). Blocks of 16
+// conditioning dims (kg < KC), 16 transformed dims (r < R) and 16 hidden
+// features (hb < HB); one 16 x 16 weight block is 64 lanes x float4, lane l
+// (c = l % 16, q = l / 16) holding element e of four k-steps:
+//   W1f [hb][kg]: W1[16 hb + c][cond(16 kg + 4e + q)]   (k in dim order)
+//   W2f [hb][r]:  W2[trans(16 r + c)][16 hb + 4q + e]
+//   W2t [hb][r]:  W2[trans(16 r + 4e + q)][16 hb + c]
+//   W1t [hb][kg]: W1[16 hb + 4q + e][cond(16 kg + c)]
+// b1 [16 HB], b2 [16 R]; the training forward's images W1s [blk][kg],
+// W2s [blk][r], b1s [16 blk] with the hidden features in its summation order
+// (RnOrder: row 4q + i of block blk is feature (blk, q, i)); and the index
+// words cond [16 KC], the same in fragment order (word 4q + e of a block is
+// cond 4e + q), trans [16 R], padding entries 0. Slots have a fixed size: KC +
+// R <= ceil(d / 16) + 1 whatever the mask, and at most HB + 16 ordered blocks.
+struct RnOrder {
+  // The sum over the hidden features of one output: S strided partial sums
+  // (features s, s + S, ..: one chain each), then pairs at distance S/2, S/4,
+  // .., 1. S = 256 / (4 ceil(n_trans / 4)) rounded down to a power of two <= 64.
+  // An ordered block holds 16 features: its k-step i (element i of all four
+  // q) belongs to one chain, so the four chains s, s + S/2, s + S/4, s + 3S/4
+  // (S >= 4) advance by four features each and end in two levels of pairs.
+  int S, Sg, G, U;  // chains; chains of a block; blocks side by side; blocks along a chain
+  __host__ __device__ RnOrder(int dtr, int h) {
+    const int tiles = 4 * ((dtr + 3) >> 2);
+    S = 1;
+    while (S < 64 && tiles * S * 2 <= 256) S <<= 1;
+    Sg = S < 4 ? S : 4;
+    G = S / Sg;
+    U = (h + S * (16 / Sg) - 1) / (S * (16 / Sg));
+  }
+  __host__ __device__ int blocks() const { return G * U; }
+  __host__ __device__ int feature(int blk, int q, int i) const {
+    const int g = blk / U, u = blk - g * U, k = i % Sg;
+    const int s = S >= 4 ? g + (k & 1) * (S >> 1) + (k >> 1) * (S >> 2) : k;
+    return s + S * ((u * (4 / Sg) + i / Sg) * 4 + q);
+  }
+};
+__host__ __device__ inline int64_t rn_slot(int d, int h) {
+  const int kr = rn_b16(d) + 1, hb = rn_b16(h);
+  const int64_t w = 512LL * hb * kr + 16LL * hb + 16LL * rn_b16(d) + 256LL * (hb + 16) * kr + 16LL * (hb + 16) + 32LL * kr;
+  return (w + 15) & ~15LL;
+}
+__host__ __device__ inline int64_t rn_packed_size(int d, int h, int L) { return 2LL * L * rn_slot(d, h); }
+struct RnFr {
+  int KC, R, HB;
+  const float *W1f, *W2f, *W2t, *W1t, *b1, *b2, *W1s, *W2s, *b1s;
+  const int32_t *cond, *condf, *trans;
+  __device__ RnFr(const float* packed, int d, int h, int l, int p, int dc, int dtr) {
+    KC = rn_b16(dc);
+    R = rn_b16(dtr);
+    HB = rn_b16(h);
+    const int nb = RnOrder(dtr, h).blocks();
+    W1f = packed + (2LL * l + p) * rn_slot(d, h);
+    W1t = W1f + 256LL * HB * KC;
+    W2f = W1t + 256LL * HB * KC;
+    W2t = W2f + 256LL * HB * R;
+    b1 = W2t + 256LL * HB * R;
+    b2 = b1 + 16 * HB;
+    W1s = b2 + 16 * R;
+    W2s = W1s + 256LL * nb * KC;
+    b1s = W2s + 256LL * nb * R;
+    cond = reinterpret_cast<const int32_t*>(b1s + 16 * nb);
+    condf = cond + 16 * KC;
+    trans = condf + 16 * KC;
   }
 };
 
-#define RN_FMA16(acc, w, c)                    \
-  do {                                         \
-    acc[0][0] = fmaf(w.x, c.x, acc[0][0]);     \
-    acc[0][1] = fmaf(w.x, c.y, acc[0][1]);     \
-    acc[0][2] = fmaf(w.x, c.z, acc[0][2]);     \
-    acc[0][3] = fmaf(w.x, c.w, acc[0][3]);     \
-    acc[1][0] = fmaf(w.y, c.x, acc[1][0]);     \
-    acc[1][1] = fmaf(w.y, c.y, acc[1][1]);     \
-    acc[1][2] = fmaf(w.y, c.z, acc[1][2]);     \
-    acc[1][3] = fmaf(w.y, c.w, acc[1][3]);     \
-    acc[2][0] = fmaf(w.z, c.x, acc[2][0]);     \
-    acc[2][1] = fmaf(w.z, c.y, acc[2][1]);     \
-    acc[2][2] = fmaf(w.z, c.z, acc[2][2]);     \
-    acc[2][3] = fmaf(w.z, c.w, acc[2][3]);     \
-    acc[3][0] = fmaf(w.w, c.x, acc[3][0]);     \
-    acc[3][1] = fmaf(w.w, c.y, acc[3][1]);     \
-    acc[3][2] = fmaf(w.w, c.z, acc[3][2]);     \
-    acc[3][3] = fmaf(w.w, c.w, acc[3][3]);     \
-  } while (0)
-
-// Wide product, h4 output rows: out[r][m] = sum_k W[k][r] in[k][m] (W rows of
-// length h4), one 4-row x 4-sample tile per thread. MODE 0: out = relu(bias +
-// .); MODE 1: out = . where hmask > 0, else 0 (ReLU derivative). Padding rows
-// come out zero (zero weights and bias).
-template <int MODE>
-__device__ __forceinline__ void rn_wide(const float* __restrict__ W, const float* __restrict__ bias, int K, int h4,
-                                        const float* inT, float* outT, const float* hmask) {
-  const int tr = h4 >> 2;
-  for (int o = threadIdx.x; o < tr * RN_Q; o += RN_THREADS) {
-    const int jq = o % tr, q = o / tr;
-    float acc[4][4];
-    const float4 b = (MODE == 0) ? *reinterpret_cast<const float4*>(bias + 4 * jq) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      acc[0][v] = b.x;
-      acc[1][v] = b.y;
-      acc[2][v] = b.z;
-      acc[3][v] = b.w;
-    }
-    for (int k = 0; k < K; ++k) {
-      const float4 w = *reinterpret_cast<const float4*>(W + (int64_t)k * h4 + 4 * jq);
-      const float4 c = *reinterpret_cast<const float4*>(inT + k * RN_TS + 4 * q);
-      RN_FMA16(acc, w, c);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      float4 r = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
-      const int row = 4 * jq + u;
-      if (MODE == 0) {
-        r.x = fmaxf(r.x, 0.f);
-        r.y = fmaxf(r.y, 0.f);
-        r.z = fmaxf(r.z, 0.f);
-        r.w = fmaxf(r.w, 0.f);
-      } else {
-        const float4 hv = *reinterpret_cast<const float4*>(hmask + row * RN_TS + 4 * q);
-        r.x = hv.x > 0.f ? r.x : 0.f;
-        r.y = hv.y > 0.f ? r.y : 0.f;
-        r.z = hv.z > 0.f ? r.z : 0.f;
-        r.w = hv.w > 0.f ? r.w : 0.f;
-      }
-      *reinterpret_cast<float4*>(outT + row * RN_TS + 4 * q) = r;
-    }
-  }
-}
-
-// Narrow product, n output rows (written up to n rounded to 4; the padding
-// rows come out zero): out[r][m] = bias[r] + sum_{j < K} W[j][r] in[j][m] (W
-// rows of length ldw). The reduction over j is split over S lanes of one
-// wavefront (S a power of two, tiles * S <= 256) and combined with xor
-// shuffles in a fixed order.
-__device__ __forceinline__ void rn_narrow(const float* __restrict__ W, int ldw, const float* __restrict__ bias, int K,
-                                          int n, const float* inT, float* outT) {
-  const int tr = (n + 3) >> 2;
-  const int tiles = tr * RN_Q;
-  int S = 1;
-  while (S < 64 && tiles * S * 2 <= RN_THREADS) S <<= 1;
-  for (int o = threadIdx.x; o < tiles * S; o += RN_THREADS) {
-    const int tile = o / S, s = o - tile * S;
-    const int iq = tile % tr, q = tile / tr;
-    float acc[4][4] = {};
-    for (int j = s; j < K; j += S) {
-      const float4 w = *reinterpret_cast<const float4*>(W + (int64_t)j * ldw + 4 * iq);
-      const float4 c = *reinterpret_cast<const float4*>(inT + j * RN_TS + 4 * q);
-      RN_FMA16(acc, w, c);
-    }
-    for (int off = S >> 1; off > 0; off >>= 1)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] += __shfl_xor(acc[u][v], off, 64);
-    if (s == 0) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int row = 4 * iq + u;
-        const float b = bias ? bias[row] : 0.f;
-        *reinterpret_cast<float4*>(outT + row * RN_TS + 4 * q) =
-            make_float4(acc[u][0] + b, acc[u][1] + b, acc[u][2] + b, acc[u][3] + b);
-      }
-    }
-  }
-}
-
-// Conditioning inputs of layer l into cT (rows >= dc zero, up to d4).
-__device__ __forceinline__ void rn_load_cond(const float* xs, int ldx, const int32_t* cond, int dc, int d4, float* cT) {
-  for (int o = threadIdx.x; o < d4 * RN_TS; o += RN_THREADS) {
-    const int k = o / RN_TS, m = o - k * RN_TS;
-    cT[o] = (k < dc) ? xs[m * ldx + cond[k]] : 0.f;
-  }
-}
-
 // ------------------------------------------------------------- packing ---
+// One thread per float4 of one (layer, p) slot (whose size fits 31 bits: d and
+// h are bounded by the kernels' LDS).
 __global__ void __launch_bounds__(256) rnvp_pack_kernel(RnvpDev f, float* packed) {
-  const int d = f.d, h = f.h, d4 = rn_r4(d), h4 = rn_r4(h);
-  const int lp = blockIdx.y, l = lp >> 1, p = lp & 1;
-  const int32_t* lay = rn_lay(f, l);
-  const int dc = lay[0], dtr = lay[1];
-  const int32_t* cond = lay + 2;
-  const int32_t* trans = lay + 2 + d;
-  const float* W1 = f.theta + rn_mlp(d, h, l, p);
-  const float* b1 = W1 + (int64_t)h * d;
-  const float* W2 = b1 + h;
-  const float* b2 = W2 + (int64_t)d * h;
-  float* dst = packed + rn_pk(d, h, l, p);
-  const int64_t sq = (int64_t)d4 * h4, n = rn_pk_mlp(d, h);
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    float v = 0.f;
-    const int region = (e < 4 * sq) ? (int)(e / sq) : 4;
-    const int64_t r = e - (int64_t)region * sq;
-    if (region == 0) {  // W1T[k][j]
-      const int k = (int)(r / h4), j = (int)(r - (int64_t)k * h4);
-      if (k < dc && j < h) v = W1[(int64_t)j * d + cond[k]];
-    } else if (region == 1) {  // W1c[j][k]
-      const int j = (int)(r / d4), k = (int)(r - (int64_t)j * d4);
-      if (k < dc && j < h) v = W1[(int64_t)j * d + cond[k]];
-    } else if (region == 2) {  // W2T[j][i]
-      const int j = (int)(r / d4), i = (int)(r - (int64_t)j * d4);
-      if (i < dtr && j < h) v = W2[(int64_t)trans[i] * h + j];
-    } else if (region == 3) {  // W2c[i][j]
-      const int i = (int)(r / h4), j = (int)(r - (int64_t)i * h4);
-      if (i < dtr && j < h) v = W2[(int64_t)trans[i] * h + j];
-    } else if (r < h4) {  // b1
-      if (r < h) v = b1[r];
-    } else {  // b2c
-      const int i = (int)(r - h4);
-      if (i < dtr) v = b2[trans[i]];
-    }
-    dst[e] = v;
-  }
-}
-
-// The fragment images of one (layer, p) slot (RnFr): one thread per word.
-__global__ void __launch_bounds__(256) rnvp_pack_frag_kernel(RnvpDev f, float* packed) {
   const int d = f.d, h = f.h;
   const int lp = blockIdx.y, l = lp >> 1, p = lp & 1;
   const int32_t* lay = rn_lay(f, l);
   const int dc = lay[0], dtr = lay[1];
   const int32_t* cond = lay + 2;
   const int32_t* trans = lay + 2 + d;
-  const RnFr fr(packed, d, h, f.L, l, p, dc, dtr);
+  const RnFr fr(packed, d, h, l, p, dc, dtr);
+  const RnOrder ord(dtr, h);
   const float* W1 = f.theta + rn_mlp(d, h, l, p);
   const float* b1 = W1 + (int64_t)h * d;
   const float* W2 = b1 + h;
   const float* b2 = W2 + (int64_t)d * h;
   float* dst = const_cast<float*>(fr.W1f);
-  const int64_t n1 = 256LL * fr.HB * fr.KC, n2 = n1 + 256LL * fr.HB * fr.R, n3 = n2 + 16 * fr.HB, n4 = n3 + 16 * fr.R;
-  const int64_t n5 = n4 + 4, n6 = n5 + 16 * fr.KC, n = n6 + 16 * fr.R;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    float v = 0.f;
-    if (e < n2) {
-      const bool first = e < n1;
-      const int64_t r = first ? e : e - n1;
-      const int nb = first ? fr.KC : fr.R;
-      const int hb = (int)(r / (256 * nb)), w = (int)(r - (int64_t)hb * 256 * nb);
-      const int b = w >> 8, lane = (w >> 2) & 63, el = w & 3, c = lane & 15, k = 4 * (lane >> 4) + el;
-      if (first) {
-        const int j = 16 * hb + c, i = 16 * b + k;
-        if (j < h && i < dc) v = W1[(int64_t)j * d + cond[i]];
-      } else {
-        const int i = 16 * b + c, j = 16 * hb + k;
-        if (j < h && i < dtr) v = W2[(int64_t)trans[i] * h + j];
+  const int64_t n = reinterpret_cast<const float*>(fr.trans + 16 * fr.R) - dst;
+  const int n4 = (int)(n >> 2), oW1t = (int)(fr.W1t - dst), oW2f = (int)(fr.W2f - dst), oW2t = (int)(fr.W2t - dst);
+  const int ob1 = (int)(fr.b1 - dst), ob2 = (int)(fr.b2 - dst), oW1s = (int)(fr.W1s - dst), oW2s = (int)(fr.W2s - dst);
+  const int ob1s = (int)(fr.b1s - dst), oc = (int)(reinterpret_cast<const float*>(fr.cond) - dst);
+  const int ocf = oc + 16 * fr.KC, ot = ocf + 16 * fr.KC;
+  for (int e4 = blockIdx.x * 256 + threadIdx.x; e4 < n4; e4 += gridDim.x * 256) {
+    const int e0 = 4 * e4;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (e0 < ob1 || (e0 >= oW1s && e0 < ob1s)) {  // a weight image
+      const bool sorted = e0 >= oW1s;
+      const bool w1 = sorted ? e0 < oW2s : e0 < oW2f;  // W1f, W1t, W1s
+      const bool tr = !sorted && ((e0 >= oW1t && e0 < oW2f) || e0 >= oW2t);
+      const int r = e0 - (sorted ? (w1 ? oW1s : oW2s) : w1 ? (tr ? oW1t : 0) : (tr ? oW2t : oW2f));
+      const int nb = w1 ? fr.KC : fr.R;
+      const int blk = r >> 8, hb = blk / nb, b = blk - hb * nb, lane = (r >> 2) & 63, c = lane & 15, q = lane >> 4;
+      const bool rows = w1 != tr;  // W1f, W1s, W2t: lane c is a feature, k the dims; else k the features
+      const int jr = sorted ? ord.feature(hb, c >> 2, c & 3) : 16 * hb + c;
+#pragma unroll
+      for (int el = 0; el < 4; ++el) {
+        const int j = rows ? jr : sorted ? ord.feature(hb, q, el) : 16 * hb + 4 * q + el;
+        const int i = rows ? 16 * b + 4 * el + q : 16 * b + c;
+        if (j < h && i < (w1 ? dc : dtr)) v[el] = w1 ? W1[(int64_t)j * d + cond[i]] : W2[(int64_t)trans[i] * h + j];
       }
-    } else if (e < n3) {
-      if (e - n2 < h) v = b1[e - n2];
-    } else if (e < n4) {
-      if (e - n3 < dtr) v = b2[trans[e - n3]];
     } else {
-      int w = 0;
-      if (e < n5)
-        w = e == n4 ? dc : (e == n4 + 1 ? dtr : 0);
-      else if (e < n6)
-        w = e - n5 < dc ? cond[e - n5] : 0;
-      else
-        w = e - n6 < dtr ? trans[e - n6] : 0;
-      v = __int_as_float(w);
+#pragma unroll
+      for (int el = 0; el < 4; ++el) {
+        const int e = e0 + el;
+        if (e < ob2) {
+          if (e - ob1 < h) v[el] = b1[e - ob1];
+        } else if (e < oW1s) {
+          if (e - ob2 < dtr) v[el] = b2[trans[e - ob2]];
+        } else if (e < oc) {
+          const int w = e - ob1s, j = ord.feature(w >> 4, (w >> 2) & 3, w & 3);
+          if (j < h) v[el] = b1[j];
+        } else {
+          int w = 0;
+          if (e < ocf) {
+            w = e - oc < dc ? cond[e - oc] : 0;
+          } else if (e < ot) {
+            const int u = e - ocf, i = (u & ~15) + 4 * (u & 3) + ((u >> 2) & 3);
+            w = i < dc ? cond[i] : 0;
+          } else {
+            w = e - ot < dtr ? trans[e - ot] : 0;
+          }
+          v[el] = __int_as_float(w);
+        }
+      }
     }
-    dst[e] = v;
+    reinterpret_cast<float4*>(dst)[e4] = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -366,109 +209,22 @@ static int rn_set_lds(K kernel, size_t shm) {
   return FMC_OK;
 }
 
-// The forward pass of a training step (saved layer inputs), on FMA register
-// tiles: the adjoint recomputes the hidden layers with the same sums, and a
-// ReLU mask that rounds differently in the two changes a weight gradient by a
-// whole sample's share.
-__global__ void __launch_bounds__(RN_THREADS) rnvp_train_pass_kernel(RnvpDev f, RnPassArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int d = f.d, h = f.h;
-  const RnSmem sm(d, h, false);
-  float* xs = reinterpret_cast<float*>(smem + sm.xs);
-  float* cT = reinterpret_cast<float*>(smem + sm.cT);
-  float* hT = reinterpret_cast<float*>(smem + sm.hT);
-  float* sT = reinterpret_cast<float*>(smem + sm.sT);
-  float* tT = reinterpret_cast<float*>(smem + sm.tT);
-  float* ldr = reinterpret_cast<float*>(smem + sm.ldr);
-  const int tid = threadIdx.x, ldx = sm.ldx;
-  const int64_t m0 = (int64_t)blockIdx.x * RN_TS;
-  const float* th = f.theta;
-  const int64_t st = rn_stats(d, h, f.L);
-  const float* dmean = th + st;
-  const float* dcov = dmean + d;
-
-  for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
-    const int m = o / d, j = o - m * d;
-    const int64_t row = m0 + m;
-    float v = 0.f;
-    if (row < a.n) {
-      v = a.x_in[row * d + j];
-      if (a.flags & RN_STD) v = (v - dmean[j]) / sqrtf(dcov[(int64_t)j * d + j]);
-    }
-    xs[m * ldx + j] = v;
-  }
-  for (int m = tid; m < RN_TS; m += RN_THREADS) ldr[m] = 0.f;
-  __syncthreads();
-
-  for (int l = 0; l < f.L; ++l) {
-    for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
-      const int m = o / d, j = o - m * d;
-      if (m0 + m < a.n) a.saved[((int64_t)l * a.n + m0 + m) * d + j] = xs[m * ldx + j];
-    }
-    const int32_t* lay = rn_lay(f, l);
-    const int dc = lay[0], dtr = lay[1];
-    const int32_t* cond = lay + 2;
-    const int32_t* trans = lay + 2 + d;
-    rn_load_cond(xs, ldx, cond, dc, sm.d4, cT);
-    __syncthreads();
-    for (int p = 0; p < 2; ++p) {
-      const RnPk pk(f.packed + rn_pk(d, h, l, p), sm.d4, sm.h4);
-      rn_wide<0>(pk.W1T, pk.b1, dc, sm.h4, cT, hT, nullptr);
-      __syncthreads();
-      rn_narrow(pk.W2T, sm.d4, pk.b2c, h, dtr, hT, p == 0 ? sT : tT);
-      __syncthreads();
-    }
-    // coupling on the transformed dims; sT keeps s for the log-det sum
-    for (int o = tid; o < dtr * RN_TS; o += RN_THREADS) {
-      const int i = o / RN_TS, m = o - i * RN_TS;
-      const int j = trans[i];
-      const float s = tanhf(sT[o]) * f.dt;
-      const float t = tT[o] * f.dt;
-      const float x = xs[m * ldx + j];
-      xs[m * ldx + j] = (x + t) * expf(s);
-      sT[o] = s;
-    }
-    __syncthreads();
-    for (int m = tid; m < RN_TS; m += RN_THREADS) {
-      float s = 0.f;
-      for (int i = 0; i < dtr; ++i) s += sT[i * RN_TS + m];
-      ldr[m] += s;
-    }
-    __syncthreads();
-  }
-  // ---- outputs
-  for (int m = tid; m < RN_TS; m += RN_THREADS) {
-    const int64_t row = m0 + m;
-    if (row >= a.n) continue;
-    float ld = ldr[m];
-    if (a.flags & RN_BASE) {
-      // log N(y; 0, I) (realNVP.py:211-213: the standard normal, not base_dist)
-      float q = 0.f;
-      for (int j = 0; j < d; ++j) {
-        const float y = xs[m * ldx + j];
-        q += y * y;
-        if (a.gy_out) a.gy_out[row * d + j] = -a.g_logp[row] * y;
-      }
-      ld += -0.5f * q - 0.91893853320467274f * (float)d;
-    }
-    if (a.logdet) a.logdet[row] = ld;
-  }
-  if (a.x_out) {
-    for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
-      const int m = o / d, j = o - m * d;
-      const int64_t row = m0 + m;
-      if (row >= a.n) continue;
-      a.x_out[row * d + j] = xs[m * ldx + j];
-    }
-  }
-}
-
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4_t rn_mfma(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ f32x4_t rn_ld4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
+__device__ __forceinline__ float rn_relu(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, INFINITY); }
+
+// A state row's conditioning dims 16 k + 4e + q, e = 0..3, as a lane's four
+// k-steps (padding 0); xr: the row of the lane's sample
+__device__ __forceinline__ f32x4_t rn_cond4(const RnFr& f, const float* xr, int k, int q, int dc) {
+  const int4 ci = *reinterpret_cast<const int4*>(f.condf + 16 * k + 4 * q);
+  const f32x4_t v{xr[ci.x], xr[ci.y], xr[ci.z], xr[ci.w]};
+  const int i = 16 * k + q;
+  return f32x4_t{i < dc ? v[0] : 0.f, i + 4 < dc ? v[1] : 0.f, i + 8 < dc ? v[2] : 0.f, i + 12 < dc ? v[3] : 0.f};
+}
 
 // One hidden block's weight fragments (a lane's share), requested one block
 // ahead of their use. Block indices past the end repeat the last block, so
@@ -513,18 +269,16 @@ __device__ __forceinline__ void rn_mlp(const RnFr& f, int r0, int hb0, int hs, i
     for (int k = NB; k < f.KC; ++k) {  // more conditioning dims than the registers hold
       const f32x4_t w = rn_ld4(f.W1f + ((int64_t)hb * f.KC + k) * 256 + 4 * lane);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 16 * k + 4 * (lane >> 4) + e;
-        const int j = f.cond[i];
+      for (int m = 0; m < MB; ++m) {
+        const f32x4_t cv = rn_cond4(f, xs + (16 * m + (lane & 15)) * ldx, k, lane >> 4, dc);
 #pragma unroll
-        for (int m = 0; m < MB; ++m)
-          a[m] = rn_mfma(w[e], i < dc ? xs[(16 * m + (lane & 15)) * ldx + j] : 0.f, a[m]);
+        for (int e = 0; e < 4; ++e) a[m] = rn_mfma(w[e], cv[e], a[m]);
       }
     }
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[m][e] = __builtin_amdgcn_fmed3f(a[m][e], 0.f, INFINITY);
+      for (int e = 0; e < 4; ++e) a[m][e] = rn_relu(a[m][e]);
 #pragma unroll
     for (int r = 0; r < NB; ++r)
       if (r0 + r < f.R) {
@@ -611,19 +365,13 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
     const int l = (a.dir == 0) ? step : f.L - 1 - step;
     const int32_t* lay = rn_lay(f, l);
     const int dc = lay[0], dtr = lay[1];
-    const RnFr fs(f.packed, d, h, f.L, l, 0, dc, dtr), ft(f.packed, d, h, f.L, l, 1, dc, dtr);
+    const RnFr fs(f.packed, d, h, l, 0, dc, dtr), ft(f.packed, d, h, l, 1, dc, dtr);
     f32x4_t c[NB][MB];  // conditioning inputs as MFMA operands
 #pragma unroll
     for (int k = 0; k < NB; ++k)
       if (k < fs.KC) {
-        const int4 ci = *reinterpret_cast<const int4*>(fs.cond + 16 * k + 4 * q);
-        const int i0 = 16 * k + 4 * q;
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-          const float* xr = xs + (16 * m + col) * ldx;
-          c[k][m] = f32x4_t{i0 < dc ? xr[ci.x] : 0.f, i0 + 1 < dc ? xr[ci.y] : 0.f, i0 + 2 < dc ? xr[ci.z] : 0.f,
-                            i0 + 3 < dc ? xr[ci.w] : 0.f};
-        }
+        for (int m = 0; m < MB; ++m) c[k][m] = rn_cond4(fs, xs + (16 * m + col) * ldx, k, q, dc);
       }
     for (int r0 = 0; r0 < fs.R; r0 += NB) {
       f32x4_t os[NB][MB], ot[NB][MB];
@@ -706,16 +454,13 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
       if (a.logdet) a.logdet[row] = ld;
     }
   }
-  if (a.x_out || a.gy_out) {
+  if (a.x_out) {
     for (int o = t; o < S * d; o += NT) {
       const int m = o / d, j = o - m * d;
       if (m0 + m >= a.n) continue;
       float v = xs[m * ldx + j];
-      if (a.gy_out) a.gy_out[m0 * d + o] = -a.g_logp[m0 + m] * v;
-      if (a.x_out) {
-        if (a.dir != 0 && (a.flags & RN_STD)) v = v * sqrtf(dcov[(int64_t)j * d + j]) + dmean[j];
-        a.x_out[m0 * d + o] = v;
-      }
+      if (a.dir != 0 && (a.flags & RN_STD)) v = v * sqrtf(dcov[(int64_t)j * d + j]) + dmean[j];
+      a.x_out[m0 * d + o] = v;
     }
   }
 }
@@ -759,222 +504,701 @@ static int rn_pass_nb(hipStream_t st, const RnvpDev& f, const RnPassArgs& a, int
   }
 }
 
-// ------------------------------------------------------------- adjoint ---
-// One layer in the forward direction: recompute s, t; the coupling's
-// reverse sweep; per MLP the hidden gradient (W2^T g), its ReLU mask, the
-// tile's weight-gradient partials, and W1^T g into the conditioning dims.
-// partial layout per tile (one layer): for p = scale, shift:
-//   dW1 [h][d] (column k = k-th conditioning dim), db1 [h],
-//   dW2 [d][h] (row i = i-th transformed dim), db2 [d].
-struct RnBwdArgs {
-  int layer;
-  const float* x_in;  // [n, d] layer input
-  int64_t n;
-  const float* g_logp;
-  const float* gy;  // [n, d] dL/d(layer output)
-  float* gx;        // [n, d] dL/d(layer input)
-  float* part;      // [n_tiles, layer_size]
+// ------------------------------------------------------------ training ---
+// The forward pass of a training step (which saves every layer's input) and
+// the adjoint sweep. Both use workgroups of eight wavefronts on tiles of 16 MS
+// samples; wave 2k + p takes MLP p and share k of its hidden features.
+// The hidden layers of both, and of the outputs that carry the state from
+// layer to layer, are summed in one order (RnOrder): a ReLU mask that rounds
+// differently in two evaluations changes a weight gradient by a whole sample's
+// share.
+
+// One ordered block's weights (a lane's share). The first block's are requested
+// ahead of the barrier before their use, the others one block ahead.
+template <int NB>
+struct RnOrdW {
+  f32x4_t w1[NB], w2, b;
+  __device__ __forceinline__ void load(const RnFr& f, int blk, int r, int lane) {
+    const int kc = f.KC > 0 ? f.KC : 1;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) w1[k] = rn_ld4(f.W1s + ((int64_t)blk * kc + (k < kc ? k : kc - 1)) * 256 + 4 * lane);
+    w2 = rn_ld4(f.W2s + ((int64_t)blk * f.R + r) * 256 + 4 * lane);
+    b = rn_ld4(f.b1s + 16 * blk + 4 * (lane >> 4));
+  }
 };
 
-// out[a][b] = sum_m A[a][m] B[b][m] over the tile's 32 samples, 4x4 register
-// tiles; A has na rows (storage padded to na4), B nb rows (padded to nb4).
-__device__ __forceinline__ void rn_outer(const float* A, int na, const float* B, int nb, float* out, int ldo) {
-  const int na4 = (na + 3) >> 2, nb4 = (nb + 3) >> 2;
-  for (int o = threadIdx.x; o < na4 * nb4; o += RN_THREADS) {
-    const int ta = o / nb4, tb = o - ta * nb4;
-    float acc[4][4] = {};
-#pragma unroll 1
-    for (int q = 0; q < RN_Q; ++q) {
-      float4 av[4], bv[4];
+// What share k (of four) of an MLP's waves does in a round: row block r of
+// the round's 4 / Gw, chain groups gcol, gcol + Gw, .. (Gc of them).
+struct RnShare {
+  int lgw, rsel, gcol, lgc;  // log2 Gw; log2 Gc
+  __device__ RnShare(const RnOrder& od, int k) {
+    lgw = od.G >= 4 ? 2 : od.G >> 1;
+    lgc = od.G >= 16 ? 2 : od.G >= 8 ? 1 : 0;  // G is a power of two <= 16
+    rsel = k >> lgw;
+    gcol = k & ((1 << lgw) - 1);
+  }
+  __device__ int rows() const { return 4 >> lgw; }  // row blocks of a round
+  // first block of chain group gi (four groups pair up at twice their distance first: 0, 2, 1, 3)
+  __device__ int group(const RnOrder& od, int gi) const {
+    return (gcol + ((lgc == 2 ? ((gi & 1) << 1 | gi >> 1) : gi) << lgw)) * od.U;
+  }
+};
+
+// Row block r of an MLP's output for the wave's share of the hidden features:
+// out[m] = the pairwise sum of its chains. cF: the conditioning inputs as
+// fragments, [KC][MS][64] float4 in LDS (rn_cond4 of every lane); nx: the
+// weights of block group(od, 0).
+template <int NB, int MS>
+__device__ __forceinline__ void rn_ordered_out(const RnFr& f, const RnOrder& od, const RnShare& sh, int r,
+                                               RnOrdW<NB>& nx, const float* cF, f32x4_t (&out)[MS], int lane) {
+  const int groups = 1 << sh.lgc;
+  f32x4_t part[MS], c[NB][MS];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        av[u] = *reinterpret_cast<const float4*>(A + (4 * ta + u) * RN_TS + 4 * q);
-        bv[u] = *reinterpret_cast<const float4*>(B + (4 * tb + u) * RN_TS + 4 * q);
+  for (int k = 0; k < NB; ++k)
+    if (k < f.KC) {
+#pragma unroll
+      for (int m = 0; m < MS; ++m) c[k][m] = rn_ld4(cF + ((k * MS + m) * 64 + lane) * 4);
+    }
+  for (int gi = 0; gi < groups; ++gi) {
+    const int blk0 = sh.group(od, gi);
+    f32x4_t acc[4][MS];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = 0; m < MS; ++m) acc[i][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < od.U; ++u) {
+      const RnOrdW<NB> w = nx;
+      const int blk = blk0 + u;
+      nx.load(f, u + 1 < od.U ? blk + 1 : gi + 1 < groups ? sh.group(od, gi + 1) : blk, r, lane);
+      f32x4_t a[MS];
+#pragma unroll
+      for (int m = 0; m < MS; ++m) a[m] = w.b;
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (k < f.KC) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int m = 0; m < MS; ++m) a[m] = rn_mfma(w.w1[k][e], c[k][m][e], a[m]);
+        }
+      for (int k = NB; k < f.KC; ++k) {
+        const f32x4_t x1 = rn_ld4(f.W1s + ((int64_t)blk * f.KC + k) * 256 + 4 * lane);
+#pragma unroll
+        for (int m = 0; m < MS; ++m) {
+          const f32x4_t cv = rn_ld4(cF + ((k * MS + m) * 64 + lane) * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[m] = rn_mfma(x1[e], cv[e], a[m]);
+        }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int m = 0; m < MS; ++m)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          acc[u][v] += av[u].x * bv[v].x + av[u].y * bv[v].y + av[u].z * bv[v].z + av[u].w * bv[v].w;
+        for (int e = 0; e < 4; ++e) a[m][e] = rn_relu(a[m][e]);
+      if (od.Sg == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int m = 0; m < MS; ++m) acc[i][m] = rn_mfma(w.w2[i], a[m][i], acc[i][m]);
+      } else if (od.Sg == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int m = 0; m < MS; ++m) acc[i & 1][m] = rn_mfma(w.w2[i], a[m][i], acc[i & 1][m]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int m = 0; m < MS; ++m) acc[0][m] = rn_mfma(w.w2[i], a[m][i], acc[0][m]);
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int m = 0; m < MS; ++m) {
+      // the accumulators of absent chains are zero: v + 0 = v
+      const f32x4_t v = (acc[0][m] + acc[1][m]) + (acc[2][m] + acc[3][m]);
+      // group sums in the order 0, 1 | 2, 3: (0 + 1) + (2 + 3)
+      if (gi == 0)
+        out[m] = v;
+      else if (gi == 1)
+        out[m] = out[m] + v;
+      else if (gi == 2)
+        part[m] = v;
+      else
+        out[m] = out[m] + (part[m] + v);
+    }
+  }
+}
+
+// A wave's output for row block rd * rows() + rsel, 16 MS samples, into red.
+template <int NB, int MS>
+__device__ __forceinline__ void rn_round_out(const RnFr& f, const RnOrder& od, const RnShare& sh, int rd,
+                                             RnOrdW<NB>& nx, const float* cF, float* red, int wave, int lane) {
+  const int r = rd * sh.rows() + sh.rsel;
+  if (r >= f.R) return;
+  f32x4_t o[MS];
+  if (rd > 0) nx.load(f, sh.group(od, 0), r, lane);
+  rn_ordered_out<NB, MS>(f, od, sh, r, nx, cF, o, lane);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int ia = 4 * ta + u, ib = 4 * tb + v;
-        if (ia < na && ib < nb) out[(int64_t)ia * ldo + ib] = acc[u][v];
-      }
-  }
+  for (int m = 0; m < MS; ++m) *reinterpret_cast<f32x4_t*>(red + ((wave * MS + m) * 64 + lane) * 4) = o[m];
+}
+// ... and the sum of the waves' outputs for row block rsel of the round and
+// 16-sample group m (waves at distance 2 first)
+template <int MS>
+__device__ __forceinline__ f32x4_t rn_round_sum(const float* red, int p, int rsel, int lgw, int m, int lane) {
+  auto at = [&](int g) { return rn_ld4(red + (((2 * ((rsel << lgw) + g) + p) * MS + m) * 64 + lane) * 4); };
+  if (lgw == 2) return (at(0) + at(2)) + (at(1) + at(3));
+  if (lgw == 1) return at(0) + at(1);
+  return at(0);
 }
 
-__device__ __forceinline__ void rn_rowsum(const float* A, int na, float* out) {
-  for (int i = threadIdx.x; i < na; i += RN_THREADS) {
-    float s = 0.f;
-    for (int m = 0; m < RN_TS; ++m) s += A[i * RN_TS + m];
-    out[i] = s;
+// What the coupling of a row block needs from memory besides the outputs.
+struct RnCpl {
+  f32x4_t bs, bt;
+  int tj[4];
+  __device__ __forceinline__ void load(const RnFr& fs, const RnFr& ft, int r, int q) {
+    const int k0 = 16 * r + 4 * q;
+    bs = rn_ld4(fs.b2 + k0);
+    bt = rn_ld4(ft.b2 + k0);
+    const int4 ti = *reinterpret_cast<const int4*>(fs.trans + k0);
+    tj[0] = ti.x, tj[1] = ti.y, tj[2] = ti.z, tj[3] = ti.w;
   }
-}
+};
 
-__global__ void __launch_bounds__(RN_THREADS) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
+template <int NB, int MS>
+__global__ void __launch_bounds__(512) rnvp_train_pass_kernel(RnvpDev f, RnPassArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int d = f.d, h = f.h, l = a.layer;
-  const RnSmem sm(d, h, true);
-  float* xs = reinterpret_cast<float*>(smem + sm.xs);
-  float* gb = reinterpret_cast<float*>(smem + sm.gb);
-  float* cT = reinterpret_cast<float*>(smem + sm.cT);
-  float* hT = reinterpret_cast<float*>(smem + sm.hT);
-  float* ghT = reinterpret_cast<float*>(smem + sm.ghT);
-  float* sT = reinterpret_cast<float*>(smem + sm.sT);
-  float* tT = reinterpret_cast<float*>(smem + sm.tT);
-  float* gcT = reinterpret_cast<float*>(smem + sm.gcT);
-  float* glp = reinterpret_cast<float*>(smem + sm.glp);
-  const int tid = threadIdx.x, ldx = sm.ldx;
-  const int64_t m0 = (int64_t)blockIdx.x * RN_TS;
-  const int32_t* lay = rn_lay(f, l);
-  const int dc = lay[0], dtr = lay[1];
-  const int32_t* cond = lay + 2;
-  const int32_t* trans = lay + 2 + d;
-
-  for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
+  constexpr int S = 16 * MS, NT = 512;
+  const int d = f.d, h = f.h, ldx = d + 1, t = threadIdx.x;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), col = lane & 15, q = lane >> 4;
+  float* xs = reinterpret_cast<float*>(smem);
+  float* red = xs + rn_rup16(S * ldx * 4) / 4;  // [8][MS][64] float4
+  float* ldp = red + 8 * MS * 256;              // [8][S] log-dets by wave
+  float* cF = ldp + 8 * S;                      // [KC][MS][64] float4
+  const int64_t m0 = (int64_t)blockIdx.x * S;
+  const float* dmean = f.theta + rn_stats(d, h, f.L);
+  const float* dcov = dmean + d;
+  for (int o = t; o < S * d; o += NT) {
     const int m = o / d, j = o - m * d;
-    const int64_t row = m0 + m;
-    const bool ok = row < a.n;
-    xs[m * ldx + j] = ok ? a.x_in[row * d + j] : 0.f;
-    gb[m * ldx + j] = ok ? a.gy[row * d + j] : 0.f;
-  }
-  for (int m = tid; m < RN_TS; m += RN_THREADS) glp[m] = (m0 + m < a.n) ? a.g_logp[m0 + m] : 0.f;
-  __syncthreads();
-  rn_load_cond(xs, ldx, cond, dc, sm.d4, cT);
-  __syncthreads();
-  // ---- recompute scale / shift pre-activations
-  for (int p = 0; p < 2; ++p) {
-    const RnPk pk(f.packed + rn_pk(d, h, l, p), sm.d4, sm.h4);
-    rn_wide<0>(pk.W1T, pk.b1, dc, sm.h4, cT, hT, nullptr);
-    __syncthreads();
-    rn_narrow(pk.W2T, sm.d4, pk.b2c, h, dtr, hT, p == 0 ? sT : tT);
-    __syncthreads();
-  }
-  // ---- coupling reverse sweep: y = (x + t) e^s, log-det += s
-  //   g_x = g e^s (transformed dim), g_t = g e^s, g_s = g y + g_logp;
-  //   g_spre = g_s dt (1 - tanh^2), g_tpre = g_t dt (in place of sT / tT;
-  //   their padding rows stay zero)
-  for (int o = tid; o < dtr * RN_TS; o += RN_THREADS) {
-    const int i = o / RN_TS, m = o - i * RN_TS;
-    const int j = trans[i];
-    const float tn = tanhf(sT[o]);
-    const float s = tn * f.dt;
-    const float t = tT[o] * f.dt;
-    const float e = expf(s);
-    const float x = xs[m * ldx + j];
-    const float y = (x + t) * e;
-    const float g = gb[m * ldx + j];
-    const float ge = g * e;
-    gb[m * ldx + j] = ge;
-    sT[o] = (g * y + glp[m]) * f.dt * (1.f - tn * tn);
-    tT[o] = ge * f.dt;
-  }
-  __syncthreads();
-  float* part = a.part + (int64_t)blockIdx.x * rn_layer_size(d, h);
-  for (int p = 0; p < 2; ++p) {
-    const RnPk pk(f.packed + rn_pk(d, h, l, p), sm.d4, sm.h4);
-    const float* goT = (p == 0) ? sT : tT;
-    float* pp = part + p * rn_mlp_size(d, h);
-    rn_wide<0>(pk.W1T, pk.b1, dc, sm.h4, cT, hT, nullptr);
-    __syncthreads();
-    // g_H[j][m] = sum_i W2[trans_i][j] g_out[i][m], masked by ReLU' (H > 0)
-    rn_wide<1>(pk.W2c, nullptr, dtr, sm.h4, goT, ghT, hT);
-    __syncthreads();
-    // tile partials: dW1[j][k] = sum_m gH[j][m] c[k][m]; db1; dW2[i][j] = sum_m g_out[i][m] H[j][m]; db2
-    rn_outer(ghT, h, cT, dc, pp, d);
-    rn_rowsum(ghT, h, pp + (int64_t)h * d);
-    rn_outer(goT, dtr, hT, h, pp + (int64_t)h * d + h, h);
-    rn_rowsum(goT, dtr, pp + 2LL * h * d + h);
-    // g_c[k][m] = sum_j W1[j][cond_k] gH[j][m], added to the conditioning dims
-    rn_narrow(pk.W1c, sm.d4, nullptr, h, dc, ghT, gcT);
-    __syncthreads();
-    for (int o = tid; o < dc * RN_TS; o += RN_THREADS) {
-      const int k = o / RN_TS, m = o - k * RN_TS;
-      gb[m * ldx + cond[k]] += gcT[o];
+    float v = 0.f;
+    if (m0 + m < a.n) {
+      v = a.x_in[m0 * d + o];
+      if (a.flags & RN_STD) v = (v - dmean[j]) / sqrtf(dcov[(int64_t)j * d + j]);
     }
+    xs[m * ldx + j] = v;
+  }
+  for (int o = t; o < 8 * S; o += NT) ldp[o] = 0.f;
+  __syncthreads();
+  for (int l = 0; l < f.L; ++l) {
+    if (a.saved) {
+      for (int o = t; o < S * d; o += NT) {
+        const int m = o / d, j = o - m * d;
+        if (m0 + m < a.n) a.saved[((int64_t)l * a.n + m0) * d + o] = xs[m * ldx + j];
+      }
+    }
+    const int32_t* lay = rn_lay(f, l);
+    const int dc = lay[0], dtr = lay[1];
+    const RnFr fs(f.packed, d, h, l, 0, dc, dtr), ft(f.packed, d, h, l, 1, dc, dtr);
+    const RnOrder od(dtr, h);
+    const RnShare sh(od, wave >> 1);
+    const RnFr& fp = (wave & 1) ? ft : fs;
+    const int rpr = sh.rows();
+    RnOrdW<NB> nx;
+    if (sh.rsel < fs.R) nx.load(fp, sh.group(od, 0), sh.rsel, lane);
+    RnCpl cp;  // of the wave's first coupling task
+    if (wave < rpr * MS && wave / MS < fs.R) cp.load(fs, ft, wave / MS, q);
+    for (int u = wave; u < fs.KC * MS; u += 8)
+      *reinterpret_cast<f32x4_t*>(cF + (u * 64 + lane) * 4) = rn_cond4(fs, xs + (16 * (u % MS) + col) * ldx, u / MS, q, dc);
     __syncthreads();
+    for (int rd = 0; rd * rpr < fs.R; ++rd) {
+      rn_round_out<NB, MS>(fp, od, sh, rd, nx, cF, red, wave, lane);
+      __syncthreads();
+      for (int k = wave; k < rpr * MS; k += 8) {
+        const int rsel = k / MS, m = k - rsel * MS, r = rd * rpr + rsel;
+        if (r >= fs.R) continue;
+        const int k0 = 16 * r + 4 * q;
+        if (rd > 0 || k >= 8) cp.load(fs, ft, r, q);
+        const f32x4_t sv = rn_round_sum<MS>(red, 0, rsel, sh.lgw, m, lane), tv = rn_round_sum<MS>(red, 1, rsel, sh.lgw, m, lane);
+        const f32x4_t bs = cp.bs, bt = cp.bt;
+        const int (&tj)[4] = cp.tj;
+        float ls = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (k0 + e < dtr) {
+            float* xp = xs + (16 * m + col) * ldx + tj[e];
+            const float s = tanhf(sv[e] + bs[e]) * f.dt;
+            const float tt = (tv[e] + bt[e]) * f.dt;
+            *xp = (*xp + tt) * expf(s);
+            ls += s;
+          }
+        ls += __shfl_xor(ls, 16, 64);
+        ls += __shfl_xor(ls, 32, 64);
+        if (lane < 16) ldp[wave * S + 16 * m + col] += ls;
+      }
+      __syncthreads();
+    }
   }
-  for (int o = tid; o < RN_TS * d; o += RN_THREADS) {
+  for (int m = t; m < S; m += NT) {
+    if (m0 + m >= a.n) continue;
+    float ld = 0.f;
+    for (int w = 0; w < 8; ++w) ld += ldp[w * S + m];
+    if (a.flags & RN_BASE) {
+      // log N(y; 0, I) (realNVP.py:211-213: the standard normal, not base_dist)
+      float s2 = 0.f;
+      for (int j = 0; j < d; ++j) s2 += xs[m * ldx + j] * xs[m * ldx + j];
+      ld += -0.5f * s2 - 0.91893853320467274f * (float)d;
+    }
+    if (a.logdet) a.logdet[m0 + m] = ld;
+  }
+  if (a.gy_out || a.x_out) {
+    for (int o = t; o < S * d; o += NT) {
+      const int m = o / d, j = o - m * d;
+      if (m0 + m >= a.n) continue;
+      const float v = xs[m * ldx + j];
+      if (a.gy_out) a.gy_out[m0 * d + o] = -a.g_logp[m0 + m] * v;
+      if (a.x_out) a.x_out[m0 * d + o] = v;
+    }
+  }
+}
+
+// ------------------------------------------------------------- adjoint ---
+// Layers l1-1 .. l0 of the forward direction for one tile: recompute s, t;
+// the coupling's reverse sweep; per MLP the hidden gradient gH = W2^T g, its
+// ReLU mask, the tile's weight gradients and W1^T gH into the conditioning
+// dims. H and gH are formed in both orientations (features x samples for the
+// next product, samples x features as the operands of the weight gradients,
+// whose k runs over the samples): swapping the operands of the product costs
+// one more pass of the matrix core where a transpose would go through LDS.
+// Weight gradients of a tile go to memory in fragment order, per (layer,
+// tile) and p: dW1 [hb][kg][64] float4 (element i of lane l: feature 16 hb +
+// 4 (l / 16) + i, dim 16 kg + l % 16), dW2 [hb][r][64] (dim 16 r + 4 (l / 16)
+// + i, feature 16 hb + l % 16), db1 [16 HB], db2 [16 R].
+struct RnBwdArgs {
+  int l0, l1;
+  const float* x;  // [l1 - l0, n, d] layer inputs, from layer l0
+  int64_t n;
+  const float* g_logp;
+  const float* gy;  // [n, d] dL/d(output of layer l1 - 1)
+  float* gx;        // [n, d] dL/d(input of layer l0)
+  float* part;      // [l1 - l0, tiles, rn_part_row]
+};
+
+__host__ __device__ inline int64_t rn_part_mlp(int hb, int kc, int r) { return 256LL * hb * (kc + r) + 16 * hb + 16 * r; }
+__host__ __device__ inline int64_t rn_part_row(int d, int h) {  // KC + R <= ceil(d / 16) + 1, R <= ceil(d / 16)
+  return 2 * (256LL * rn_b16(h) * (rn_b16(d) + 1) + 16LL * rn_b16(h) + 16LL * rn_b16(d));
+}
+
+template <int NB>
+struct RnBwdFrag {
+  f32x4_t w1[NB], w2t[NB], w1t[NB], b;
+  float bc;
+  __device__ __forceinline__ void load(const RnFr& f, int hb, int k0, int lane) {
+    const int kc = f.KC > 0 ? f.KC : 1, rc = f.R > 0 ? f.R : 1;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      w1[k] = rn_ld4(f.W1f + ((int64_t)hb * kc + (k < kc ? k : kc - 1)) * 256 + 4 * lane);
+      w2t[k] = rn_ld4(f.W2t + ((int64_t)hb * rc + (k < rc ? k : rc - 1)) * 256 + 4 * lane);
+      w1t[k] = rn_ld4(f.W1t + ((int64_t)hb * kc + (k0 + k < kc ? k0 + k : kc - 1)) * 256 + 4 * lane);
+    }
+    b = rn_ld4(f.b1 + 16 * hb + 4 * (lane >> 4));
+    bc = f.b1[16 * hb + (lane & 15)];
+  }
+};
+
+template <int NB, int MS>
+__global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int S = 16 * MS, NT = 512;
+  const int d = f.d, h = f.h, ldx = d + 1, t = threadIdx.x;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), col = lane & 15, q = lane >> 4;
+  const int p = wave & 1, share = wave >> 1;
+  float* gb = reinterpret_cast<float*>(smem);  // [S][ldx] gradient of the state
+  float* glp = gb + rn_rup16(S * ldx * 4) / 4;  // [S]
+  float* red = glp + S;                         // [8][NB][MS][64] float4
+  // fragments [block][MS][64] float4 of the conditioning inputs, then of the
+  // gradients of the scale and of the shift outputs: F with the product's k
+  // over the dims, T with k over the samples
+  float* cF = red + 8 * NB * MS * 256;
+  const int64_t m0 = (int64_t)blockIdx.x * S;
+  const f32x4_t zero{0.f, 0.f, 0.f, 0.f};
+
+  for (int o = t; o < S * d; o += NT) {
     const int m = o / d, j = o - m * d;
-    const int64_t row = m0 + m;
-    if (row < a.n) a.gx[row * d + j] = gb[m * ldx + j];
+    gb[m * ldx + j] = m0 + m < a.n ? a.gy[m0 * d + o] : 0.f;
+  }
+  for (int m = t; m < S; m += NT) glp[m] = m0 + m < a.n ? a.g_logp[m0 + m] : 0.f;
+
+  for (int l = a.l1 - 1; l >= a.l0; --l) {
+    const float* x = a.x + (int64_t)(l - a.l0) * a.n * d;
+    auto x_at = [&](int m, int j) {  // entry j of the tile's sample m (0 past the batch)
+      const int64_t row = m0 + m < a.n ? m0 + m : a.n - 1;
+      const float v = x[row * d + j];
+      return m0 + m < a.n ? v : 0.f;
+    };
+    const int32_t* lay = rn_lay(f, l);
+    const int dc = lay[0], dtr = lay[1];
+    const RnFr fs(f.packed, d, h, l, 0, dc, dtr), ft(f.packed, d, h, l, 1, dc, dtr);
+    const RnFr& fp = p ? ft : fs;
+    const RnOrder od(dtr, h);
+    const RnShare sh(od, share);
+    const int rpr = sh.rows(), KC = fs.KC, R = fs.R, HB = fs.HB;
+    float* cT = cF + KC * MS * 256;
+    float* gF = cT + KC * MS * 256;       // [2][R]
+    float* gT = gF + 2 * R * MS * 256;    // [2][R]
+    for (int u = wave; u < 2 * KC * MS; u += 8) {
+      const int v = u >> 1, k = v / MS, m = v - k * MS;
+      f32x4_t o;
+      int ci[4];
+      if (u & 1) {
+        ci[0] = ci[1] = ci[2] = ci[3] = fs.cond[16 * k + col];
+      } else {
+        const int4 c4 = *reinterpret_cast<const int4*>(fs.condf + 16 * k + 4 * q);
+        ci[0] = c4.x, ci[1] = c4.y, ci[2] = c4.z, ci[3] = c4.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float xv = x_at(16 * m + ((u & 1) ? 4 * q + e : col), ci[e]);
+        o[e] = 16 * k + ((u & 1) ? col : 4 * e + q) < dc ? xv : 0.f;
+      }
+      *reinterpret_cast<f32x4_t*>(((u & 1) ? cT : cF) + (v * 64 + lane) * 4) = o;
+    }
+    RnOrdW<NB> nx;
+    if (sh.rsel < R) nx.load(fp, sh.group(od, 0), sh.rsel, lane);
+    RnCpl cp;  // of the wave's first coupling task, with its samples' inputs
+    float xv[4];
+    auto cpl = [&](int r, int m) {
+      cp.load(fs, ft, r, q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xv[e] = x_at(16 * m + col, cp.tj[e]);
+    };
+    if (wave < rpr * MS && wave / MS < R) cpl(wave / MS, wave % MS);
+    __syncthreads();
+    RnBwdFrag<NB> w, wn;
+    // ---- scale / shift, then the coupling's reverse sweep: y = (x + t) e^s,
+    // log-det += s:  g_x = g e^s, g_t = g e^s, g_s = g y + g_logp;
+    // g_spre = g_s dt (1 - tanh^2), g_tpre = g_t dt
+    for (int rd = 0; rd * rpr < R; ++rd) {
+      rn_round_out<NB, MS>(fp, od, sh, rd, nx, cF, red, wave, lane);
+      if (rd == 0 && share < HB) wn.load(fp, share, 0, lane);
+      __syncthreads();
+      for (int k = wave; k < rpr * MS; k += 8) {
+        const int rsel = k / MS, m = k - rsel * MS, r = rd * rpr + rsel;
+        if (r >= R) continue;
+        const int k0 = 16 * r + 4 * q, ms = 16 * m + col;
+        if (rd > 0 || k >= 8) cpl(r, m);
+        const f32x4_t sv = rn_round_sum<MS>(red, 0, rsel, sh.lgw, m, lane), tv = rn_round_sum<MS>(red, 1, rsel, sh.lgw, m, lane);
+        const f32x4_t bs = cp.bs, bt = cp.bt;
+        const int (&tj)[4] = cp.tj;
+        float* oF = gF + (r * MS + m) * 256;
+        float* oT = gT + (r * MS + m) * 256;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float g1 = 0.f, g2 = 0.f;
+          if (k0 + e < dtr) {
+            const float tn = tanhf(sv[e] + bs[e]);
+            const float s = tn * f.dt;
+            const float tt = (tv[e] + bt[e]) * f.dt;
+            const float es = expf(s);
+            const float y = (xv[e] + tt) * es;
+            const float g = gb[ms * ldx + tj[e]];
+            const float ge = g * es;
+            gb[ms * ldx + tj[e]] = ge;
+            g1 = (g * y + glp[ms]) * f.dt * (1.f - tn * tn);
+            g2 = ge * f.dt;
+          }
+          // dim 4q + e of sample col: k-step q of lane (col, e) / k-step col % 4
+          // of lane (4q + e, col / 4)
+          const int iF = (col + 16 * e) * 4 + q, iT = (4 * q + e + 16 * (col >> 2)) * 4 + (col & 3);
+          oF[iF] = g1;
+          oT[iT] = g1;
+          oF[R * MS * 256 + iF] = g2;
+          oT[R * MS * 256 + iT] = g2;
+        }
+      }
+      __syncthreads();
+    }
+    // ---- per MLP (p) and hidden block (share, share + 4, ..)
+    const float* gpF = gF + p * R * MS * 256;
+    const float* gpT = gT + p * R * MS * 256;
+    auto frag = [&](const float* v, int blk, int m) { return rn_ld4(v + ((blk * MS + m) * 64 + lane) * 4); };
+    float* pp = a.part + ((int64_t)(l - a.l0) * gridDim.x + blockIdx.x) * rn_part_row(d, h) + p * rn_part_mlp(HB, KC, R);
+    float* pw2 = pp + 256LL * HB * KC;
+    float* pb1 = pw2 + 256LL * HB * R;
+    for (int k0 = 0; k0 == 0 || k0 < KC || k0 < R; k0 += NB) {
+      f32x4_t gc[NB][MS];
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int m = 0; m < MS; ++m) gc[k][m] = zero;
+      if ((k0 > 0 || R == 0) && share < HB) wn.load(fp, share, k0, lane);
+      for (int hb = share; hb < HB; hb += 4) {
+        w = wn;
+        wn.load(fp, hb + 4 < HB ? hb + 4 : hb, k0, lane);
+        f32x4_t o1[NB], o2[NB];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) o1[k] = o2[k] = zero;
+        float sb = 0.f;
+#pragma unroll
+        for (int m = 0; m < MS; ++m) {
+          f32x4_t H = w.b, Ht{w.bc, w.bc, w.bc, w.bc}, g = zero, gt = zero;
+#pragma unroll
+          for (int k = 0; k < NB; ++k)
+            if (k < KC) {
+              const f32x4_t cv = frag(cF, k, m);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                H = rn_mfma(w.w1[k][e], cv[e], H);
+                Ht = rn_mfma(cv[e], w.w1[k][e], Ht);
+              }
+            }
+          for (int k = NB; k < KC; ++k) {
+            const f32x4_t cv = frag(cF, k, m), x1 = rn_ld4(fp.W1f + ((int64_t)hb * KC + k) * 256 + 4 * lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              H = rn_mfma(x1[e], cv[e], H);
+              Ht = rn_mfma(cv[e], x1[e], Ht);
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < NB; ++r)
+            if (r < R) {
+              const f32x4_t gv = frag(gpF, r, m);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                g = rn_mfma(w.w2t[r][e], gv[e], g);
+                gt = rn_mfma(gv[e], w.w2t[r][e], gt);
+              }
+            }
+          for (int r = NB; r < R; ++r) {
+            const f32x4_t gv = frag(gpF, r, m), x2 = rn_ld4(fp.W2t + ((int64_t)hb * R + r) * 256 + 4 * lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              g = rn_mfma(x2[e], gv[e], g);
+              gt = rn_mfma(gv[e], x2[e], gt);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            g[e] = H[e] > 0.f ? g[e] : 0.f;
+            gt[e] = Ht[e] > 0.f ? gt[e] : 0.f;
+            Ht[e] = rn_relu(Ht[e]);
+            sb += gt[e];
+          }
+#pragma unroll
+          for (int k = 0; k < NB; ++k)
+            if (k0 + k < KC) {
+              const f32x4_t cv = frag(cT, k0 + k, m);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                gc[k][m] = rn_mfma(w.w1t[k][e], g[e], gc[k][m]);
+                o1[k] = rn_mfma(gt[e], cv[e], o1[k]);
+              }
+            }
+#pragma unroll
+          for (int r = 0; r < NB; ++r)
+            if (k0 + r < R) {
+              const f32x4_t gv = frag(gpT, k0 + r, m);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o2[r] = rn_mfma(gv[e], Ht[e], o2[r]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          if (k0 + k < KC) *reinterpret_cast<f32x4_t*>(pp + ((int64_t)hb * KC + k0 + k) * 256 + 4 * lane) = o1[k];
+          if (k0 + k < R) *reinterpret_cast<f32x4_t*>(pw2 + ((int64_t)hb * R + k0 + k) * 256 + 4 * lane) = o2[k];
+        }
+        if (k0 == 0) {
+          sb += __shfl_xor(sb, 16, 64);
+          sb += __shfl_xor(sb, 32, 64);
+          if (lane < 16) pb1[16 * hb + lane] = sb;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (k0 + k < KC) {
+#pragma unroll
+          for (int m = 0; m < MS; ++m)
+            *reinterpret_cast<f32x4_t*>(red + (((wave * NB + k) * MS + m) * 64 + lane) * 4) = gc[k][m];
+        }
+      __syncthreads();
+      for (int u = wave; u < NB * MS; u += 8) {  // conditioning-input gradients: all shares of both MLPs
+        const int k = u / MS, m = u - k * MS;
+        if (k0 + k >= KC) continue;
+        f32x4_t v = zero;
+#pragma unroll
+        for (int w8 = 0; w8 < 8; ++w8) v += rn_ld4(red + (((w8 * NB + k) * MS + m) * 64 + lane) * 4);
+        const int i0 = 16 * (k0 + k) + 4 * q;
+        const int4 ci = *reinterpret_cast<const int4*>(fs.cond + i0);
+        const int cj[4] = {ci.x, ci.y, ci.z, ci.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (i0 + e < dc) gb[(16 * m + col) * ldx + cj[e]] += v[e];
+      }
+      __syncthreads();
+    }
+    if (share == 0) {  // db2: sums over the samples
+      for (int r = 0; r < R; ++r) {
+        float s = 0.f;
+        for (int m = 0; m < MS; ++m) {
+          const f32x4_t gv = frag(gpT, r, m);
+          s += (gv[0] + gv[1]) + (gv[2] + gv[3]);
+        }
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        if (lane < 16) pb1[16 * HB + 16 * r + lane] = s;
+      }
+    }
+    __syncthreads();  // the fragments are rewritten by the next layer
+  }
+  for (int o = t; o < S * d; o += NT) {
+    const int m = o / d, j = o - m * d;
+    if (m0 + m < a.n) a.gx[m0 * d + o] = gb[m * ldx + j];
   }
 }
 
-// Sum of the tile partials of one layer, in two fixed-order stages so that
-// enough lanes stream the partial buffer: stage 1 sums chunk c of the tiles
-// (tiles c, c + C, c + 2C, ...) into row n_tiles + c of the buffer; stage 2
-// sums the C chunk rows in order and scatters the result to the
-// reference-shaped leaves of the gradient vector.
-constexpr int RN_RED_CHUNKS = 16;
-
-__host__ __device__ inline int rn_chunks(int64_t n_tiles) {
-  const int64_t c = (n_tiles + 15) / 16;
-  return (int)(c < 1 ? 1 : (c > RN_RED_CHUNKS ? RN_RED_CHUNKS : c));
-}
-
-__global__ void __launch_bounds__(256) rnvp_wgrad_stage1(int64_t LS, float* part, int64_t n_tiles, int C) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = blockIdx.y;
-  if (e >= LS) return;
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  int64_t t = c;
-  for (; t + 3 * C < n_tiles; t += 4 * C) {
-    s0 += part[t * LS + e];
-    s1 += part[(t + C) * LS + e];
-    s2 += part[(t + 2 * C) * LS + e];
-    s3 += part[(t + 3 * C) * LS + e];
-  }
-  for (; t < n_tiles; t += C) s0 += part[t * LS + e];
-  part[(n_tiles + c) * LS + e] = (s0 + s1) + (s2 + s3);
-}
-
-__global__ void __launch_bounds__(256) rnvp_wgrad_stage2(RnvpDev f, int l, const float* __restrict__ part,
-                                                         int64_t n_tiles, int C, float* __restrict__ grad) {
-  const int d = f.d, h = f.h;
-  const int64_t LS = rn_layer_size(d, h), MS = rn_mlp_size(d, h);
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= LS) return;
+// Sum of the tiles' weight gradients, scattered to the reference-shaped
+// leaves of the gradient vector: a workgroup takes 64 float4 of one layer,
+// wave w the tiles w, w + 4, .. in order; the four sums meet in LDS. Bound by
+// reading the tiles' rows (a wave reads 1 KB of one row at a time).
+__global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, const float* __restrict__ part, int tiles,
+                                                         float* __restrict__ grad) {
+  __shared__ f32x4_t sh[4][64];
+  const int d = f.d, h = f.h, l = l0 + blockIdx.y;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int32_t* lay = rn_lay(f, l);
-  const int dc = lay[0], dtr = lay[1];
+  const int dc = lay[0], dtr = lay[1], KC = rn_b16(dc), R = rn_b16(dtr), HB = rn_b16(h);
+  const int64_t pm = rn_part_mlp(HB, KC, R), row = rn_part_row(d, h);
+  const int64_t e4 = (int64_t)blockIdx.x * 64 + lane;
+  const bool in = 4 * e4 < 2 * pm;
+  f32x4_t v{0.f, 0.f, 0.f, 0.f};
+  if (in) {
+    const float* src = part + (int64_t)blockIdx.y * tiles * row + 4 * e4;
+    int t = w;
+    for (; t + 12 < tiles; t += 16) {
+      f32x4_t u[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) u[k] = rn_ld4(src + (int64_t)(t + 4 * k) * row);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v += u[k];
+    }
+    for (; t < tiles; t += 4) v += rn_ld4(src + (int64_t)t * row);
+  }
+  sh[w][lane] = v;
+  __syncthreads();
+  if (w != 0 || !in) return;
+  v = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+  const int p = 4 * e4 >= pm;
+  const int64_t r = 4 * e4 - p * pm, n1 = 256LL * HB * KC, n2 = n1 + 256LL * HB * R, n3 = n2 + 16 * HB;
+  float* W1 = grad + rn_mlp(d, h, l, p);
+  float* b1 = W1 + (int64_t)h * d;
+  float* W2 = b1 + h;
+  float* b2 = W2 + (int64_t)d * h;
   const int32_t* cond = lay + 2;
   const int32_t* trans = lay + 2 + d;
-  const int p = (int)(e / MS);
-  const int64_t r = e - p * MS;
-  int64_t dst = -1;
-  if (r < (int64_t)h * d) {
-    const int j = (int)(r / d), k = (int)(r - (int64_t)j * d);
-    if (k < dc) dst = (int64_t)j * d + cond[k];
-  } else if (r < (int64_t)h * d + h) {
-    dst = r;
-  } else if (r < 2LL * h * d + h) {
-    const int64_t rr = r - (int64_t)h * d - h;
-    const int i = (int)(rr / h), j = (int)(rr - (int64_t)i * h);
-    if (i < dtr) dst = (int64_t)h * d + h + (int64_t)trans[i] * h + j;
-  } else {
-    const int i = (int)(r - 2LL * h * d - h);
-    if (i < dtr) dst = 2LL * h * d + h + trans[i];
+  const int fl = (int)(r >> 2) & 63, c = fl & 15, q = fl >> 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (r < n1) {
+      const int b = (int)(r >> 8), hb = b / KC, j = 16 * hb + 4 * q + i, k = 16 * (b - hb * KC) + c;
+      if (j < h && k < dc) W1[(int64_t)j * d + cond[k]] = v[i];
+    } else if (r < n2) {
+      const int b = (int)((r - n1) >> 8), hb = b / R, k = 16 * (b - hb * R) + 4 * q + i, j = 16 * hb + c;
+      if (j < h && k < dtr) W2[(int64_t)trans[k] * h + j] = v[i];
+    } else if (r < n3) {
+      const int j = (int)(r - n2) + i;
+      if (j < h) b1[j] = v[i];
+    } else {
+      const int k = (int)(r - n3) + i;
+      if (k < dtr) b2[trans[k]] = v[i];
+    }
   }
-  if (dst < 0) return;
-  float s = 0.f;
-  for (int c = 0; c < C; ++c) s += part[(n_tiles + c) * LS + e];
-  grad[rn_mlp(d, h, l, p) + dst] = s;
 }
 
+// ---------------------------------------------------------------- host ---
 static int check_rnvp(const fmc_rnvp* r, RnvpDev& f, bool need_packed) {
   FMC_ARG(r != nullptr, "RealNVP description is NULL");
   FMC_ARG(r->n_dim >= 1 && r->n_layers >= 1 && r->n_hidden >= 1, "n_dim, n_layers and n_hidden must be >= 1");
   FMC_ARG(r->theta != nullptr && r->layout != nullptr, "theta or layout is NULL");
   FMC_ARG(!need_packed || r->packed != nullptr, "packed buffer is NULL");
-  const RnSmem sm(r->n_dim, r->n_hidden, true);
-  FMC_ARG(sm.total <= 160 * 1024, "n_dim %d / n_hidden %d exceed the LDS budget of the RealNVP kernels",
-          r->n_dim, r->n_hidden);
+  // the sizes these kernels take: 16 samples' state, gradient and hidden rows in 160 KB
+  const int64_t d4 = (r->n_dim + 3) & ~3, h4 = (r->n_hidden + 3) & ~3;
+  const int64_t need = 2 * ((64LL * (r->n_dim + 1) + 15) & ~15LL) + 64 * (4 * d4 + 2 * h4) + 128;
+  FMC_ARG(need <= 160 * 1024, "n_dim %d / n_hidden %d exceed the LDS budget of the RealNVP kernels", r->n_dim,
+          r->n_hidden);
   f = RnvpDev{r->n_dim, r->n_layers, r->n_hidden, r->dt, r->theta, r->packed, r->layout};
   return FMC_OK;
+}
+
+// blocks of 16 dims held in registers: a mask that halves the dims fits (up
+// to 128 dims; past 256, two, for the adjoint's LDS)
+static inline int rn_nb(int d) {
+  const int nb = rn_b16((d + 1) / 2);
+  return nb <= 1 ? 1 : (nb <= 2 || d > 256) ? 2 : 4;
+}
+static inline int64_t rn_bwd_lds(int d, int nb, int ms) {
+  // fragments: 2 KC + 4 R blocks of 1 KB, KC + R <= ceil(d / 16) + 1
+  return (int64_t)rn_rup16(16 * ms * (d + 1) * 4) + 64 * ms + 8192LL * nb * ms + 1024LL * ms * (4 * rn_b16(d) + 2);
+}
+// 16-sample groups per workgroup of the training kernels: as many as leave one
+// workgroup a CU, up to three (four spill; measured at d = 32, 8 layers,
+// hidden 256, adjoint + forward, n = 10,000: one group 433 + 120 us, two 353 +
+// 134, three 237 + 85; n = 4000: 141 + 54, 177 + 68, 220 + 82)
+static int rn_ms(int64_t tiles16, int d) {
+  const int nb = rn_nb(d), cap = nb <= 2 ? 3 : 1;
+  int64_t ms = (tiles16 + 255) / 256;
+  ms = ms < 1 ? 1 : ms > cap ? cap : ms;
+  while (ms > 1 && rn_bwd_lds(d, nb, (int)ms) > 160 * 1024) --ms;
+  return (int)ms;
+}
+
+template <int NB, int MS>
+static int rn_launch_train(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) {
+  const size_t shm = (size_t)rn_rup16(16 * MS * (f.d + 1) * 4) + (8192 + 512 + 1024 * rn_b16(f.d)) * MS;
+  if (const int rc = rn_set_lds(rnvp_train_pass_kernel<NB, MS>, shm)) return rc;
+  const int64_t grid = (a.n + 16 * MS - 1) / (16 * MS);
+  FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
+  hipLaunchKernelGGL((rnvp_train_pass_kernel<NB, MS>), dim3((unsigned)grid), dim3(512), shm, st, f, a);
+  return check_launch("realnvp training pass");
+}
+
+template <int NB, int MS>
+static int rn_launch_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a) {
+  const size_t shm = (size_t)rn_bwd_lds(f.d, NB, MS);
+  if (const int rc = rn_set_lds(rnvp_bwd_kernel<NB, MS>, shm)) return rc;
+  const int64_t grid = (a.n + 16 * MS - 1) / (16 * MS);
+  FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
+  hipLaunchKernelGGL((rnvp_bwd_kernel<NB, MS>), dim3((unsigned)grid), dim3(512), shm, st, f, a);
+  return check_launch("realnvp adjoint");
+}
+
+static int rn_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a) {
+  switch (4 * rn_nb(f.d) + rn_ms((a.n + 15) / 16, f.d)) {
+    case 5: return rn_launch_bwd<1, 1>(st, f, a);
+    case 6: return rn_launch_bwd<1, 2>(st, f, a);
+    case 7: return rn_launch_bwd<1, 3>(st, f, a);
+    case 9: return rn_launch_bwd<2, 1>(st, f, a);
+    case 10: return rn_launch_bwd<2, 2>(st, f, a);
+    case 11: return rn_launch_bwd<2, 3>(st, f, a);
+    default: return rn_launch_bwd<4, 1>(st, f, a);
+  }
+}
+
+static int rn_train_pass(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) {
+  switch (4 * rn_nb(f.d) + rn_ms((a.n + 15) / 16, f.d)) {
+    case 5: return rn_launch_train<1, 1>(st, f, a);
+    case 6: return rn_launch_train<1, 2>(st, f, a);
+    case 7: return rn_launch_train<1, 3>(st, f, a);
+    case 9: return rn_launch_train<2, 1>(st, f, a);
+    case 10: return rn_launch_train<2, 2>(st, f, a);
+    case 11: return rn_launch_train<2, 3>(st, f, a);
+    default: return rn_launch_train<4, 1>(st, f, a);
+  }
+}
+
+static int rn_wgrad(hipStream_t st, const RnvpDev& f, int l0, int nl, const float* part, int64_t tiles16, float* grad) {
+  const int ms = rn_ms(tiles16, f.d);
+  const int64_t tiles = (tiles16 + ms - 1) / ms;
+  const unsigned gx = (unsigned)((rn_part_row(f.d, f.h) / 4 + 63) / 64);
+  hipLaunchKernelGGL(rnvp_wgrad_kernel, dim3(gx, (unsigned)nl), dim3(256), 0, st, f, l0, part, (int)tiles, grad);
+  return check_launch("realnvp weight gradient");
 }
 
 }  // namespace fmc
@@ -988,8 +1212,8 @@ extern "C" int fmc_rnvp_sizes(const fmc_rnvp* r, int64_t* theta_size, int64_t* p
   if (rc) return rc;
   if (theta_size) *theta_size = rn_theta_size(f.d, f.h, f.L);
   if (packed_size) *packed_size = rn_packed_size(f.d, f.h, f.L);
-  if (partial_per_tile) *partial_per_tile = rn_layer_size(f.d, f.h);  // rows: tiles + chunk rows
-  if (tile) *tile = RN_TS;
+  if (partial_per_tile) *partial_per_tile = rn_part_row(f.d, f.h);
+  if (tile) *tile = 16;
   return FMC_OK;
 }
 
@@ -997,14 +1221,9 @@ extern "C" int fmc_rnvp_pack(void* stream, const fmc_rnvp* r) {
   RnvpDev f;
   int rc = check_rnvp(r, f, true);
   if (rc) return rc;
-  const int64_t n = rn_pk_mlp(f.d, f.h);
-  const unsigned gx = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
+  const unsigned gx = (unsigned)((rn_slot(f.d, f.h) / 4 + 255) / 256);
   hipLaunchKernelGGL(rnvp_pack_kernel, dim3(gx, 2 * f.L), dim3(256), 0, (hipStream_t)stream, f, r->packed);
-  if ((rc = check_launch("realnvp pack"))) return rc;
-  const int64_t nf = rn_fr_slot(f.d, f.h);
-  hipLaunchKernelGGL(rnvp_pack_frag_kernel, dim3((unsigned)((nf + 255) / 256 < 4096 ? (nf + 255) / 256 : 4096), 2 * f.L),
-                     dim3(256), 0, (hipStream_t)stream, f, r->packed);
-  return check_launch("realnvp pack (fragments)");
+  return check_launch("realnvp pack");
 }
 
 extern "C" int fmc_rnvp_pass(void* stream, const fmc_rnvp* r, int32_t dir, int32_t flags, const float* x_in,
@@ -1023,18 +1242,11 @@ extern "C" int fmc_rnvp_pass(void* stream, const fmc_rnvp* r, int32_t dir, int32
   if (n == 0) return FMC_OK;
   RnPassArgs a{dir, flags, x_in, n, key0, key1, sample0, x_out, logdet, saved, g_logp, gy_out};
   hipStream_t st = (hipStream_t)stream;
-  if (saved) {
-    const RnSmem sm(f.d, f.h, false);
-    if ((rc = rn_set_lds(rnvp_train_pass_kernel, (size_t)sm.total))) return rc;
-    const int64_t grid = (n + RN_TS - 1) / RN_TS;
-    FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
-    hipLaunchKernelGGL(rnvp_train_pass_kernel, dim3((unsigned)grid), dim3(RN_THREADS), (size_t)sm.total, st, f, a);
-    return check_launch("realnvp training pass");
-  }
-  const int nb = rn_b16((f.d + 1) / 2);  // blocks of a mask that halves the dims
+  if (saved || gy_out) return rn_train_pass(st, f, a);
+  const int nb = rn_nb(f.d);
   const int var = rn_pass_variant(n, f.d, f.h);
-  if (nb <= 1) return rn_pass_nb<1>(st, f, a, var);
-  if (nb <= 2) return rn_pass_nb<2>(st, f, a, var);
+  if (nb == 1) return rn_pass_nb<1>(st, f, a, var);
+  if (nb == 2) return rn_pass_nb<2>(st, f, a, var);
   return rn_pass_nb<4>(st, f, a, var);
 }
 
@@ -1048,16 +1260,11 @@ extern "C" int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* r, int32_t 
   FMC_ARG(n >= 0, "n < 0");
   FMC_ARG(x_in && g_logp && gy && gx && partials, "NULL pointer");
   FMC_ARG(gy != gx, "gx must not alias gy");
-  const int64_t tiles = (n + RN_TS - 1) / RN_TS;
+  const int64_t tiles = (n + 15) / 16;
   FMC_ARG(n_partial_tiles >= tiles, "partials hold %lld tiles, %lld needed", (long long)n_partial_tiles,
           (long long)tiles);
   if (n == 0) return FMC_OK;
-  const RnSmem sm(f.d, f.h, true);
-  if ((rc = rn_set_lds(rnvp_bwd_kernel, (size_t)sm.total))) return rc;
-  RnBwdArgs a{layer, x_in, n, g_logp, gy, gx, partials};
-  hipLaunchKernelGGL(rnvp_bwd_kernel, dim3((unsigned)tiles), dim3(RN_THREADS), (size_t)sm.total,
-                     (hipStream_t)stream, f, a);
-  return check_launch("realnvp adjoint");
+  return rn_bwd((hipStream_t)stream, f, RnBwdArgs{layer, layer + 1, x_in, n, g_logp, gy, gx, partials});
 }
 
 extern "C" int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* r, int32_t layer, float* partials,
@@ -1067,15 +1274,35 @@ extern "C" int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* r, int32_t lay
   if (rc) return rc;
   FMC_ARG(layer >= 0 && layer < f.L, "layer %d out of range", layer);
   FMC_ARG(partials && grad, "NULL pointer");
-  FMC_ARG(n_tiles >= 1, "n_tiles must be >= 1");
-  const int C = rn_chunks(n_tiles);
-  FMC_ARG(partial_rows >= n_tiles + C, "partials hold %lld rows, %lld needed (tiles + %d reduction rows)",
-          (long long)partial_rows, (long long)(n_tiles + C), C);
-  const int64_t LS = rn_layer_size(f.d, f.h);
-  const unsigned gx = (unsigned)((LS + 255) / 256);
-  hipLaunchKernelGGL(rnvp_wgrad_stage1, dim3(gx, C), dim3(256), 0, (hipStream_t)stream, LS, partials, n_tiles, C);
-  if ((rc = check_launch("realnvp weight gradient (tile sums)"))) return rc;
-  hipLaunchKernelGGL(rnvp_wgrad_stage2, dim3(gx), dim3(256), 0, (hipStream_t)stream, f, layer, partials, n_tiles,
-                     C, grad);
-  return check_launch("realnvp weight gradient");
+  FMC_ARG(n_tiles >= 1 && n_tiles <= 0x7fffffffLL, "n_tiles must be >= 1");
+  FMC_ARG(partial_rows >= n_tiles, "partials hold %lld rows, %lld needed", (long long)partial_rows, (long long)n_tiles);
+  return rn_wgrad((hipStream_t)stream, f, layer, 1, partials, n_tiles, grad);
+}
+
+extern "C" int fmc_rnvp_backward_ws_size(const fmc_rnvp* r, int64_t n, int64_t* floats) {
+  RnvpDev f;
+  int rc = check_rnvp(r, f, false);
+  if (rc) return rc;
+  FMC_ARG(n >= 1 && floats != nullptr, "n must be >= 1 and floats not NULL");
+  const int64_t t16 = (n + 15) / 16;
+  const int ms = rn_ms(t16, f.d);
+  *floats = (int64_t)f.L * ((t16 + ms - 1) / ms) * rn_part_row(f.d, f.h);
+  return FMC_OK;
+}
+
+extern "C" int fmc_rnvp_backward(void* stream, const fmc_rnvp* r, const float* saved, int64_t n, const float* g_logp,
+                                 const float* gy, float* gx, float* grad, float* workspace, int64_t workspace_floats) {
+  RnvpDev f;
+  int rc = check_rnvp(r, f, true);
+  if (rc) return rc;
+  FMC_ARG(n >= 1, "n must be >= 1");
+  FMC_ARG(saved && g_logp && gy && gx && grad && workspace, "NULL pointer");
+  FMC_ARG((uintptr_t)workspace % 16 == 0, "workspace must be 16-byte aligned");
+  int64_t need = 0;
+  if ((rc = fmc_rnvp_backward_ws_size(r, n, &need))) return rc;
+  FMC_ARG(workspace_floats >= need, "workspace holds %lld floats, need %lld (fmc_rnvp_backward_ws_size)",
+          (long long)workspace_floats, (long long)need);
+  hipStream_t st = (hipStream_t)stream;
+  if ((rc = rn_bwd(st, f, RnBwdArgs{0, f.L, saved, n, g_logp, gy, gx, workspace}))) return rc;
+  return rn_wgrad(st, f, 0, f.L, workspace, (n + 15) / 16, grad);
 }

@@ -1,7 +1,7 @@
 """RealNVP and AffineCoupling — src/flowMC/resource/model/nf_model/realNVP.py:18-228.
 
 All arithmetic runs in the RealNVP kernels of libflowmc_hip (fmc_rnvp_pass,
-fmc_rnvp_backward_layer, fmc_rnvp_weight_grad, fmc_adamw_clip). Parameters
+fmc_rnvp_backward, fmc_adamw_clip). Parameters
 live in one flat FP32 vector ``theta``: per layer the scale MLP (W1 [h, d],
 b1 [h], W2 [d, h], b2 [d]) and then the shift MLP, followed by data_mean,
 data_cov, base_mean and base_cov. The coupling masks of realNVP.py:155-158
@@ -54,9 +54,10 @@ class _Workspace:
         self.g_logp = torch.full((B,), -1.0 / B, dtype=torch.float32, device=dev)
         self.gy = torch.empty((B, d), dtype=torch.float32, device=dev)
         self.gx = torch.empty((B, d), dtype=torch.float32, device=dev)
-        self.n_tiles = (B + model._tile - 1) // model._tile
-        # tile rows plus the reduction's chunk rows (at most 16)
-        self.part = torch.empty((self.n_tiles + 16, model._part_per_tile), dtype=torch.float32, device=dev)
+        nf = C.c_int64(0)
+        _native.call("fmc_rnvp_backward_ws_size", C.byref(model._struct()), B, C.byref(nf))
+        self.part = torch.empty(nf.value, dtype=torch.float32, device=dev)  # weight gradients by layer and tile
+        # cleared once: the sweep writes every entry a masked coupling can make non-zero
         self.grad = torch.zeros(model.theta.numel(), dtype=torch.float32, device=dev)
         self.norm_ws = torch.empty(1024, dtype=torch.float64, device=dev)
         self.gnorm = torch.empty(1, dtype=torch.float32, device=dev)
@@ -68,9 +69,9 @@ class _RnvpBase(NFModel):
     def _configure(self):
         self.layout = _layout(self._masks, self._n_features, self.device)
         probe = self._struct(theta_ptr=1)
-        th, pk, pp, tile = C.c_int64(), C.c_int64(), C.c_int64(), C.c_int32()
-        _native.call("fmc_rnvp_sizes", C.byref(probe), C.byref(th), C.byref(pk), C.byref(pp), C.byref(tile))
-        self._theta_size, self._part_per_tile, self._tile = th.value, pp.value, tile.value
+        th, pk = C.c_int64(), C.c_int64()
+        _native.call("fmc_rnvp_sizes", C.byref(probe), C.byref(th), C.byref(pk), None, None)
+        self._theta_size = th.value
         self.packed = torch.empty(pk.value, dtype=torch.float32, device=self.device)
         d, h = self._n_features, self.n_hidden
         self._mlp_size = 2 * h * d + h + d
@@ -210,17 +211,12 @@ class _RnvpBase(NFModel):
         return ws
 
     def _backward(self, ws: _Workspace, B: int):
+        """The backward sweep over all layers; dL/d(input of layer 0) in ws.gx."""
         s = self._struct()
-        st = _native.stream_ptr()
-        ws.grad.zero_()
-        gy, gx = ws.gy, ws.gx
-        for layer in reversed(range(self.n_layers)):
-            _native.call("fmc_rnvp_backward_layer", st, C.byref(s), layer, ws.saved[layer].data_ptr(), B,
-                         ws.g_logp.data_ptr(), gy.data_ptr(), gx.data_ptr(), ws.part.data_ptr(), ws.n_tiles)
-            _native.call("fmc_rnvp_weight_grad", st, C.byref(s), layer, ws.part.data_ptr(), ws.n_tiles,
-                         ws.part.shape[0], ws.grad.data_ptr())
-            gy, gx = gx, gy
-        return gy  # dL/d(input of layer 0)
+        _native.call("fmc_rnvp_backward", _native.stream_ptr(), C.byref(s), ws.saved.data_ptr(), B,
+                     ws.g_logp.data_ptr(), ws.gy.data_ptr(), ws.gx.data_ptr(), ws.grad.data_ptr(), ws.part.data_ptr(),
+                     ws.part.numel())
+        return ws.gx
 
     def grad_log_prob_sum(self, x, g_logp=None):
         """Hand-written adjoint: d/dtheta of sum_i g_logp[i] * log_prob(x_i) (flat,
@@ -304,7 +300,7 @@ class RealNVP(_RnvpBase):
 
     def log_prob(self, x):
         """realNVP.py:207-214. Differentiable in x: the backward pass runs the
-        adjoint kernels (fmc_rnvp_backward_layer)."""
+        adjoint kernels (fmc_rnvp_backward)."""
         if isinstance(x, torch.Tensor) and x.requires_grad and torch.is_grad_enabled():
             return _RnvpLogProb.apply(x, self)
         return self._log_prob_value(x)

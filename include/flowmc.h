@@ -383,14 +383,24 @@ int fmc_rnvp_pass(void* stream, const fmc_rnvp* flow, int32_t dir, int32_t flags
 /* log_prob: replaces eqx.filter_value_and_grad in NFModel.train_step       */
 /* (nf_model/base.py:98-125) for RealNVP. gy [n, d] = dL/d(layer output)    */
 /* -> gx [n, d] (no aliasing); partials [rows, partial_per_tile] receive    */
-/* the per-tile weight gradients (rows 0 .. tiles-1), summed in a fixed     */
-/* order by fmc_rnvp_weight_grad, which uses up to 16 more rows             */
-/* (partial_rows >= tiles + min(16, ceil(tiles / 16))).                     */
+/* the weight gradients by tile, summed in a fixed order by                 */
+/* fmc_rnvp_weight_grad (n_tiles = ceil(n / tile); partial_rows >= n_tiles).*/
 int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* flow, int32_t layer, const float* x_in,
                             int64_t n, const float* g_logp, const float* gy, float* gx,
                             float* partials, int64_t n_partial_tiles);
 int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* flow, int32_t layer, float* partials,
                          int64_t n_tiles, int64_t partial_rows, float* grad);
+/* The whole backward sweep in two launches: the adjoint of every layer and */
+/* tile, then the weight gradients of all layers (every parameter entry of  */
+/* grad that can be non-zero is written; masked weights and the statistics  */
+/* are left alone: clear grad once). saved [L, n, d] and gy as              */
+/* fmc_rnvp_pass wrote them; gx [n, d] = dL/d(standardised input) (no       */
+/* aliasing); workspace of fmc_rnvp_backward_ws_size floats, 16-byte        */
+/* aligned.                                                                 */
+int fmc_rnvp_backward_ws_size(const fmc_rnvp* flow, int64_t n, int64_t* floats);
+int fmc_rnvp_backward(void* stream, const fmc_rnvp* flow, const float* saved, int64_t n,
+                      const float* g_logp, const float* gy, float* gx, float* grad,
+                      float* workspace, int64_t workspace_floats);
 
 /* ------------------------------------------------------------------------ */
 /* MaskedCouplingRQSpline flow                                              */
