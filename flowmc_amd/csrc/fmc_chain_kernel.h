@@ -5,6 +5,8 @@
 // condition matrix).
 #pragma once
 
+#include <type_traits>
+
 #include "fmc_chain_steps.h"
 
 namespace fmc {
@@ -15,31 +17,81 @@ namespace fmc {
 // allocation (and lower its occupancy).
 enum KernelKind { KK_MALA = 0, KK_HMC = 1, KK_GRW = 2, KK_HMC_DENSE = 3 };
 
-// One kernel per (lane layout NV, step kind, target kind TK): the target's
-// value and gradient are inlined without a run-time dispatch. HMC keeps
-// position, momentum, gradient, metric and the leapfrog copies in registers:
-// its workgroups are bounded at 512 threads, which gives it 256 VGPRs
-// instead of the 128 of a 1024-thread bound (spills at NV >= 2).
-template <int NV, int KIND, int TK>
-__global__ void __launch_bounds__((KIND == KK_HMC || KIND == KK_HMC_DENSE) ? 512 : 1024) chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg,
-                                                     int lpc, int n_lds) {
-  extern __shared__ float smem[];
-  TargetDev t = stage_target(tg, smem, n_lds);
+// Bound by instruction issue: the state stays in registers, and rows leave at
+// 5.2 TB/s at most. What a step costs is its VALU instructions (a MALA step of
+// the 128-D Rosenbrock 350, of the 8-mode 64-D mixture 469) and, with few
+// chains, the wait of a lone wavefront between them. us, the same calls with
+// one kernel for all targets, parameters read from memory and runtime lane
+// counts -> now: 1000 MALA steps of 1000 5-D dense-Gaussian chains 3133 -> 712;
+// 64 of 16384 128-D Rosenbrock chains 237 -> 164; 100 tempered steps of 20480
+// 64-D mixture rows 660 -> 370; 128 HMC steps of 2301 27-D Rosenbrock chains
+// 9.6 -> 4.5 a step.
+//
+// One kernel per (lane layout NV, step kind, target kind TK, lanes per chain
+// LPC): the target's value and gradient are inlined without a run-time
+// dispatch, and with LPC > 0 (the default layouts, workgroups of at most 256
+// threads) the group sums and broadcasts are straight-line DPP code and
+// parameters are always staged. LPC = 0 takes the lane count at run time, any
+// workgroup up to 1024 threads (HMC keeps position, momentum, gradient, metric
+// and the leapfrog copies in registers: bounded at 512 threads, which gives it
+// 256 VGPRs instead of 128, where NV >= 2 spilled) and parameters too large
+// for LDS.
+//
+// RING: wavefront 0 advances the workgroup's 64 / lpc chains and the others
+// draw its random numbers, a block of steps ahead, into LDS (use_ring has
+// the rule).
+template <int NV, int KIND, int TK, int LPC, bool RING>
+__global__ void __launch_bounds__(LPC ? 256 : (KIND == KK_HMC || KIND == KK_HMC_DENSE) ? 512 : 1024)
+chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg, int lpc_rt, int dp, NoiseRing nr) {
+  constexpr bool PARAMS = TK != FMC_TARGET_ROSENBROCK && TK != FMC_TARGET_FUNNEL;
+  const int lpc = LPC ? LPC : lpc_rt;
+  const TargetDev t{tg.kind, tg.n_dim, tg.n_modes, (gparam_t)tg.params, dp};
+  if (PARAMS && dp > 0) stage_target<TK>(t);
   const int lane = threadIdx.x & 63;
   const int r = lane & (lpc - 1);
   const int gbase = lane - r;
-  const int64_t c = (int64_t)blockIdx.x * (blockDim.x / lpc) + threadIdx.x / lpc;
+  int64_t c = (int64_t)blockIdx.x * (blockDim.x / lpc) + threadIdx.x / lpc;
+  if constexpr (RING) {
+    const int64_t c0 = (int64_t)blockIdx.x * (64 / lpc);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nblk = (nr.n_steps + ring_T<NV> - 1) / ring_T<NV>;
+    constexpr uint32_t SN = KIND == KK_MALA ? RNG_MALA_NOISE : RNG_GRW_NOISE;
+    constexpr uint32_t SU = KIND == KK_MALA ? RNG_MALA_UNIFORM : RNG_GRW_UNIFORM;
+    if (wave > 0) {
+      for (int b = 0; b < nblk; ++b) {
+        fill_ring<NV>(io, nr, cfg, t.d, lpc, c0, b, wave - 1, (int)(blockDim.x >> 6) - 1, SN, SU);
+        __syncthreads();  // block b full, block b - 1 consumed
+      }
+      return;
+    }
+    __syncthreads();
+    c = c0 + lane / lpc;
+  }
   if (c >= io.C) return;  // whole group leaves together
-  if (KIND == KK_MALA)
-    mala_group<NV, TK>(t, io, cfg, c, r, lpc, gbase);
-  else if (KIND == KK_GRW)
-    grw_group<NV, TK>(t, io, cfg, c, r, lpc, gbase);
-  else if (KIND == KK_HMC_DENSE)
-    hmc_group<NV, MK_DENSE, TK>(t, io, cfg, c, r, lpc, gbase);
-  else if (io.metric)
-    hmc_group<NV, MK_DIAG, TK>(t, io, cfg, c, r, lpc, gbase);
-  else
-    hmc_group<NV, MK_UNIT, TK>(t, io, cfg, c, r, lpc, gbase);
+  auto run = [&](auto staged) {
+    constexpr bool LDSP = decltype(staged)::value;
+    using RG = std::conditional_t<TK == FMC_TARGET_GAUSS_DENSE && LPC == 1 && NV <= 2, DenseRegs<NV>, NoRegs>;
+    if constexpr (KIND == KK_MALA)
+      mala_group<NV, TK, LDSP, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+    else if constexpr (KIND == KK_GRW)
+      grw_group<NV, TK, LDSP, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+    else if constexpr (KIND == KK_HMC_DENSE)
+      hmc_group<NV, MK_DENSE, TK, LDSP, NoRegs>(t, io, cfg, c, r, lpc, gbase);
+    else if (io.metric)
+      hmc_group<NV, MK_DIAG, TK, LDSP, RG>(t, io, cfg, c, r, lpc, gbase);
+    else
+      hmc_group<NV, MK_UNIT, TK, LDSP, RG>(t, io, cfg, c, r, lpc, gbase);
+  };
+  if constexpr (!PARAMS) {
+    run(std::false_type{});
+  } else if constexpr (LPC > 0) {
+    run(std::true_type{});
+  } else {
+    if (dp > 0)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+  }
 }
 
 // ----------------------------------------------------------- host side ----
@@ -103,19 +155,108 @@ static inline int check_layout(const Layout& L, int d) {
   return FMC_OK;
 }
 
-static inline int lds_floats(const fmc_target* t) {
-  int64_t n = target_param_count(t->kind, t->n_dim, t->n_modes);
-  return (n > 0 && n * 4 <= 48 * 1024) ? (int)n : 0;
+// Row stride of the staged parameters for a layout (0: not staged).
+static inline int staged_stride(const fmc_target* t, const Layout& L) {
+  const int dp = 4 * L.nv * L.lpc;
+  const int64_t n = target_staged_count(t->kind, t->n_dim, t->n_modes, dp);
+  return (n > 0 && n * 4 <= 48 * 1024) ? dp : 0;
+}
+static inline int staged_floats(const fmc_target* t, int dp) {
+  return dp ? (int)((target_staged_count(t->kind, t->n_dim, t->n_modes, dp) + 3) & ~3LL) : 0;
 }
 
+// Whether a workgroup is one chain wavefront and three that draw its random
+// numbers, or four that draw their own. A lone wavefront on a SIMD issues an instruction every
+// ~6.5 clocks (4 with company), and the Philox draws are half of a small
+// target's step: while the chains fill at most one wavefront a SIMD (1024), the
+// idle issue slots take them over. us a step, without / with the ring: MALA
+// dense Gaussian d = 5, C = 1000 (16 wavefronts) 1.29 / 0.76, d = 12, C = 1000
+// 3.16 / 2.32; funnel d = 7, C = 1343 0.90 / 0.54; Rosenbrock d = 128, C = 500
+// (125) 1.22 / 0.81, C = 4096 (1024) 1.32 / 1.15; mixture d = 64, C = 500 2.07 /
+// 1.85. Above, the SIMDs are full and the ring only adds LDS traffic: funnel
+// d = 100, C = 4000 (2000) 1.01 / 1.24, Rosenbrock d = 128, C = 16384 (4096)
+// 2.80 / 4.18. More than three filling wavefronts give nothing (0.93 -> 0.92).
+// The launch stays within the 64 KB of LDS that need no attribute: a mixture's
+// staged parameters can leave no room for the ring.
+constexpr int RING_MAX_WAVES = 1024;
+constexpr size_t RING_MAX_LDS = 64 * 1024;
+
+template <int NV>
+static size_t ring_bytes(int lpc) { return 4 * 2 * (size_t)ring_T<NV> * (NV * 256 + 64 / lpc); }
+
+template <int NV>
+static bool use_ring(const ChainIO& io, const StepCfg& cfg, const Layout& L, int staged) {
+  return !io.noise && !io.log_u && L.block == 256 && cfg.n_steps >= 8 &&
+         (io.C * L.lpc + 63) / 64 <= RING_MAX_WAVES && 4 * (size_t)staged + ring_bytes<NV>(L.lpc) <= RING_MAX_LDS;
+}
+
+template <int NV, int KIND, int TK, int LPC>
+static void launch_chain_lpc(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
+                             const Layout& L, int dp) {
+  const int nf = staged_floats(t, dp);
+  const NoiseRing nr{nf, cfg.n_steps};
+  if constexpr (LPC > 0 && (KIND == KK_MALA || KIND == KK_GRW)) {
+    if (use_ring<NV>(io, cfg, L, nf)) {
+      const int per_block = 64 / LPC;
+      hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, true>), dim3((unsigned)((io.C + per_block - 1) / per_block)),
+                         dim3(256), 4 * (size_t)nf + ring_bytes<NV>(LPC), st, *t, io, cfg, L.lpc, dp, nr);
+      return;
+    }
+  }
+  const int per_block = L.block / L.lpc;
+  hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, false>), dim3((unsigned)((io.C + per_block - 1) / per_block)),
+                     dim3((unsigned)L.block), 4 * (size_t)nf, st, *t, io, cfg, L.lpc, dp, nr);
+}
+
+// The kernels specialised on their lane count: the layouts choose_layout gives
+// to up to 256 dims (512 for Rosenbrock, 32 for a dense Gaussian).
 template <int KIND, int TK>
-static void launch_chain_nv(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
-                            const Layout& L, dim3 g, dim3 b, size_t shm, int n_lds) {
+static void launch_chain_kind(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
+                              const Layout& L) {
+  const int dp = staged_stride(t, L);
+  if constexpr (KIND != KK_HMC_DENSE) {
+    const bool staged = dp > 0 || TK == FMC_TARGET_ROSENBROCK || TK == FMC_TARGET_FUNNEL;
+    if (staged && L.block <= 256) {
+#define FMC_LPC(NV_, LPC_)                                                      \
+  case LPC_:                                                                    \
+    launch_chain_lpc<NV_, KIND, TK, LPC_>(st, t, io, cfg, L, dp);               \
+    return;
+      constexpr int NVD = TK == FMC_TARGET_ROSENBROCK ? 2 : 1;  // chunks a lane holds by default
+      if constexpr (TK == FMC_TARGET_GAUSS_DENSE) {
+        if (L.lpc == 1) {
+          switch (L.nv) {
+            case 1: launch_chain_lpc<1, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
+            case 2: launch_chain_lpc<2, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
+            case 4: launch_chain_lpc<4, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
+            default: break;
+          }
+        }
+      } else {
+        if (TK == FMC_TARGET_ROSENBROCK && L.nv == 1 && L.lpc == 1) {
+          launch_chain_lpc<1, KIND, TK, 1>(st, t, io, cfg, L, dp);
+          return;
+        }
+        if (L.nv == NVD) {
+          switch (L.lpc) {
+            FMC_LPC(NVD, 1)
+            FMC_LPC(NVD, 2)
+            FMC_LPC(NVD, 4)
+            FMC_LPC(NVD, 8)
+            FMC_LPC(NVD, 16)
+            FMC_LPC(NVD, 32)
+            FMC_LPC(NVD, 64)
+            default: break;
+          }
+        }
+      }
+#undef FMC_LPC
+    }
+  }
   switch (L.nv) {
-    case 1: hipLaunchKernelGGL((chain_kernel<1, KIND, TK>), g, b, shm, st, *t, io, cfg, L.lpc, n_lds); break;
-    case 2: hipLaunchKernelGGL((chain_kernel<2, KIND, TK>), g, b, shm, st, *t, io, cfg, L.lpc, n_lds); break;
-    case 4: hipLaunchKernelGGL((chain_kernel<4, KIND, TK>), g, b, shm, st, *t, io, cfg, L.lpc, n_lds); break;
-    default: hipLaunchKernelGGL((chain_kernel<8, KIND, TK>), g, b, shm, st, *t, io, cfg, L.lpc, n_lds); break;
+    case 1: launch_chain_lpc<1, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
+    case 2: launch_chain_lpc<2, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
+    case 4: launch_chain_lpc<4, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
+    default: launch_chain_lpc<8, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
   }
 }
 
@@ -124,33 +265,23 @@ static int launch_chain_impl(hipStream_t st, const fmc_target* t, const ChainIO&
                              const Layout& L) {
   FMC_ARG((KIND != KK_HMC && KIND != KK_HMC_DENSE) || L.block <= 512,
           "fused HMC launches take at most 512 threads per workgroup (got %d)", L.block);
-  const int per_block = L.block / L.lpc;
-  const int64_t grid = (io.C + per_block - 1) / per_block;
-  FMC_ARG(grid <= 0x7fffffffLL, "too many chains for one launch");
-  const int n_lds = lds_floats(t);
-  const size_t shm = (size_t)n_lds * sizeof(float);
-  dim3 g((unsigned)grid), b((unsigned)L.block);
+  FMC_ARG((io.C * L.lpc + 63) / 64 <= 0x7fffffffLL, "too many chains for one launch");
   switch (t->kind) {  // check_target has accepted the kind
-    case FMC_TARGET_GAUSS_DIAG: launch_chain_nv<KIND, FMC_TARGET_GAUSS_DIAG>(st, t, io, cfg, L, g, b, shm, n_lds); break;
-    case FMC_TARGET_GAUSS_DENSE: launch_chain_nv<KIND, FMC_TARGET_GAUSS_DENSE>(st, t, io, cfg, L, g, b, shm, n_lds); break;
-    case FMC_TARGET_ROSENBROCK: launch_chain_nv<KIND, FMC_TARGET_ROSENBROCK>(st, t, io, cfg, L, g, b, shm, n_lds); break;
-    case FMC_TARGET_FUNNEL: launch_chain_nv<KIND, FMC_TARGET_FUNNEL>(st, t, io, cfg, L, g, b, shm, n_lds); break;
-    case FMC_TARGET_GMM_DIAG: launch_chain_nv<KIND, FMC_TARGET_GMM_DIAG>(st, t, io, cfg, L, g, b, shm, n_lds); break;
-    default: launch_chain_nv<KIND, FMC_TARGET_DUAL_MOON>(st, t, io, cfg, L, g, b, shm, n_lds); break;
+    case FMC_TARGET_GAUSS_DIAG: launch_chain_kind<KIND, FMC_TARGET_GAUSS_DIAG>(st, t, io, cfg, L); break;
+    case FMC_TARGET_GAUSS_DENSE: launch_chain_kind<KIND, FMC_TARGET_GAUSS_DENSE>(st, t, io, cfg, L); break;
+    case FMC_TARGET_ROSENBROCK: launch_chain_kind<KIND, FMC_TARGET_ROSENBROCK>(st, t, io, cfg, L); break;
+    case FMC_TARGET_FUNNEL: launch_chain_kind<KIND, FMC_TARGET_FUNNEL>(st, t, io, cfg, L); break;
+    case FMC_TARGET_GMM_DIAG: launch_chain_kind<KIND, FMC_TARGET_GMM_DIAG>(st, t, io, cfg, L); break;
+    default: launch_chain_kind<KIND, FMC_TARGET_DUAL_MOON>(st, t, io, cfg, L); break;
   }
   return check_launch(KIND == KK_MALA ? "mala chain kernel" : KIND == KK_GRW ? "grw chain kernel" : "hmc chain kernel");
 }
 
+// One translation unit per step kind (they build in parallel).
+int launch_mala(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg, const Layout& L);
+int launch_grw(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg, const Layout& L);
+int launch_hmc(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg, const Layout& L);
 // Fused HMC with a dense condition matrix (defined in fmc_hmc_dense.hip).
 int launch_hmc_dense(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg, const Layout& L);
-
-template <int KIND>
-static int launch_chain(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
-                        const Layout& L) {
-  if constexpr (KIND == KK_HMC) {
-    if (io.chol) return launch_hmc_dense(st, t, io, cfg, L);
-  }
-  return launch_chain_impl<KIND>(st, t, io, cfg, L);
-}
 
 }  // namespace fmc

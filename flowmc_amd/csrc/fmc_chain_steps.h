@@ -56,28 +56,52 @@ __device__ __forceinline__ void load_row(const float* __restrict__ src, int d, i
   }
 }
 
+// A float4 at any 4-byte aligned address (global accesses need no more)
+struct __attribute__((packed, aligned(4))) float4_a4 {
+  float x, y, z, w;
+};
+
 template <int NV>
 __device__ __forceinline__ void store_row(float* __restrict__ dst, int d, int r, int lpc,
                                           const float4 (&x)[NV]) {
-  const bool vec = (d & 3) == 0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    int j0 = (v * lpc + r) * 4;
-    if (vec) {
-      if (j0 < d) *reinterpret_cast<float4*>(dst + j0) = x[v];
-    } else {
+    const int j0 = (v * lpc + r) * 4;
+    if (j0 + 3 < d) {
+      *reinterpret_cast<float4_a4*>(dst + j0) = float4_a4{x[v].x, x[v].y, x[v].z, x[v].w};
+    } else if (j0 < d) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < 3; ++e)
         if (j0 + e < d) dst[j0 + e] = f4c(x[v], e);
     }
   }
 }
 
-// Standard normals of (chain, step) for this lane's chunks; padding zeroed.
+// Where a step's random numbers come from: memory (injected), the Philox
+// stream, or LDS blocks that other wavefronts of the workgroup fill from the
+// same stream (NoiseRing).
+struct NoiseRing {
+  int base;     // float offset of the ring in LDS: [2][T][NV][64] float4, then [2][T][64 / lpc] log u
+  int n_steps;
+};
+
+// Steps a ring block holds
 template <int NV>
-__device__ __forceinline__ void draw_normals(const ChainIO& io, int d, int r, int lpc, int64_t c,
+constexpr int ring_T = NV == 1 ? 16 : NV == 2 ? 8 : 4;
+
+template <int NV>
+__device__ __forceinline__ int ring_lu(const NoiseRing& nr) { return nr.base + 2 * ring_T<NV> * NV * 256; }
+
+// Standard normals of (chain, step) for this lane's chunks; padding zeroed.
+template <int NV, bool RING>
+__device__ __forceinline__ void draw_normals(const ChainIO& io, const NoiseRing& nr, int d, int r, int lpc, int64_t c,
                                              int s, int t_glob, uint32_t sid, float4 (&xi)[NV]) {
-  if (io.noise) {
+  if (RING) {
+    const int slot = s & (2 * ring_T<NV> - 1);
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      xi[v] = *reinterpret_cast<const float4*>(fmc_chain_lds + nr.base + ((slot * NV + v) * 64 + (threadIdx.x & 63)) * 4);
+  } else if (io.noise) {
     load_row<NV>(io.noise + ((int64_t)s * io.C + c) * d, d, r, lpc, xi);
   } else {
 #pragma unroll
@@ -91,24 +115,90 @@ __device__ __forceinline__ void draw_normals(const ChainIO& io, int d, int r, in
   }
 }
 
-__device__ __forceinline__ float draw_log_u(const ChainIO& io, int64_t c, int s, int t_glob,
-                                            uint32_t sid) {
+// log u of (chain, step). A group's lanes would all compute the same Philox
+// block: each computes another step's instead, once every lpc steps (keep),
+// and hands it over in its turn.
+template <int NV, bool RING>
+__device__ __forceinline__ float draw_log_u(const ChainIO& io, const NoiseRing& nr, int r, int lpc, int gbase, int64_t c,
+                                            int s, int t_glob, uint32_t sid, float& keep) {
+  if (RING) return fmc_chain_lds[ring_lu<NV>(nr) + (s & (2 * ring_T<NV> - 1)) * (64 / lpc) + (threadIdx.x & 63) / lpc];
   if (io.log_u) return io.log_u[(int64_t)s * io.C + c];
-  return philox_log_uniform(io.key0, io.key1, (uint32_t)c, (uint32_t)t_glob, sid);
+  const int k = s & (lpc - 1);
+  if (k == 0) keep = philox_log_uniform(io.key0, io.key1, (uint32_t)c, (uint32_t)(t_glob + r), sid);
+  return lpc == 1 ? keep : __shfl(keep, gbase + k, 64);
 }
 
+// Fills ring block `blk` (steps blk T .. ) for the chain wavefront of this
+// workgroup: wavefront w of nw takes every nw-th (step, chunk) item, a log u
+// item being 64 (step, chain) pairs. c0: the workgroup's first chain.
 template <int NV>
-__device__ __forceinline__ void write_rows(const ChainIO& io, int d, int r, int lpc, int64_t c,
-                                           int t_glob, int thinning, const float4 (&x)[NV], float lp,
-                                           bool acc) {
-  if (t_glob % thinning != 0) return;
-  int64_t row = io.cursor + t_glob / thinning;
-  if (io.out_pos) store_row<NV>(io.out_pos + (c * io.buf_len + row) * d, d, r, lpc, x);
-  if (r == 0) {
-    if (io.out_logp) io.out_logp[c * io.buf_len + row] = lp;
-    if (io.out_acc) io.out_acc[c * io.buf_len + row] = acc ? 1.f : 0.f;
+__device__ __forceinline__ void fill_ring(const ChainIO& io, const NoiseRing& nr, const StepCfg& cfg, int d, int lpc,
+                                          int64_t c0, int blk, int w, int nw, uint32_t sid, uint32_t sid_u) {
+  constexpr int T = ring_T<NV>;
+  const int lane = threadIdx.x & 63, r = lane & (lpc - 1), cpw = 64 / lpc;
+  const int s0 = blk * T, half = (blk & 1) * T;
+  const int ns = nr.n_steps - s0 < T ? nr.n_steps - s0 : T;  // steps of the block
+  const int n_norm = ns * NV, n_u = (ns * cpw + 63) / 64;
+  const uint32_t c = (uint32_t)(c0 + lane / lpc);
+  for (int i = w; i < n_norm + n_u; i += nw) {
+    if (i < n_norm) {
+      const int st = i / NV, v = i - st * NV, chunk = v * lpc + r;
+      float4 z = philox_normal4(io.key0, io.key1, (uint32_t)chunk, c, (uint32_t)(cfg.step0 + s0 + st), sid);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (chunk * 4 + e >= d) f4(z, e) = 0.f;
+      *reinterpret_cast<float4*>(fmc_chain_lds + nr.base + (((half + st) * NV + v) * 64 + lane) * 4) = z;
+    } else {
+      const int k = (i - n_norm) * 64 + lane, st = k / cpw, cl = k - st * cpw;
+      if (st < ns)
+        fmc_chain_lds[ring_lu<NV>(nr) + (half + st) * cpw + cl] =
+            philox_log_uniform(io.key0, io.key1, (uint32_t)(c0 + cl), (uint32_t)(cfg.step0 + s0 + st), sid_u);
+    }
   }
 }
+// A ring block ends: its filler and its reader change places.
+template <int NV, bool RING>
+__device__ __forceinline__ void ring_step(const NoiseRing& nr, int s) {
+  if (RING && ((s + 1) & (ring_T<NV> - 1)) == 0 && s + 1 < nr.n_steps) __syncthreads();
+}
+
+// The thinned buffer rows of one chain: global step t with t % thinning == 0
+// lands on row cursor + t / thinning (pointers and the next such step carried
+// along: no division or product a step).
+struct RowWriter {
+  float *pos = nullptr, *lp = nullptr, *acc = nullptr;
+  int next, thinning;
+  bool has_pos, has_lp, has_acc;  // the same for every lane: tested without the lanes' pointers
+  __device__ __forceinline__ RowWriter(const ChainIO& io, const StepCfg& cfg, int d, int64_t c) {
+    thinning = cfg.thinning;
+    const int k = (cfg.step0 + thinning - 1) / thinning;
+    next = k * thinning;
+    const int64_t row = c * io.buf_len + io.cursor + k;
+    has_pos = io.out_pos != nullptr;
+    has_lp = io.out_logp != nullptr;
+    has_acc = io.out_acc != nullptr;
+    if (has_pos) pos = io.out_pos + row * d;
+    if (has_lp) lp = io.out_logp + row;
+    if (has_acc) acc = io.out_acc + row;
+  }
+  template <int NV>
+  __device__ __forceinline__ void write(int t_glob, int d, int r, int lpc, const float4 (&x)[NV], float lpv, bool a) {
+    if (t_glob != next) return;
+    next += thinning;
+    if (has_pos) {
+      store_row<NV>(pos, d, r, lpc, x);
+      pos += d;
+    }
+    if (has_lp) {
+      if (r == 0) *lp = lpv;
+      ++lp;
+    }
+    if (has_acc) {
+      if (r == 0) *acc = a ? 1.f : 0.f;
+      ++acc;
+    }
+  }
+};
 
 // Tempered rows (parallel tempering): row c of a tempered launch targets
 // log p(x) / T with T = temps[c % n_temps] — TemperedPDF.tempered_log_pdf
@@ -133,43 +223,46 @@ __device__ __forceinline__ float temper(const ChainIO& io, float beta, float lp,
 // MALA.py:26-89). The gradient at the current point is carried from the
 // previous step instead of being re-evaluated: MALA.py:59 recomputes it at the
 // same point, which for a deterministic target is the same value.
-template <int NV, int TK>
-__device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg, int64_t c,
-                           int r, int lpc, int gbase) {
+template <int NV, int TK, bool LDSP, bool RING, class RG>
+__device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg,
+                                           const NoiseRing& nr, int64_t c, int r, int lpc, int gbase) {
   const int d = t.d;
+  const RG rg(t);
   float4 x[NV], g[NV];
   load_row<NV>(io.x + c * d, d, r, lpc, x);
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK>(t, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, true>(t, rg, x, g, r, lpc, gbase), g);
   const float dt = cfg.dt;
   const float h = 0.5f * dt * dt;
   const float inv2dt2 = 1.f / (2.f * dt * dt);
+  RowWriter rows(io, cfg, d, c);
+  float lu_keep = 0.f;
   for (int s = 0; s < cfg.n_steps; ++s) {
     const int tg = cfg.step0 + s;
     float4 xi[NV], prop[NV], g1[NV];
-    draw_normals<NV>(io, d, r, lpc, c, s, tg, RNG_MALA_NOISE, xi);
+    draw_normals<NV, RING>(io, nr, d, r, lpc, c, s, tg, RNG_MALA_NOISE, xi);
+    const float lu = draw_log_u<NV, RING>(io, nr, r, lpc, gbase, c, s, tg, RNG_MALA_UNIFORM, lu_keep);
     float s1 = 0.f;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float n = dt * f4c(xi[v], e);
-        f4(prop[v], e) = f4c(x[v], e) + h * f4c(g[v], e) + n;
-        s1 += n * n;
+        f4(prop[v], e) = fmaf(dt, f4c(xi[v], e), fmaf(h, f4c(g[v], e), f4c(x[v], e)));
+        s1 = fmaf(n, n, s1);
       }
-    float lp1 = temper<NV>(io, beta, target_vg<NV, TK>(t, prop, g1, r, lpc, gbase), g1);
+    float lp1 = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, prop, g1, r, lpc, gbase), g1);
     float s2 = 0.f;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float q = f4c(x[v], e) - f4c(prop[v], e) - h * f4c(g1[v], e);
-        s2 += q * q;
+        const float q = fmaf(-h, f4c(g1[v], e), f4c(x[v], e) - f4c(prop[v], e));
+        s2 = fmaf(q, q, s2);
       }
     // padding lanes contribute exactly 0 to s1 and s2
     float ds = group_sum(s1 - s2, lpc);
-    float ratio = (lp1 - lp) + ds * inv2dt2;
-    float lu = draw_log_u(io, c, s, tg, RNG_MALA_UNIFORM);
+    const float ratio = fmaf(ds, inv2dt2, lp1 - lp);
     bool acc = lu < ratio;
     if (acc) {
 #pragma unroll
@@ -179,7 +272,8 @@ __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io
       }
       lp = lp1;
     }
-    write_rows<NV>(io, d, r, lpc, c, tg, cfg.thinning, x, lp, acc);
+    rows.write<NV>(tg, d, r, lpc, x, lp, acc);
+    ring_step<NV, RING>(nr, s);
   }
   store_row<NV>(io.x + c * d, d, r, lpc, x);
   if (r == 0 && io.logp) io.logp[c] = lp;
@@ -191,32 +285,36 @@ __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io
 // log u < logp(x') - logp(x). The log-density of the entry state is evaluated
 // once (take_steps.py:177) and carried; the target's gradient output is dead
 // and removed by the compiler.
-template <int NV, int TK>
-__device__ __forceinline__ void grw_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg, int64_t c,
-                          int r, int lpc, int gbase) {
+template <int NV, int TK, bool LDSP, bool RING, class RG>
+__device__ __forceinline__ void grw_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg,
+                                          const NoiseRing& nr, int64_t c, int r, int lpc, int gbase) {
   const int d = t.d;
+  const RG rg(t);
   float4 x[NV], g[NV];
   load_row<NV>(io.x + c * d, d, r, lpc, x);
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK>(t, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, true>(t, rg, x, g, r, lpc, gbase), g);
   const float dt = cfg.dt;
+  RowWriter rows(io, cfg, d, c);
+  float lu_keep = 0.f;
   for (int s = 0; s < cfg.n_steps; ++s) {
     const int tg = cfg.step0 + s;
     float4 xi[NV], prop[NV];
-    draw_normals<NV>(io, d, r, lpc, c, s, tg, RNG_GRW_NOISE, xi);
+    draw_normals<NV, RING>(io, nr, d, r, lpc, c, s, tg, RNG_GRW_NOISE, xi);
+    const float lu = draw_log_u<NV, RING>(io, nr, r, lpc, gbase, c, s, tg, RNG_GRW_UNIFORM, lu_keep);
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) f4(prop[v], e) = f4c(x[v], e) + dt * f4c(xi[v], e);
-    const float lp1 = temper<NV>(io, beta, target_vg<NV, TK>(t, prop, g, r, lpc, gbase), g);
-    const float lu = draw_log_u(io, c, s, tg, RNG_GRW_UNIFORM);
+      for (int e = 0; e < 4; ++e) f4(prop[v], e) = fmaf(dt, f4c(xi[v], e), f4c(x[v], e));
+    const float lp1 = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, prop, g, r, lpc, gbase), g);
     const bool acc = lu < lp1 - lp;
     if (acc) {
 #pragma unroll
       for (int v = 0; v < NV; ++v) x[v] = prop[v];
       lp = lp1;
     }
-    write_rows<NV>(io, d, r, lpc, c, tg, cfg.thinning, x, lp, acc);
+    rows.write<NV>(tg, d, r, lpc, x, lp, acc);
+    ring_step<NV, RING>(nr, s);
   }
   store_row<NV>(io.x + c * d, d, r, lpc, x);
   if (r == 0 && io.logp) io.logp[c] = lp;
@@ -273,11 +371,12 @@ __device__ __forceinline__ void dense_momentum(const float* __restrict__ Lc, int
   }
 }
 
-template <int NV, int MK, int TK>
+template <int NV, int MK, int TK, bool LDSP = false, class RG = NoRegs>
 __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg, int64_t c,
                           int r, int lpc, int gbase) {
   constexpr bool UNIT_M = MK == MK_UNIT;
   const int d = t.d;
+  const RG rg(t);
   float4 x[NV], g[NV], m[NV];
   load_row<NV>(io.x + c * d, d, r, lpc, x);
   if (!UNIT_M) {
@@ -287,13 +386,16 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
     for (int v = 0; v < NV; ++v) m[v] = make_float4(1.f, 1.f, 1.f, 1.f);
   }
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK>(t, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, x, g, r, lpc, gbase), g);
   const float eps = cfg.dt;
   const int L = cfg.n_leapfrog;
+  RowWriter rows(io, cfg, d, c);
+  float lu_keep = 0.f;
   for (int s = 0; s < cfg.n_steps; ++s) {
     const int tg = cfg.step0 + s;
     float4 p[NV], xl[NV], gl[NV];
-    draw_normals<NV>(io, d, r, lpc, c, s, tg, RNG_HMC_MOMENTUM, p);
+    draw_normals<NV, false>(io, NoiseRing{0, 0}, d, r, lpc, c, s, tg, RNG_HMC_MOMENTUM, p);
+    const float lu = draw_log_u<NV, false>(io, NoiseRing{0, 0}, r, lpc, gbase, c, s, tg, RNG_HMC_UNIFORM, lu_keep);
     if (MK == MK_DENSE) {
       float4 xi[NV];
 #pragma unroll
@@ -329,19 +431,19 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) f4(p[v], e) += eps * 0.5f * f4c(gl[v], e);
+      for (int e = 0; e < 4; ++e) f4(p[v], e) = fmaf(eps * 0.5f, f4c(gl[v], e), f4c(p[v], e));
     float lpl = lp;
     for (int i = 1; i <= L + 1; ++i) {
       const float kick = (i <= L) ? 1.f : 0.5f;
 #pragma unroll
       for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f4(xl[v], e) += eps * (UNIT_M ? f4c(p[v], e) : f4c(m[v], e) * f4c(p[v], e));
-      lpl = temper<NV>(io, beta, target_vg<NV, TK>(t, xl, gl, r, lpc, gbase), gl);
+        for (int e = 0; e < 4; ++e) f4(xl[v], e) = fmaf(eps, UNIT_M ? f4c(p[v], e) : f4c(m[v], e) * f4c(p[v], e), f4c(xl[v], e));
+      lpl = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, xl, gl, r, lpc, gbase), gl);
 #pragma unroll
       for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f4(p[v], e) += eps * kick * f4c(gl[v], e);
+        for (int e = 0; e < 4; ++e) f4(p[v], e) = fmaf(eps * kick, f4c(gl[v], e), f4c(p[v], e));
     }
     double k1 = 0.0;
 #pragma unroll
@@ -361,7 +463,6 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
     double h0 = -(double)lp + k0;
     double h1 = -(double)lpl + k1;
     double log_acc = h0 - h1;
-    float lu = draw_log_u(io, c, s, tg, RNG_HMC_UNIFORM);
     bool acc = (double)lu < log_acc;
     if (acc) {
 #pragma unroll
@@ -371,21 +472,10 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
       }
       lp = lpl;
     }
-    write_rows<NV>(io, d, r, lpc, c, tg, cfg.thinning, x, lp, acc);
+    rows.write<NV>(tg, d, r, lpc, x, lp, acc);
   }
   store_row<NV>(io.x + c * d, d, r, lpc, x);
   if (r == 0 && io.logp) io.logp[c] = lp;
-}
-
-// Copies the target parameter block to LDS when it fits (n_lds > 0).
-__device__ __forceinline__ TargetDev stage_target(const fmc_target& tg, float* smem, int n_lds) {
-  TargetDev t{tg.kind, tg.n_dim, tg.n_modes, tg.params};
-  if (n_lds > 0) {
-    for (int i = threadIdx.x; i < n_lds; i += blockDim.x) smem[i] = tg.params[i];
-    __syncthreads();
-    t.p = smem;
-  }
-  return t;
 }
 
 }  // namespace fmc

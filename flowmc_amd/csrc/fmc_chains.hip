@@ -12,12 +12,12 @@
 namespace fmc {
 
 // ------------------------------------------------------- target eval ------
-template <int NV>
-__global__ void __launch_bounds__(1024) target_eval_kernel(fmc_target tg, const float* __restrict__ x,
-                                                           int64_t n, float* logp, float* grad,
-                                                           int lpc, int n_lds) {
-  extern __shared__ float smem[];
-  TargetDev t = stage_target(tg, smem, n_lds);
+template <int NV, int TK>
+__global__ void __launch_bounds__(256) target_eval_kernel(fmc_target tg, const float* __restrict__ x,
+                                                          int64_t n, float* logp, float* grad,
+                                                          int lpc, int dp) {
+  const TargetDev t{tg.kind, tg.n_dim, tg.n_modes, (gparam_t)tg.params, dp};
+  if (dp > 0) stage_target<TK>(t);
   const int lane = threadIdx.x & 63;
   const int r = lane & (lpc - 1);
   const int gbase = lane - r;
@@ -26,9 +26,24 @@ __global__ void __launch_bounds__(1024) target_eval_kernel(fmc_target tg, const 
   const int d = t.d;
   float4 xv[NV], g[NV];
   load_row<NV>(x + c * d, d, r, lpc, xv);
-  float lp = target_vg<NV>(t, xv, g, r, lpc, gbase);
+  const float lp = dp > 0 ? target_vg<NV, TK, true, false>(t, NoRegs(t), xv, g, r, lpc, gbase)
+                          : target_vg<NV, TK, false, false>(t, NoRegs(t), xv, g, r, lpc, gbase);
   if (grad) store_row<NV>(grad + c * d, d, r, lpc, g);
   if (r == 0 && logp) logp[c] = lp;
+}
+
+template <int TK>
+static void launch_eval(hipStream_t st, const fmc_target& t, const float* x, int64_t n, float* logp, float* grad,
+                        const Layout& L) {
+  const int dp = staged_stride(&t, L), block = L.block < 256 ? L.block : 256, per = block / L.lpc;
+  const size_t shm = 4 * (size_t)staged_floats(&t, dp);
+  const dim3 g((unsigned)((n + per - 1) / per)), b((unsigned)block);
+  switch (L.nv) {
+    case 1: hipLaunchKernelGGL((target_eval_kernel<1, TK>), g, b, shm, st, t, x, n, logp, grad, L.lpc, dp); break;
+    case 2: hipLaunchKernelGGL((target_eval_kernel<2, TK>), g, b, shm, st, t, x, n, logp, grad, L.lpc, dp); break;
+    case 4: hipLaunchKernelGGL((target_eval_kernel<4, TK>), g, b, shm, st, t, x, n, logp, grad, L.lpc, dp); break;
+    default: hipLaunchKernelGGL((target_eval_kernel<8, TK>), g, b, shm, st, t, x, n, logp, grad, L.lpc, dp); break;
+  }
 }
 
 // ------------------------------------------- per-step pieces (any target) --
@@ -298,10 +313,15 @@ __global__ void __launch_bounds__(256) finite_rows_kernel(const float* __restric
 // is final, so the scan carries only the walker that may still move up (its
 // source slot and log-likelihood). Phase 1 (one thread per chain) writes the
 // slot -> source permutation to LDS and the log-likelihoods and decisions to
-// memory; phase 2 gathers the rows, one wave per row.
-constexpr int PT_CPB = 64;
+// memory; phase 2 gathers the rows. Bound by memory latency, not bytes (10 MB
+// at 1000 chains, 20 temperatures, d = 64): few chains a block fill the chip,
+// and every thread has rows of its own in flight (34 -> 7 us there; 64
+// chains a block with a wavefront per row left 16 blocks, one row at a time).
+constexpr int PT_CPB = 8;
 constexpr int PT_TMAX = 64;
+constexpr int PT_ADAPT = 1024;
 
+template <bool VEC>
 __global__ void __launch_bounds__(256) pt_exchange_kernel(const float* __restrict__ x_in, float* __restrict__ x_out,
                                                           float* loglik, const float* __restrict__ temps,
                                                           int64_t C, int T, int d, uint32_t k0, uint32_t k1,
@@ -309,7 +329,7 @@ __global__ void __launch_bounds__(256) pt_exchange_kernel(const float* __restric
                                                           float* __restrict__ acc) {
   __shared__ int src[PT_CPB * PT_TMAX];
   const int64_t c0 = (int64_t)blockIdx.x * PT_CPB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x;
   const int nc = (C - c0) < PT_CPB ? (int)(C - c0) : PT_CPB;
   if (tid < nc) {
     const int64_t c = c0 + tid;
@@ -338,12 +358,15 @@ __global__ void __launch_bounds__(256) pt_exchange_kernel(const float* __restric
     L[T - 1] = lc;
   }
   __syncthreads();
-  for (int row = wave; row < nc * T; row += 4) {
-    const int cl = row / T, t = row - cl * T;
-    const int64_t base = (c0 + cl) * T;
-    const float* s = x_in + (base + src[cl * PT_TMAX + t]) * d;
-    float* o = x_out + (base + t) * d;
-    for (int j = lane; j < d; j += 64) o[j] = s[j];
+  // the rows of the block's chains, spread over all threads (the copies are
+  // independent; a wavefront per row walked them one memory round trip each)
+  using V = std::conditional_t<VEC, float4, float>;
+  const int w = VEC ? d / 4 : d;
+  const V* in = reinterpret_cast<const V*>(x_in + c0 * T * d);
+  V* out = reinterpret_cast<V*>(x_out + c0 * T * d);
+  for (int e = tid; e < nc * T * w; e += 256) {
+    const int row = e / w, j = e - row * w, cl = row / T, t = row - cl * T;
+    out[e] = in[(cl * T + src[cl * PT_TMAX + t]) * w + j];
   }
 }
 
@@ -352,18 +375,32 @@ __global__ void __launch_bounds__(256) pt_exchange_kernel(const float* __restric
 // damping_p = (100 / C) (a_p - a_{p+1});
 // T'[i] = T'[i-1] + (T[i] - T[i-1]) exp(damping_{i-1}) for i = 1 .. T-2;
 // the first and last temperatures are unchanged.
-__global__ void __launch_bounds__(256) pt_adapt_kernel(float* temps, const float* __restrict__ acc, int64_t C,
-                                                       int T) {
+__global__ void __launch_bounds__(PT_ADAPT) pt_adapt_kernel(float* temps, const float* __restrict__ acc, int64_t C,
+                                                            int T) {
   __shared__ float rate[PT_TMAX];
-  __shared__ float part[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int p = 0; p + 1 < T; ++p) {
+  __shared__ float part[PT_ADAPT];
+  const int tid = threadIdx.x, P = T - 1;
+  if (P > 0) {
+    // all pairs at once: a thread keeps to one pair and walks the rows of
+    // chains, so that the block reads the table front to back
+    const int rows = PT_ADAPT / P, p = tid % P;
     float s = 0.f;  // sums of 0/1 values: exact below 2^24 per partial
-    for (int64_t c = tid; c < C; c += 256) s += acc[c * (T - 1) + p];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) part[wave] = s;
+    if (tid < rows * P)
+      for (int64_t e = tid; e < C * P; e += rows * P) s += acc[e];
+    part[tid] = s;
     __syncthreads();
-    if (tid == 0) rate[p] = ((part[0] + part[1]) + (part[2] + part[3])) / (float)C;
+    s = 0.f;
+    if (tid < 16 * P)
+      for (int q = tid / P; q < rows; q += 16) s += part[q * P + p];
+    __syncthreads();
+    part[tid] = s;
+    __syncthreads();
+    if (tid < P) {
+      float n = 0.f;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) n += part[q * P + tid];
+      rate[tid] = n / (float)C;
+    }
     __syncthreads();
   }
   if (tid == 0) {
@@ -427,17 +464,15 @@ extern "C" int fmc_target_eval(void* stream, const fmc_target* target, const flo
   if (n_points == 0) return FMC_OK;
   Layout L = choose_layout(target->n_dim, target->kind, cfg);
   if ((rc = check_layout(L, target->n_dim))) return rc;
-  const int per_block = L.block / L.lpc;
-  const int64_t grid = (n_points + per_block - 1) / per_block;
-  const int n_lds = lds_floats(target);
-  const size_t shm = (size_t)n_lds * sizeof(float);
+  FMC_ARG((n_points * L.lpc + 63) / 64 <= 0x7fffffffLL, "too many points for one launch");
   hipStream_t st = (hipStream_t)stream;
-  dim3 g((unsigned)grid), b((unsigned)L.block);
-  switch (L.nv) {
-    case 1: hipLaunchKernelGGL(target_eval_kernel<1>, g, b, shm, st, *target, x, n_points, logp, grad, L.lpc, n_lds); break;
-    case 2: hipLaunchKernelGGL(target_eval_kernel<2>, g, b, shm, st, *target, x, n_points, logp, grad, L.lpc, n_lds); break;
-    case 4: hipLaunchKernelGGL(target_eval_kernel<4>, g, b, shm, st, *target, x, n_points, logp, grad, L.lpc, n_lds); break;
-    default: hipLaunchKernelGGL(target_eval_kernel<8>, g, b, shm, st, *target, x, n_points, logp, grad, L.lpc, n_lds); break;
+  switch (target->kind) {
+    case FMC_TARGET_GAUSS_DIAG: launch_eval<FMC_TARGET_GAUSS_DIAG>(st, *target, x, n_points, logp, grad, L); break;
+    case FMC_TARGET_GAUSS_DENSE: launch_eval<FMC_TARGET_GAUSS_DENSE>(st, *target, x, n_points, logp, grad, L); break;
+    case FMC_TARGET_ROSENBROCK: launch_eval<FMC_TARGET_ROSENBROCK>(st, *target, x, n_points, logp, grad, L); break;
+    case FMC_TARGET_FUNNEL: launch_eval<FMC_TARGET_FUNNEL>(st, *target, x, n_points, logp, grad, L); break;
+    case FMC_TARGET_GMM_DIAG: launch_eval<FMC_TARGET_GMM_DIAG>(st, *target, x, n_points, logp, grad, L); break;
+    default: launch_eval<FMC_TARGET_DUAL_MOON>(st, *target, x, n_points, logp, grad, L); break;
   }
   return check_launch("target eval kernel");
 }
@@ -459,7 +494,7 @@ extern "C" int fmc_mala_run(void* stream, const fmc_target* target, float* x, fl
   if ((rc = check_layout(L, target->n_dim))) return rc;
   ChainIO io{x, logp, nullptr, noise, log_u, out_pos, out_logp, out_acc, n_chains, buf_len, cursor, key0, key1};
   StepCfg sc{n_steps, step0, step_size, 0, thinning};
-  return launch_chain<KK_MALA>((hipStream_t)stream, target, io, sc, L);
+  return launch_mala((hipStream_t)stream, target, io, sc, L);
 }
 
 extern "C" int fmc_grw_run(void* stream, const fmc_target* target, float* x, float* logp, int64_t n_chains,
@@ -479,7 +514,7 @@ extern "C" int fmc_grw_run(void* stream, const fmc_target* target, float* x, flo
   if ((rc = check_layout(L, target->n_dim))) return rc;
   ChainIO io{x, logp, nullptr, noise, log_u, out_pos, out_logp, out_acc, n_chains, buf_len, cursor, key0, key1};
   StepCfg sc{n_steps, step0, step_size, 0, thinning};
-  return launch_chain<KK_GRW>((hipStream_t)stream, target, io, sc, L);
+  return launch_grw((hipStream_t)stream, target, io, sc, L);
 }
 
 extern "C" int fmc_tempered_run(void* stream, int32_t kernel, const fmc_target* target, float* x, float* logp,
@@ -508,9 +543,9 @@ extern "C" int fmc_tempered_run(void* stream, int32_t kernel, const fmc_target* 
   io.chol = kernel == FMC_KERNEL_HMC ? momentum_chol : nullptr;
   StepCfg sc{n_steps, step0, step_size, n_leapfrog, 1};
   hipStream_t st = (hipStream_t)stream;
-  if (kernel == FMC_KERNEL_MALA) return launch_chain<KK_MALA>(st, target, io, sc, L);
-  if (kernel == FMC_KERNEL_GRW) return launch_chain<KK_GRW>(st, target, io, sc, L);
-  return launch_chain<KK_HMC>(st, target, io, sc, L);
+  if (kernel == FMC_KERNEL_MALA) return launch_mala(st, target, io, sc, L);
+  if (kernel == FMC_KERNEL_GRW) return launch_grw(st, target, io, sc, L);
+  return launch_hmc(st, target, io, sc, L);
 }
 
 extern "C" int fmc_finite_rows(void* stream, const float* data, int64_t n_rows, int32_t n_dim, int32_t* out) {
@@ -540,8 +575,10 @@ extern "C" int fmc_pt_exchange(void* stream, const float* x_in, float* x_out, fl
   if (n_chains == 0) return FMC_OK;
   const int64_t grid = (n_chains + PT_CPB - 1) / PT_CPB;
   FMC_ARG(grid <= 0x7fffffffLL, "too many chains for one launch");
-  hipLaunchKernelGGL(pt_exchange_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, x_in, x_out,
-                     loglik, temperatures, n_chains, n_temps, n_dim, key0, key1, log_u, accepts);
+  const bool vec = n_dim % 4 == 0 && ((uintptr_t)x_in | (uintptr_t)x_out) % 16 == 0;
+  auto k = vec ? pt_exchange_kernel<true> : pt_exchange_kernel<false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, x_in, x_out, loglik, temperatures,
+                     n_chains, n_temps, n_dim, key0, key1, log_u, accepts);
   return check_launch("tempering exchange");
 }
 
@@ -552,7 +589,7 @@ extern "C" int fmc_pt_adapt(void* stream, float* temperatures, const float* acce
   FMC_ARG(n_chains >= 1, "n_chains must be >= 1");
   if (n_temps < 3) return FMC_OK;  // no interior temperature to move
   FMC_ARG(accepts != nullptr, "accepts is NULL");
-  hipLaunchKernelGGL(pt_adapt_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, temperatures, accepts,
+  hipLaunchKernelGGL(pt_adapt_kernel, dim3(1), dim3(PT_ADAPT), 0, (hipStream_t)stream, temperatures, accepts,
                      n_chains, n_temps);
   return check_launch("temperature adaptation");
 }
@@ -604,7 +641,7 @@ extern "C" int fmc_hmc_run(void* stream, const fmc_target* target, float* x, flo
   ChainIO io{x, logp, metric, noise, log_u, out_pos, out_logp, out_acc, n_chains, buf_len, cursor, key0, key1};
   io.chol = momentum_chol;
   StepCfg sc{n_steps, step0, step_size, n_leapfrog, thinning};
-  return launch_chain<KK_HMC>((hipStream_t)stream, target, io, sc, L);
+  return launch_hmc((hipStream_t)stream, target, io, sc, L);
 }
 
 extern "C" int fmc_mala_propose(void* stream, const float* x, const float* grad, float* prop, int64_t n_chains,

@@ -1,0 +1,12 @@
+// Fused MALA (MALA.kernel, src/flowMC/resource/kernel/MALA.py:26-89): the chain kernels
+// of fmc_chain_kernel.h instantiated for that step kind, in a translation unit
+// of their own.
+#include "fmc_chain_kernel.h"
+
+namespace fmc {
+
+int launch_mala(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg, const Layout& L) {
+  return launch_chain_impl<KK_MALA>(st, t, io, cfg, L);
+}
+
+}  // namespace fmc

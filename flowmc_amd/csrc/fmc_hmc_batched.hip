@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(512) hmc_batched_kernel(const fmc_hmc_slot* __
   const int local = threadIdx.x / lpc;
   if (local >= it.n_chains) return;  // whole chain groups leave together
   const int64_t c = (int64_t)it.chain0 + local;
-  TargetDev t{sl.target.kind, sl.target.n_dim, sl.target.n_modes, sl.target.params};
+  TargetDev t{sl.target.kind, sl.target.n_dim, sl.target.n_modes, (gparam_t)sl.target.params, 0};
   ChainIO io{sl.x,        sl.logp,     sl.metric,  sl.noise,  sl.log_u,  sl.out_pos, sl.out_logp,
              sl.out_acc,  sl.n_chains, sl.buf_len, sl.cursor, sl.key0,   sl.key1};
   io.chol = sl.momentum_chol;
@@ -62,7 +62,7 @@ __device__ __forceinline__ void hmc_unit_fixed(const fmc_work_item& it, const fm
   const int local = threadIdx.x / LPC;
   if (local >= it.n_chains) return;
   const int64_t c = (int64_t)it.chain0 + local;
-  TargetDev t{TK, sl.target.n_dim, sl.target.n_modes, sl.target.params};
+  TargetDev t{TK, sl.target.n_dim, sl.target.n_modes, (gparam_t)sl.target.params, 0};
   ChainIO io{sl.x,        sl.logp,     nullptr,    sl.noise,  sl.log_u,  sl.out_pos, sl.out_logp,
              sl.out_acc,  sl.n_chains, sl.buf_len, sl.cursor, sl.key0,   sl.key1};
   hmc_group<NV, MK_UNIT, TK>(t, io, cfg, c, r, LPC, gbase);

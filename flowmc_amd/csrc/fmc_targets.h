@@ -4,8 +4,11 @@
 // Lane layout: a chain is held by `lpc` consecutive lanes (lane r = 0..lpc-1
 // of the group whose first lane is `gbase`); lane r holds NV float4 chunks,
 // element e of chunk v being dimension  j = (v*lpc + r)*4 + e  (j >= d is
-// padding and must hold 0). Every function returns the full log-density in
+// padding and must hold 0, and its gradient is 0). Every function returns the full log-density in
 // every lane of the group and writes the lane's gradient chunks.
+//
+// Sums of products are written as the FMAs they run as, so that every kernel
+// that inlines a target (fused, batched, per-step evaluation) rounds alike.
 //
 // These replace jax.value_and_grad(logpdf) of the user target at
 // src/flowMC/resource/kernel/MALA.py:59 and jax.grad(potential) at
@@ -13,73 +16,124 @@
 // include/flowmc.h.
 #pragma once
 
+#include <type_traits>
+
 #include "fmc_common.h"
 
 namespace fmc {
+
+// Parameters in global memory (an explicit address space: a generic pointer
+// would make every access a FLAT one), or staged in LDS by stage_target.
+typedef const __attribute__((address_space(1))) float* gparam_t;
+extern __shared__ float fmc_chain_lds[];
 
 struct TargetDev {
   int kind;
   int d;
   int K;           // modes (GMM)
-  const float* p;  // parameter block (LDS copy or global)
+  gparam_t p;      // parameter block
+  int dp;          // row stride of the staged copy: the dims the lanes of a group hold, zero-padded
 };
 
 __device__ __forceinline__ int dim_of(int v, int e, int r, int lpc) { return (v * lpc + r) * 4 + e; }
 
-template <int NV>
+// Four consecutive parameters of a staged row (LDS; zero past the dims)
+__device__ __forceinline__ float4 staged4(int off) { return *reinterpret_cast<const float4*>(fmc_chain_lds + off); }
+
+template <int NV, bool LDSP>
 __device__ __forceinline__ float tgt_gauss_diag(const TargetDev& t, const float4 (&x)[NV],
                                                 float4 (&g)[NV], int r, int lpc) {
-  const float* mean = t.p;
-  const float* prec = t.p + t.d;
   float acc = 0.f;
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
+  for (int v = 0; v < NV; ++v) {
+    float4 m4, p4;
+    if (LDSP) {
+      m4 = staged4(dim_of(v, 0, r, lpc));
+      p4 = staged4(t.dp + dim_of(v, 0, r, lpc));
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       int j = dim_of(v, e, r, lpc);
       float gj = 0.f;
-      if (j < t.d) {
-        float y = f4c(x[v], e) - mean[j];
-        float pr = prec[j];
+      if (LDSP || j < t.d) {
+        float y = f4c(x[v], e) - (LDSP ? f4c(m4, e) : t.p[j]);
+        float pr = LDSP ? f4c(p4, e) : t.p[t.d + j];
         gj = -pr * y;
-        acc += 0.5f * gj * y;
+        acc = fmaf(0.5f * gj, y, acc);
       }
       f4(g[v], e) = gj;
     }
+  }
   return group_sum(acc, lpc);
 }
 
+// Staged: mean, then the precision transposed row by row (row j2 holds P[j][j2]
+// for all j, zero-padded to the dims of the lane group), so that a lane reads
+// its dims of one column as float4 without an index test. With one lane a
+// chain every lane reads the same address (an LDS broadcast); up to 8 dims are
+// held in registers over the steps (DenseRegs: an LDS read a column was 5 round
+// trips a step at d = 5).
 template <int NV>
-__device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const float4 (&x)[NV],
+struct DenseRegs {
+  float4 m[NV], P[4 * NV][NV];
+  __device__ __forceinline__ explicit DenseRegs(const TargetDev& t) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) m[v] = staged4(4 * v);
+#pragma unroll
+    for (int j = 0; j < 4 * NV; ++j)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) P[j][v] = j < t.d ? staged4(t.dp * (j + 1) + 4 * v) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+};
+struct NoRegs {
+  __device__ __forceinline__ explicit NoRegs(const TargetDev&) {}
+};
+
+template <int NV, bool LDSP, class RG>
+__device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                                  float4 (&g)[NV], int r, int lpc, int gbase) {
-  const float* mean = t.p;
-  const float* P = t.p + t.d;  // symmetric [d,d]
+  constexpr bool REG = !std::is_same<RG, NoRegs>::value;
   const int d = t.d;
   float4 y[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
+  for (int v = 0; v < NV; ++v) {
+    float4 m4;
+    if constexpr (REG) m4 = rg.m[v];
+    else if (LDSP) m4 = staged4(dim_of(v, 0, r, lpc));
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       int j = dim_of(v, e, r, lpc);
-      f4(y[v], e) = (j < d) ? f4c(x[v], e) - mean[j] : 0.f;
+      if (LDSP)
+        f4(y[v], e) = f4c(x[v], e) - f4c(m4, e);
+      else
+        f4(y[v], e) = (j < d) ? f4c(x[v], e) - t.p[j] : 0.f;
       f4(g[v], e) = 0.f;
     }
+  }
   // g_i = -sum_j P_ij y_j; y_j gathered from the lane that owns it.
-  for (int s = 0; s < lpc; ++s) {
+  for (int s = 0; s < (REG ? 1 : lpc); ++s) {
 #pragma unroll
     for (int v2 = 0; v2 < NV; ++v2)
 #pragma unroll
       for (int e2 = 0; e2 < 4; ++e2) {
-        float ys = __shfl(f4c(y[v2], e2), gbase + s, 64);
-        int j2 = dim_of(v2, e2, s, lpc);
-        if (j2 < d) {
+        const int j2 = REG ? 4 * v2 + e2 : dim_of(v2, e2, s, lpc);
+        // (in registers by two columns: a zero column costs less than its test)
+        if ((REG ? j2 & ~1 : j2) < d) {
+          const float ys = (REG || lpc == 1) ? f4c(y[v2], e2) : __shfl(f4c(y[v2], e2), gbase + s, 64);
 #pragma unroll
-          for (int v = 0; v < NV; ++v)
+          for (int v = 0; v < NV; ++v) {
+            float4 p4;
+            if constexpr (REG) p4 = rg.P[4 * v2 + e2][v];
+            else if (LDSP) p4 = staged4(t.dp * (j2 + 1) + dim_of(v, 0, r, lpc));
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               int j = dim_of(v, e, r, lpc);
-              if (j < d) f4(g[v], e) -= P[(int64_t)j * d + j2] * ys;
+              if (LDSP)
+                f4(g[v], e) = fmaf(-f4c(p4, e), ys, f4c(g[v], e));
+              else if (j < d)
+                f4(g[v], e) = fmaf(-t.p[d + (int64_t)j * d + j2], ys, f4c(g[v], e));
             }
+          }
         }
       }
   }
@@ -87,8 +141,31 @@ __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const float
 #pragma unroll
   for (int v = 0; v < NV; ++v)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc += 0.5f * f4c(y[v], e) * f4c(g[v], e);
+    for (int e = 0; e < 4; ++e) acc = fmaf(0.5f * f4c(y[v], e), f4c(g[v], e), acc);
   return group_sum(acc, lpc);
+}
+
+// x of the next / previous lane of the wavefront, on the VALU (row shifts
+// stay inside a group of at most 16 lanes; wave shifts above); the lanes at a
+// group's ends take their neighbour elsewhere.
+__device__ __forceinline__ float lane_next(float v, int lpc) {
+  return lpc <= 16 ? dpp_all<0x101>(v) : dpp_all<0x130>(v);  // row_shl:1 / wave_shl:1
+}
+__device__ __forceinline__ float lane_prev(float v, int lpc) {
+  return lpc <= 16 ? dpp_all<0x111>(v) : dpp_all<0x138>(v);  // row_shr:1 / wave_shr:1
+}
+// in the group's first lane: the value of its last lane
+__device__ __forceinline__ float group_last_to_first(float v, int lpc) {
+  if (lpc == 1) return v;
+  if (lpc == 2) return dpp_all<DPP_XOR1>(v);
+  if (lpc == 4) return dpp_all<0x1B>(v);  // quad_perm [3,2,1,0]
+  if (lpc == 8) return dpp_all<DPP_HALF_MIRROR>(v);
+  if (lpc == 64) return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+  const float m = dpp_all<DPP_MIRROR>(v);
+  if (lpc == 16) return m;
+  float lo, hi;
+  swap16(m, lo, hi);
+  return hi;  // lane 0 of a 32-lane half: lane 0 of its second row, which mirrored lane 31
 }
 
 // log p = -scale * sum_{i<d-1} [100 (x_{i+1} - x_i^2)^2 + (1 - x_i)^2]
@@ -101,10 +178,10 @@ __device__ __forceinline__ float tgt_rosenbrock(const TargetDev& t, const float4
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     // x_{j+1} for element 3 and x_{j-1} for element 0 live in neighbouring lanes.
-    float nx_same = __shfl(x[v].x, gbase + ((r + 1) & (lpc - 1)), 64);
+    float nx_same = lane_next(x[v].x, lpc);
     float nx_next = group_bcast0(x[(v + 1 < NV) ? v + 1 : v].x, lpc);
-    float pw_same = __shfl(x[v].w, gbase + ((r - 1) & (lpc - 1)), 64);
-    float pw_prev = __shfl(x[(v > 0) ? v - 1 : 0].w, gbase + lpc - 1, 64);
+    float pw_same = lane_prev(x[v].w, lpc);
+    float pw_prev = group_last_to_first(x[(v > 0) ? v - 1 : 0].w, lpc);
     float nxt3 = (r < lpc - 1) ? nx_same : nx_next;
     float prv0 = (r > 0) ? pw_same : pw_prev;
 #pragma unroll
@@ -115,12 +192,12 @@ __device__ __forceinline__ float tgt_rosenbrock(const TargetDev& t, const float4
       float xp = (e > 0) ? f4c(x[v], e - 1) : prv0;
       float gi = 0.f;
       if (j < d - 1) {
-        float tt = xn - xi * xi;
-        float om = 1.f - xi;
-        acc += 100.f * tt * tt + om * om;
-        gi += -400.f * xi * tt - 2.f * om;
+        const float tt = fmaf(-xi, xi, xn);
+        const float om = 1.f - xi;
+        acc += fmaf(om, om, 100.f * tt * tt);
+        gi = fmaf(-400.f * xi, tt, -2.f * om);
       }
-      if (j > 0 && j < d) gi += 200.f * (xi - xp * xp);
+      if (j > 0 && j < d) gi = fmaf(200.f, fmaf(-xp, xp, xi), gi);
       f4(g[v], e) = -scale * gi;
     }
   }
@@ -132,17 +209,19 @@ __device__ __forceinline__ float tgt_rosenbrock(const TargetDev& t, const float4
 // and get a zero gradient without a per-element index test; only element 0
 // of the group's first lane (v itself) is special. exp(-v) is capped at
 // FLT_MAX so that 0 * exp(-v) stays 0 on padding when e^-v overflows.
-template <int NV>
+// ENTRY (the evaluation at the entry of a MALA / random-walk launch): the
+// first two squares are added the other way round, as in every release so far.
+template <int NV, bool ENTRY>
 __device__ __forceinline__ float tgt_funnel(const TargetDev& t, const float4 (&x)[NV],
                                             float4 (&g)[NV], int r, int lpc, int gbase) {
   const int d = t.d;
   const float v0 = group_bcast0(x[0].x, lpc);
   const float x00 = (r == 0) ? 0.f : x[0].x;
-  float s = x00 * x00;
+  float s = ENTRY ? fmaf(x00, x00, x[0].y * x[0].y) : fmaf(x[0].y, x[0].y, x00 * x00);
 #pragma unroll
   for (int v = 0; v < NV; ++v)
 #pragma unroll
-    for (int e = (v == 0) ? 1 : 0; e < 4; ++e) s += f4c(x[v], e) * f4c(x[v], e);
+    for (int e = (v == 0) ? 2 : 0; e < 4; ++e) s = fmaf(f4c(x[v], e), f4c(x[v], e), s);
   s = group_sum(s, lpc);
   const float em = fminf(expf(-v0), 3.402823466e38f);
   const float nm1 = (float)(d - 1);
@@ -150,56 +229,96 @@ __device__ __forceinline__ float tgt_funnel(const TargetDev& t, const float4 (&x
   for (int v = 0; v < NV; ++v)
 #pragma unroll
     for (int e = 0; e < 4; ++e) f4(g[v], e) = -f4c(x[v], e) * em;
-  const float g0 = -v0 * (1.f / 9.f) - 0.5f * nm1 + 0.5f * em * s;
+  const float g0 = fmaf(0.5f * em, s, fmaf(v0, -1.f / 9.f, -0.5f * nm1));
   if (r == 0) g[0].x = g0;
-  return -v0 * v0 * (1.f / 18.f) - 0.5f * nm1 * v0 - 0.5f * em * s;
+  return fmaf(-0.5f * em, s, fmaf(v0 * v0, -1.f / 18.f, -(0.5f * nm1 * v0)));
 }
 
 // Diagonal Gaussian mixture: log p = logsumexp_k [ c_k - 1/2 sum_j ((x_j - mu_kj) / s_kj)^2 ]
-// with c_k = log w_k - sum_j log s_kj. Online softmax over modes.
-template <int NV>
+// with c_k = log w_k - sum_j log s_kj. Online softmax over modes, without a
+// branch on the lanes: with e = exp(-|q - m|) a new largest mode scales what
+// was summed by e and adds itself once, another adds itself e times (the same
+// FMAs, their operands selected). Where e underflows to 0 for every chain of
+// the wavefront (modes a few sigma apart in many dims), the mode replaces the
+// sums or leaves them alone: no exponential, and its gradient is only formed
+// if it is some chain's largest so far (d = 64, 8 modes, 16 lanes a chain: 624
+// -> 469 VALU instructions a MALA step). Two modes' forms are summed
+// together: their loads and lane sums overlap (20480 tempered rows, 100 steps:
+// 442 -> 420 us, 500 chains 2.1 -> 1.84 us a step; four together take the
+// registers of the fifth wavefront on a SIMD, 487 us).
+template <int NV, bool LDSP>
 __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (&x)[NV],
                                               float4 (&g)[NV], int r, int lpc) {
   const int d = t.d, K = t.K;
-  const float* mu = t.p;
-  const float* is = t.p + (int64_t)K * d;
-  const float* c = t.p + 2 * (int64_t)K * d;
+  const int o_is = K * t.dp, o_c = 2 * K * t.dp;  // staged: mu [K][dp], 1 / s [K][dp], c [K]
   float m = -INFINITY, sw = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) g[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int k = 0; k < K; ++k) {
-    float4 gk[NV];
-    float q = 0.f;
+  // U modes' quadratic forms at once: their loads and sums over the lanes overlap
+  constexpr int U = LDSP && NV <= 2 ? 2 : 1;
+  for (int k0 = 0; k0 < K; k0 += U) {
+    float4 z[U][NV], i4[U][NV];
+    float qs[U];
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u < K ? k0 + u : k0;
+      float q = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        int j = dim_of(v, e, r, lpc);
-        float gj = 0.f;
-        if (j < d) {
-          float isg = is[(int64_t)k * d + j];
-          float z = (f4c(x[v], e) - mu[(int64_t)k * d + j]) * isg;
-          q += z * z;
-          gj = -z * isg;
+      for (int v = 0; v < NV; ++v) {
+        float4 m4;
+        if (LDSP) {
+          m4 = staged4(k * t.dp + dim_of(v, 0, r, lpc));
+          i4[u][v] = staged4(o_is + k * t.dp + dim_of(v, 0, r, lpc));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = dim_of(v, e, r, lpc);
+            f4(m4, e) = j < d ? t.p[(int64_t)k * d + j] : 0.f;
+            f4(i4[u][v], e) = j < d ? t.p[(int64_t)(K + k) * d + j] : 0.f;
+          }
         }
-        f4(gk[v], e) = gj;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f4(z[u][v], e) = (f4c(x[v], e) - f4c(m4, e)) * f4c(i4[u][v], e);
+          q = fmaf(f4c(z[u][v], e), f4c(z[u][v], e), q);
+        }
       }
-    q = c[k] - 0.5f * group_sum(q, lpc);
-    if (q > m) {  // group-uniform branch: q is bitwise equal across the group
-      float sc = expf(m - q);
-      sw = sw * sc + 1.f;
+      qs[u] = q;
+    }
 #pragma unroll
-      for (int v = 0; v < NV; ++v)
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u < K ? k0 + u : k0;
+      qs[u] = fmaf(-0.5f, group_sum(qs[u], lpc), LDSP ? fmc_chain_lds[o_c + k] : t.p[2 * (int64_t)K * d + k]);
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f4(g[v], e) = f4c(g[v], e) * sc + f4c(gk[v], e);
-      m = q;
-    } else {
-      float w = expf(q - m);
-      sw += w;
+    for (int u = 0; u < U; ++u) {
+      if (k0 + u >= K) break;
+      const float q = qs[u];
+      const bool top = q > m;
+      const float a = fabsf(q - m);
+      // (expf gives 0 below -103.97; not for a NaN)
+      if (__builtin_amdgcn_ballot_w64(!(a > 104.f)) == 0) {
+        if (__builtin_amdgcn_ballot_w64(top) != 0) {
+          sw = top ? 1.f : sw;
 #pragma unroll
-      for (int v = 0; v < NV; ++v)
+          for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f4(g[v], e) += w * f4c(gk[v], e);
+            for (int e = 0; e < 4; ++e)
+              f4(g[v], e) = top ? -f4c(z[u][v], e) * f4c(i4[u][v], e) : f4c(g[v], e);
+          m = top ? q : m;
+        }
+      } else {
+        const float w = expf(-a);
+        sw = fmaf(top ? sw : 1.f, w, top ? 1.f : sw);
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float gk = -f4c(z[u][v], e) * f4c(i4[u][v], e);
+            f4(g[v], e) = fmaf(top ? f4c(g[v], e) : gk, w, top ? gk : f4c(g[v], e));
+          }
+        m = top ? q : m;
+      }
     }
   }
   float inv = 1.f / sw;
@@ -213,11 +332,20 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
 // Dual moon (docs/tutorials/dualmoon.ipynb, test/integration/test_MALA.py:11-20):
 // log p = -50 (|x - center| - 2)^2 + LSE_a(-(x0 + a)^2 / (2*0.8^2)) + LSE_a(-(x1 + a)^2 / (2*0.6^2)),
 // a in {-3, +3}. Requires d >= 2.
-template <int NV>
+template <int NV, bool LDSP>
 __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 (&x)[NV],
                                                float4 (&g)[NV], int r, int lpc, int gbase) {
   const int d = t.d;
-  const float* ctr = t.p;
+  float4 ctr[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (LDSP) {
+      ctr[v] = staged4(dim_of(v, 0, r, lpc));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f4(ctr[v], e) = dim_of(v, e, r, lpc) < d ? t.p[dim_of(v, e, r, lpc)] : 0.f;
+    }
+  }
   float n2 = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v)
@@ -225,8 +353,8 @@ __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 
     for (int e = 0; e < 4; ++e) {
       int j = dim_of(v, e, r, lpc);
       if (j < d) {
-        float y = f4c(x[v], e) - ctr[j];
-        n2 += y * y;
+        float y = f4c(x[v], e) - f4c(ctr[v], e);
+        n2 = fmaf(y, y, n2);
       }
     }
   n2 = group_sum(n2, lpc);
@@ -255,7 +383,7 @@ __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 
       int j = dim_of(v, e, r, lpc);
       float gj = 0.f;
       if (j < d) {
-        gj = radial * (f4c(x[v], e) - ctr[j]);
+        gj = radial * (f4c(x[v], e) - f4c(ctr[v], e));
         if (j == 0) gj += g0;
         if (j == 1) gj += g1;
       }
@@ -265,25 +393,55 @@ __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 
 }
 
 // TK >= 0: the kind is fixed at compile time (one target per kernel);
-// TK = -1: dispatch on t.kind at run time.
-template <int NV, int TK = -1>
-__device__ __forceinline__ float target_vg(const TargetDev& t, const float4 (&x)[NV],
+// TK = -1: dispatch on t.kind at run time. LDSP: the parameters are staged in
+// LDS (stage_target).
+// RG: parameters held in registers (DenseRegs), or NoRegs.
+template <int NV, int TK, bool LDSP, bool ENTRY, class RG>
+__device__ __forceinline__ float target_vg(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                            float4 (&g)[NV], int r, int lpc, int gbase) {
   switch (TK >= 0 ? TK : t.kind) {
     case FMC_TARGET_GAUSS_DIAG:
-      return tgt_gauss_diag<NV>(t, x, g, r, lpc);
+      return tgt_gauss_diag<NV, LDSP>(t, x, g, r, lpc);
     case FMC_TARGET_GAUSS_DENSE:
-      return tgt_gauss_dense<NV>(t, x, g, r, lpc, gbase);
+      return tgt_gauss_dense<NV, LDSP>(t, rg, x, g, r, lpc, gbase);
     case FMC_TARGET_ROSENBROCK:
       return tgt_rosenbrock<NV>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_FUNNEL:
-      return tgt_funnel<NV>(t, x, g, r, lpc, gbase);
+      return tgt_funnel<NV, ENTRY>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_GMM_DIAG:
-      return tgt_gmm_diag<NV>(t, x, g, r, lpc);
+      return tgt_gmm_diag<NV, LDSP>(t, x, g, r, lpc);
     case FMC_TARGET_DUAL_MOON:
     default:
-      return tgt_dual_moon<NV>(t, x, g, r, lpc, gbase);
+      return tgt_dual_moon<NV, LDSP>(t, x, g, r, lpc, gbase);
   }
+}
+
+// Floats of the staged parameters of a kind for lane groups holding dp dims.
+inline int64_t target_staged_count(int kind, int d, int K, int dp) {
+  switch (kind) {
+    case FMC_TARGET_GAUSS_DIAG: return 2LL * dp;
+    case FMC_TARGET_GAUSS_DENSE: return (int64_t)dp * (d + 1);
+    case FMC_TARGET_GMM_DIAG: return 2LL * K * dp + K;
+    case FMC_TARGET_DUAL_MOON: return dp;
+    default: return 0;  // Rosenbrock's scale is one scalar load, the funnel has none
+  }
+}
+
+// Copies the parameters of kind TK to LDS rows of dp dims (the whole workgroup).
+template <int TK>
+__device__ __forceinline__ void stage_target(const TargetDev& t) {
+  const int d = t.d, dp = t.dp;
+  const int rows = TK == FMC_TARGET_GAUSS_DIAG ? 2 : TK == FMC_TARGET_GAUSS_DENSE ? d + 1
+                   : TK == FMC_TARGET_GMM_DIAG ? 2 * t.K : TK == FMC_TARGET_DUAL_MOON ? 1 : 0;
+  for (int i = threadIdx.x; i < rows * dp; i += blockDim.x) {
+    const int w = i / dp, j = i - w * dp;
+    float v = 0.f;
+    if (j < d) v = (TK == FMC_TARGET_GAUSS_DENSE && w > 0) ? t.p[d + (int64_t)j * d + (w - 1)] : t.p[(int64_t)w * d + j];
+    fmc_chain_lds[i] = v;
+  }
+  if (TK == FMC_TARGET_GMM_DIAG)
+    for (int k = threadIdx.x; k < t.K; k += blockDim.x) fmc_chain_lds[rows * dp + k] = t.p[2 * (int64_t)t.K * d + k];
+  __syncthreads();
 }
 
 // Number of floats of the parameter block of each kind (host check).
