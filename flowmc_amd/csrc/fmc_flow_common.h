@@ -90,21 +90,26 @@ struct PBF16 {
     return (((float)x[0] + (float)x[1]) + ((float)x[2] + (float)x[3])) +
            (((float)x[4] + (float)x[5]) + ((float)x[6] + (float)x[7]));
   }
+  // e^{2x} as exp2 of one product: 2 log2(e) is twice the rounded log2(e), so
+  // the product rounds as that of 2x and log2(e) does
+  static __device__ __forceinline__ float exp2x(float x) { return __builtin_amdgcn_exp2f(x * 2.885390081777927f); }
   static __device__ __forceinline__ float act(float x) {
     // 1 - 2 / (e^{2x} + 1); the reciprocal from v_rcp_f32 refined by one
     // Newton step (correctly rounded but for rare last-bit cases)
-    const float den = __expf(2.f * x) + 1.f;
+    const float den = exp2x(x) + 1.f;
     float r = __builtin_amdgcn_rcpf(den);
     r = fmaf(fmaf(-den, r, 1.f), r, r);
     return fmaf(-2.f, r, 1.f);
   }
   // two activations with one reciprocal: 1/da = r db, 1/db = r da with
   // r = 1/(da db) (Newton-refined); arguments clamped to |x| <= 15, where
-  // tanh is 1 to FP32 precision, so da db <= (e^30 + 1)^2 stays finite
+  // tanh is 1 to FP32 precision, so da db <= (e^30 + 1)^2 stays finite (the
+  // median of three clamps in one instruction; a NaN gives -15, as max and
+  // min did)
   static __device__ __forceinline__ void act2(float a, float b, float& ha, float& hb) {
-    a = fminf(fmaxf(a, -15.f), 15.f);
-    b = fminf(fmaxf(b, -15.f), 15.f);
-    const float da = __expf(2.f * a) + 1.f, db = __expf(2.f * b) + 1.f;
+    a = __builtin_amdgcn_fmed3f(a, -15.f, 15.f);
+    b = __builtin_amdgcn_fmed3f(b, -15.f, 15.f);
+    const float da = exp2x(a) + 1.f, db = exp2x(b) + 1.f;
     const float p = da * db;
     float r = __builtin_amdgcn_rcpf(p);
     r = fmaf(fmaf(-p, r, 1.f), r, r);
@@ -590,6 +595,24 @@ struct RsBin {
 template <bool FL = false>
 __device__ __forceinline__ float rs_softplus(float v) { return fmaxf(v, 0.f) + fln<FL>(1.f + __expf(-fabsf(v))); }
 
+// The bin of t among S bins (knots 0..S), moved to knots 0 and 1: the half that
+// holds t is kept, S odd keeping the larger count on either side (a bin past
+// the smaller half is never chosen: t is below its left knot).
+template <bool INV, int S, int M>
+__device__ __forceinline__ void rs_halve(float (&X)[M], float (&Y)[M], float (&U)[M], float t) {
+  if constexpr (S > 1) {
+    constexpr int h = S / 2, S1 = S - h;
+    const bool c = t >= (INV ? Y[h] : X[h]);
+#pragma unroll
+    for (int i = 0; i <= S1; ++i) {
+      X[i] = c ? X[h + i] : X[i];
+      Y[i] = c ? Y[h + i] : Y[i];
+      U[i] = c ? U[h + i] : U[i];
+    }
+    rs_halve<INV, S1>(X, Y, U, t);
+  }
+}
+
 // knots of the bin holding t (t along x when INV is false, along y otherwise)
 // KT > 0: the bin count is the compile-time constant KT (loops unrolled to
 // exactly KT, no predication); KT == 0: runtime K <= 10, loops predicated.
@@ -634,9 +657,23 @@ __device__ __forceinline__ RsBin rs_bin(const float (&pp)[32], int Kr, const Flo
     yc = yn[i];
   }
   // The knots increase (every bin is at least mb wide), so the bins whose
-  // right knot t has reached form a prefix: start in bin 0 and move one bin
-  // right, by selects, for every interior knot with t >= knot. This is the
-  // first bin whose right knot exceeds t (t < hi on entry).
+  // right knot t has reached form a prefix; the bin is the first whose right
+  // knot exceeds t (t < hi on entry). A compile-time K halves the candidates
+  // by selects (K = 8: 33 instructions; moving right knot by knot takes 49).
+  if constexpr (KT > 0) {
+    float X[KT + 1], Y[KT + 1], U[KT + 1];
+    X[0] = f.lo;
+    Y[0] = f.lo;
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+      X[i + 1] = xn[i];
+      Y[i + 1] = yn[i];
+      U[i] = pp[20 + i];
+    }
+    U[KT] = pp[30];
+    rs_halve<INV, KT>(X, Y, U, t);
+    return RsBin{X[0], X[1], Y[0], Y[1], U[0], U[1]};
+  }
   RsBin b{f.lo, xn[0], f.lo, yn[0], pp[20], (K == 1) ? pp[30] : pp[21]};
 #pragma unroll
   for (int i = 0; i + 1 < N; ++i) {

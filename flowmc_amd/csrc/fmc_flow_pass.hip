@@ -3,6 +3,7 @@
 // conditioner GEMMs on MFMA with activations in LDS and the spline fused as
 // the epilogue of the last GEMM (rqSpline.py:450-504).
 #include "fmc_flow_common.h"
+#include "fmc_flow_wide.h"
 
 namespace fmc {
 
@@ -424,7 +425,9 @@ extern "C" int fmc_flow_pass(void* stream, const fmc_flow* fl, int32_t direction
   dim3 g((unsigned)((n + MT - 1) / MT)), b(256);
   hipStream_t st = (hipStream_t)stream;
   const int kt = spline_kt(fd.dm.K);
-  if (bf)
+  if (bf && flow_wide(fd.dm, a, device_cus()))
+    launch_flow_wide(st, fd, a);
+  else if (bf)
     launch_pass_kt<PBF16>(kt, fd.dm.nh, g, b, shm, st, fd, a);
   else
     launch_pass_kt<PF32>(kt, fd.dm.nh, g, b, shm, st, fd, a);
