@@ -1,7 +1,7 @@
 // The fused chain kernel (one kernel per lane layout NV, step kind and target
 // kind) and its host-side launch helpers: target-descriptor check, lane
-// layout heuristic and launch. Shared by fmc_chains.hip (MALA, GRW, HMC with
-// a unit or diagonal metric) and fmc_hmc_dense.hip (HMC with a dense
+// layout heuristic and launch. Shared by fmc_chains_mala.hip, fmc_chains_grw.hip,
+// fmc_chains_hmc.hip (a unit or diagonal metric) and fmc_hmc_dense.hip (HMC with a dense
 // condition matrix).
 #pragma once
 

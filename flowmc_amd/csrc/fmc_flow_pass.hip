@@ -14,8 +14,9 @@ namespace fmc {
 // One panel of the pass: EX (grids of at most two workgroups per CU, e.g.
 // training batches of 10^4 samples) uses the exact-wait ring, four k-steps
 // deep, which pays where a wave has few neighbours to hide its waits; the
-// guarded 8-deep ring otherwise (sampling passes of 10^5 samples and more,
-// three workgroups per CU, where the clamped ring's extra loads cost more).
+// guarded 8-deep ring otherwise (large grids that fmc_flow_wide.hip does not
+// take, three workgroups per CU, where the clamped ring's extra loads cost
+// more).
 constexpr int PASS_PF_EX = 4;
 template <bool EX, class PT, int MB, bool TR, int CB = 2>
 __device__ __forceinline__ void pass_panel(const typename PT::T* As, int lda, const typename PT::T* Bp, int KBtot,
