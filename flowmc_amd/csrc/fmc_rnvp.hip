@@ -9,8 +9,8 @@
 // them sums in the order its operands are laid out in). A hidden block of 16
 // features x 16 samples stays in registers from the first product to the
 // next: a lane's four accumulators are the second product's four k-steps.
-//   passes   409,600 samples at d = 32, 8 layers, hidden 256 drawn in 1.10 ms,
-//            98 TFLOP/s (FMA register tiles over LDS: 4.05 ms)
+//   passes   409,600 samples at d = 32, 8 layers, hidden 256 drawn in 1.17 ms,
+//            92 TFLOP/s (FMA register tiles over LDS: 4.05 ms)
 //   training one step of 10,000 samples, same flow: 0.32 ms (1.10 ms with FMA
 //            tiles, one adjoint launch a layer and a partial weight gradient
 //            for every 16 samples): forward 72 us, adjoint of all layers 200,
@@ -243,17 +243,69 @@ struct RnFrag {
   }
 };
 
-// out[r][m] += W2 relu(W1 c + b1) over the hidden blocks hb0, hb0 + hs, ..,
+// Adds the hidden blocks' outputs pairwise in groups of 2^LV and the groups
+// one after the other: the count of blocks so far says which partials merge.
+template <int MB, int LV>
+struct RnPairSum {
+  static_assert(LV == 2 || LV == 3, "levels of pairs");
+  f32x4_t l0[MB], l1[MB], l2[LV == 3 ? MB : 1], total[MB];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      l0[m] = l1[m] = total[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (LV == 3) l2[m] = total[m];
+    }
+  }
+  __device__ __forceinline__ void add(f32x4_t (&v)[MB], int j) {  // block j (0, 1, ..)
+    auto merge = [&](f32x4_t (&l)[MB], bool up) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        if (up)
+          v[m] = l[m] + v[m];
+        else
+          l[m] = v[m];
+      }
+      return up;
+    };
+    if (!merge(l0, j & 1) || !merge(l1, j & 2)) return;
+    if constexpr (LV == 3)
+      if (!merge(l2, j & 4)) return;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) total[m] += v[m];
+  }
+  // the sum after n blocks (partials without a partner, smallest first)
+  __device__ __forceinline__ void finish(int n, f32x4_t (&out)[MB]) const {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      f32x4_t v{0.f, 0.f, 0.f, 0.f};
+      if (n & 1) v = l0[m];
+      if (n & 2) v = l1[m] + v;
+      if constexpr (LV == 3)
+        if (n & 4) v = l2[m] + v;
+      out[m] = total[m] + v;
+    }
+  }
+};
+
+// out[r][m] = W2 relu(W1 c + b1) over the hidden blocks hb0, hb0 + hs, ..,
 // for the row blocks r0 .. r0 + NB - 1. The hidden block (16 features x 16
 // samples) never leaves the registers: a lane's four accumulators are the
-// second product's four k-steps.
-template <int NB, int MB>
+// second product's four k-steps. The sum over the features starts a chain
+// anew every LEAF of them and adds the chains pairwise: one chain through the
+// whole layer had 1.5 times the error of the outputs at d = 32, hidden 256
+// (rms against FP64 2.8e-7 / 1.8e-7) and 2.3 times at hidden 1000.
+template <int NB, int MB, int LEAF>
 __device__ __forceinline__ void rn_mlp(const RnFr& f, int r0, int hb0, int hs, int dc, const f32x4_t (&c)[NB][MB],
                                        const float* xs, int ldx, f32x4_t (&out)[NB][MB], int lane) {
-  if (hb0 >= f.HB) return;
+  constexpr int N = 16 / LEAF;  // chains of a block, one every LEAF / 4 k-steps
+  static_assert(N == 2 || N == 4, "chains of a block");
+  RnPairSum<MB, N == 4 ? 3 : 2> sum[NB];  // (three levels beside chains of eight spill)
+#pragma unroll
+  for (int r = 0; r < NB; ++r) sum[r].clear();
   RnFrag<NB> cur, nxt;
-  cur.load(f, hb0, r0, lane);
-  for (int hb = hb0; hb < f.HB; hb += hs) {
+  if (hb0 < f.HB) cur.load(f, hb0, r0, lane);
+  int j = 0;
+  for (int hb = hb0; hb < f.HB; hb += hs, ++j) {
     nxt.load(f, hb + hs < f.HB ? hb + hs : hb, r0, lane);
     f32x4_t a[MB];
 #pragma unroll
@@ -282,19 +334,42 @@ __device__ __forceinline__ void rn_mlp(const RnFr& f, int r0, int hb0, int hs, i
 #pragma unroll
     for (int r = 0; r < NB; ++r)
       if (r0 + r < f.R) {
+        f32x4_t t[N][MB], v[MB];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int m = 0; m < MB; ++m) out[r][m] = rn_mfma(cur.w2[r][e], a[m][e], out[r][m]);
+          for (int m = 0; m < MB; ++m)
+            t[e * N / 4][m] = rn_mfma(cur.w2[r][e], a[m][e],
+                                      e % (4 / N) == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[e * N / 4][m]);
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+          v[m] = N == 2 ? t[0][m] + t[N - 1][m] : (t[0][m] + t[1][m]) + (t[N / 2][m] + t[N - 1][m]);
+        sum[r].add(v, j);
       }
     cur = nxt;
   }
+#pragma unroll
+  for (int r = 0; r < NB; ++r) sum[r].finish(j, out[r]);
+}
+
+// fine: chains of four features instead of eight, where the sum over S strided
+// chains and their pairs (RnOrder) has chains that short: the error is then no
+// larger than that sum's at any width.
+template <int NB, int MB>
+__device__ __forceinline__ void rn_mlp(bool fine, const RnFr& f, int r0, int hb0, int hs, int dc,
+                                       const f32x4_t (&c)[NB][MB], const float* xs, int ldx, f32x4_t (&out)[NB][MB],
+                                       int lane) {
+  if (fine)
+    rn_mlp<NB, MB, 4>(f, r0, hb0, hs, dc, c, xs, ldx, out, lane);
+  else
+    rn_mlp<NB, MB, 8>(f, r0, hb0, hs, dc, c, xs, ldx, out, lane);
 }
 
 // All layers of a pass for 16 MB samples on the FP32 matrix cores, which bound
-// it at large n (65 % of a large FP32 product's rate at 409,600 samples, the
-// rest tails, tanh / exp and weight reads); small batches are bound by the
-// serial chain of hidden blocks and layers.
+// it at large n (61 % of a large FP32 product's rate at 409,600 samples, the
+// rest the pairwise sums, tails, tanh / exp and weight reads; one chain a layer
+// for 1.10 ms, see rn_mlp); small batches are bound by the serial chain of
+// hidden blocks and layers.
 // SPLIT = false: every wavefront owns 16 MB samples and runs alone (no
 // barrier); SPLIT = true: the eight wavefronts of a workgroup share one
 // 16-sample tile, each taking one MLP (wave & 1) and every fourth hidden
@@ -302,7 +377,7 @@ __device__ __forceinline__ void rn_mlp(const RnFr& f, int r0, int hb0, int hs, i
 // 16 conditioning / transformed dims held in registers; masks that leave more
 // on one side take the loops over the rest.
 template <int NB, int MB, bool SPLIT>
-__global__ void __launch_bounds__(SPLIT ? 512 : 256) __attribute__((amdgpu_waves_per_eu(NB <= 1 ? 4 : 2)))
+__global__ void __launch_bounds__(SPLIT ? 512 : 256) __attribute__((amdgpu_waves_per_eu(NB <= 1 || (SPLIT && NB == 2) ? 4 : 2)))
 rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
   static_assert(!SPLIT || MB == 1, "a shared tile holds 16 samples");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -366,6 +441,10 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
     const int32_t* lay = rn_lay(f, l);
     const int dc = lay[0], dtr = lay[1];
     const RnFr fs(f.packed, d, h, l, 0, dc, dtr), ft(f.packed, d, h, l, 1, dc, dtr);
+    const bool fine = h < 8 * RnOrder(dtr, h).S;
+    float ls[MB];  // the layer's share of the log-dets
+#pragma unroll
+    for (int m = 0; m < MB; ++m) ls[m] = 0.f;
     f32x4_t c[NB][MB];  // conditioning inputs as MFMA operands
 #pragma unroll
     for (int k = 0; k < NB; ++k)
@@ -375,18 +454,14 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
       }
     for (int r0 = 0; r0 < fs.R; r0 += NB) {
       f32x4_t os[NB][MB], ot[NB][MB];
-#pragma unroll
-      for (int r = 0; r < NB; ++r)
-#pragma unroll
-        for (int m = 0; m < MB; ++m) os[r][m] = ot[r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if constexpr (SPLIT) {
-        rn_mlp<NB, MB>((wave & 1) ? ft : fs, r0, wave >> 1, 4, dc, c, xs, ldx, os, lane);
+        rn_mlp<NB, MB>(fine, (wave & 1) ? ft : fs, r0, wave >> 1, 4, dc, c, xs, ldx, os, lane);
 #pragma unroll
         for (int r = 0; r < NB; ++r) *reinterpret_cast<f32x4_t*>(red + ((wave * NB + r) * 64 + lane) * 4) = os[r][0];
         __syncthreads();
       } else {
-        rn_mlp<NB, MB>(fs, r0, 0, 1, dc, c, xs, ldx, os, lane);
-        rn_mlp<NB, MB>(ft, r0, 0, 1, dc, c, xs, ldx, ot, lane);
+        rn_mlp<NB, MB>(fine, fs, r0, 0, 1, dc, c, xs, ldx, os, lane);
+        rn_mlp<NB, MB>(fine, ft, r0, 0, 1, dc, c, xs, ldx, ot, lane);
       }
       // coupling on the transformed dims: a lane holds the scale and shift of
       // dims 16 r + 4 q + e of its sample (SPLIT: row block r by wave r)
@@ -394,13 +469,9 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
       for (int r = 0; r < NB; ++r) {
         if (r0 + r >= fs.R || (SPLIT && wave != r)) continue;
         if constexpr (SPLIT) {
-#pragma unroll
-          for (int w = 0; w < 8; w += 2) {
-            const f32x4_t u = rn_ld4(red + ((w * NB + r) * 64 + lane) * 4);
-            const f32x4_t v = rn_ld4(red + (((w + 1) * NB + r) * 64 + lane) * 4);
-            os[r][0] = w == 0 ? u : os[r][0] + u;
-            ot[r][0] = w == 0 ? v : ot[r][0] + v;
-          }
+          auto part = [&](int w) { return rn_ld4(red + ((w * NB + r) * 64 + lane) * 4); };
+          os[r][0] = (part(0) + part(2)) + (part(4) + part(6));
+          ot[r][0] = (part(1) + part(3)) + (part(5) + part(7));
         }
         const int k0 = 16 * (r0 + r) + 4 * q;
         const f32x4_t bs = rn_ld4(fs.b2 + k0), bt = rn_ld4(ft.b2 + k0);
@@ -415,11 +486,13 @@ rnvp_pass_kernel(RnvpDev f, RnPassArgs a) {
               const float s = tanhf(os[r][m][e] + bs[e]) * f.dt;
               const float tt = (ot[r][m][e] + bt[e]) * f.dt;
               *xp = (a.dir == 0) ? (*xp + tt) * expf(s) : *xp * expf(-s) - tt;
-              ldacc[m] += s;
+              ls[m] += s;
             }
       }
       sync();
     }
+#pragma unroll
+    for (int m = 0; m < MB; ++m) ldacc[m] += ls[m];
   }
   // ---- log-det of each sample: the four lanes that share it (SPLIT: and the
   // waves), in a fixed order
@@ -477,21 +550,24 @@ static int rn_launch_pass(hipStream_t st, const RnvpDev& f, const RnPassArgs& a)
 }
 
 // Which pass runs a batch of n samples (measured, sampling, us; d = 32, 8
-// layers, hidden 256 | d = 64, 10 layers, hidden 128 | d = 5, 4 layers, hidden 64):
-//   n         shared tile (8 waves)   16 samples a wave   32 samples a wave
-//   1000        29 |   39 |  14          82 |   95 |  19      129 |  157 |  26
-//   10000       67 |   92 |  22          86 |  101 |  18      131 |  159 |  25
-//   20000      108 |  147 |  32         123 |  151 |  24      135 |  164 |  25
-//   50000      262 |  350 |  75         219 |  291 |  36      211 |  261 |  36
-//   409600    1825 | 2495 | 534        1177 | 1627 | 186     1101 | 1433 | 171
+// layers, hidden 256 | d = 64, 10 layers, hidden 128 | d = 5, 4 layers, hidden
+// 64 | d = 32, 4 layers, hidden 32):
+//   n         shared tile (8 waves)     16 samples a wave       32 samples a wave
+//   1000        39 |   49 |  17 |  16    106 |  119 |  25 |  22   156 |  183 |  34 |  31
+//   4000        41 |   51 |  17 |  16    107 |  119 |  25 |  22   157 |  183 |  34 |  31
+//   10000       90 |  111 |  36 |  33    106 |  120 |  25 |  23   157 |  183 |  33 |  32
+//   20000      140 |  173 |  55 |  50    140 |  165 |  30 |  27   157 |  184 |  33 |  32
+//   50000      332 |  415 | 132 | 121    225 |  307 |  45 |  39   221 |  270 |  43 |  39
+//   409600    2500 | 3108 | 981 | 906   1290 | 1686 | 231 | 195  1173 | 1696 | 193 | 166
 // A shared tile spreads the serial hidden blocks of a layer over eight waves,
-// which pays until a wave for every 16 samples fills the chip's SIMDs, and
-// less so the fewer hidden blocks there are to spread; 32 samples a wave halve
-// the weight reads once the grid is several waves a SIMD deep. Wide states,
-// whose four tiles would not leave room for two workgroups a CU, share one.
+// which pays up to two workgroups a CU (512 tiles) and, with eight and more
+// blocks to spread, until a wave for every 16 samples fills the chip's SIMDs;
+// 32 samples a wave halve the weight reads once the grid is several waves a
+// SIMD deep. Wide states, whose four tiles would not leave room for two
+// workgroups a CU, share one.
 static int rn_pass_variant(int64_t n, int d, int h) {
-  const int64_t tiles = (n + 15) / 16, split_to = 100 * rn_b16(h);
-  if (4 * rn_rup16(16 * (d + 1) * 4) > 64 * 1024 || tiles <= (split_to < 1280 ? split_to : 1280)) return 0;
+  const int64_t tiles = (n + 15) / 16, hb = rn_b16(h), split_to = hb < 8 ? 512 : hb < 13 ? 100 * hb : 1280;
+  if (4 * rn_rup16(16 * (d + 1) * 4) > 64 * 1024 || tiles <= split_to) return 0;
   return tiles <= 2048 ? 1 : 2;
 }
 
@@ -500,7 +576,7 @@ static int rn_pass_nb(hipStream_t st, const RnvpDev& f, const RnPassArgs& a, int
   switch (var) {
     case 0: return rn_launch_pass<NB, 1, true>(st, f, a);
     case 1: return rn_launch_pass<NB, 1, false>(st, f, a);
-    default: return rn_launch_pass<NB, 2, false>(st, f, a);
+    default: return rn_launch_pass<NB, NB <= 2 ? 2 : 1, false>(st, f, a);  // (four blocks and 32 samples spill)
   }
 }
 
