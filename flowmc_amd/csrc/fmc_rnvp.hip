@@ -1058,22 +1058,30 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
             Ht[e] = rn_relu(Ht[e]);
             sb += gt[e];
           }
+          // (chains of 16 features / samples, then their sums: with one chain
+          // through all of them the input gradients' error was up to 1.14 times
+          // that of short chains, at hidden 1000)
 #pragma unroll
           for (int k = 0; k < NB; ++k)
             if (k0 + k < KC) {
               const f32x4_t cv = frag(cT, k0 + k, m);
+              f32x4_t t1 = zero, t2 = zero;
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                gc[k][m] = rn_mfma(w.w1t[k][e], g[e], gc[k][m]);
-                o1[k] = rn_mfma(gt[e], cv[e], o1[k]);
+                t1 = rn_mfma(w.w1t[k][e], g[e], t1);
+                t2 = rn_mfma(gt[e], cv[e], t2);
               }
+              gc[k][m] += t1;
+              o1[k] += t2;
             }
 #pragma unroll
           for (int r = 0; r < NB; ++r)
             if (k0 + r < R) {
               const f32x4_t gv = frag(gpT, k0 + r, m);
+              f32x4_t t = zero;
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o2[r] = rn_mfma(gv[e], Ht[e], o2[r]);
+              for (int e = 0; e < 4; ++e) t = rn_mfma(gv[e], Ht[e], t);
+              o2[r] += t;
             }
         }
 #pragma unroll
@@ -1098,9 +1106,8 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
       for (int u = wave; u < NB * MS; u += 8) {  // conditioning-input gradients: all shares of both MLPs
         const int k = u / MS, m = u - k * MS;
         if (k0 + k >= KC) continue;
-        f32x4_t v = zero;
-#pragma unroll
-        for (int w8 = 0; w8 < 8; ++w8) v += rn_ld4(red + (((w8 * NB + k) * MS + m) * 64 + lane) * 4);
+        auto at = [&](int w8) { return rn_ld4(red + (((w8 * NB + k) * MS + m) * 64 + lane) * 4); };
+        const f32x4_t v = ((at(0) + at(2)) + (at(4) + at(6))) + ((at(1) + at(3)) + (at(5) + at(7)));
         const int i0 = 16 * (k0 + k) + 4 * q;
         const int4 ci = *reinterpret_cast<const int4*>(fs.cond + i0);
         const int cj[4] = {ci.x, ci.y, ci.z, ci.w};
@@ -1132,8 +1139,10 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
 
 // Sum of the tiles' weight gradients, scattered to the reference-shaped
 // leaves of the gradient vector: a workgroup takes 64 float4 of one layer,
-// wave w the tiles w, w + 4, .. in order; the four sums meet in LDS. Bound by
-// reading the tiles' rows (a wave reads 1 KB of one row at a time).
+// wave w the tiles w, w + 4, .. in four sums that take turns; the sixteen meet
+// in LDS pairwise (four sums over a quarter of the tiles each had twice the
+// error at 60,000 samples and 4.5 times at 400,000). Bound by reading the tiles'
+// rows (a wave reads 1 KB of one row at a time).
 __global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, const float* __restrict__ part, int tiles,
                                                          float* __restrict__ grad) {
   __shared__ f32x4_t sh[4][64];
@@ -1147,15 +1156,19 @@ __global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, cons
   f32x4_t v{0.f, 0.f, 0.f, 0.f};
   if (in) {
     const float* src = part + (int64_t)blockIdx.y * tiles * row + 4 * e4;
+    f32x4_t u[4] = {v, v, v, v};
     int t = w;
     for (; t + 12 < tiles; t += 16) {
-      f32x4_t u[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) u[k] = rn_ld4(src + (int64_t)(t + 4 * k) * row);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v += u[k];
+      for (int k = 0; k < 4; ++k) u[k] += rn_ld4(src + (int64_t)(t + 4 * k) * row);
     }
-    for (; t < tiles; t += 4) v += rn_ld4(src + (int64_t)t * row);
+    for (int k = 0; t < tiles; t += 4, ++k) {
+      const f32x4_t x = rn_ld4(src + (int64_t)t * row);
+      if (k == 0) u[0] += x;
+      else if (k == 1) u[1] += x;
+      else u[2] += x;
+    }
+    v = (u[0] + u[1]) + (u[2] + u[3]);
   }
   sh[w][lane] = v;
   __syncthreads();
