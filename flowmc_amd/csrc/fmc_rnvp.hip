@@ -214,6 +214,8 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4_t rn_mfma(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+// (partial weight gradients may start at any float of a caller's buffer)
+typedef float f32x4_a4_t __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ f32x4_t rn_ld4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
 __device__ __forceinline__ float rn_relu(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, INFINITY); }
 
@@ -1086,8 +1088,8 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
         }
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
-          if (k0 + k < KC) *reinterpret_cast<f32x4_t*>(pp + ((int64_t)hb * KC + k0 + k) * 256 + 4 * lane) = o1[k];
-          if (k0 + k < R) *reinterpret_cast<f32x4_t*>(pw2 + ((int64_t)hb * R + k0 + k) * 256 + 4 * lane) = o2[k];
+          if (k0 + k < KC) *reinterpret_cast<f32x4_a4_t*>(pp + ((int64_t)hb * KC + k0 + k) * 256 + 4 * lane) = o1[k];
+          if (k0 + k < R) *reinterpret_cast<f32x4_a4_t*>(pw2 + ((int64_t)hb * R + k0 + k) * 256 + 4 * lane) = o2[k];
         }
         if (k0 == 0) {
           sb += __shfl_xor(sb, 16, 64);
@@ -1156,14 +1158,15 @@ __global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, cons
   f32x4_t v{0.f, 0.f, 0.f, 0.f};
   if (in) {
     const float* src = part + (int64_t)blockIdx.y * tiles * row + 4 * e4;
+    auto at = [&](int t) -> f32x4_t { return *reinterpret_cast<const f32x4_a4_t*>(src + (int64_t)t * row); };
     f32x4_t u[4] = {v, v, v, v};
     int t = w;
     for (; t + 12 < tiles; t += 16) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) u[k] += rn_ld4(src + (int64_t)(t + 4 * k) * row);
+      for (int k = 0; k < 4; ++k) u[k] += at(t + 4 * k);
     }
     for (int k = 0; t < tiles; t += 4, ++k) {
-      const f32x4_t x = rn_ld4(src + (int64_t)t * row);
+      const f32x4_t x = at(t);
       if (k == 0) u[0] += x;
       else if (k == 1) u[1] += x;
       else u[2] += x;
@@ -1258,8 +1261,9 @@ static int rn_launch_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a) {
   return check_launch("realnvp adjoint");
 }
 
-static int rn_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a) {
-  switch (4 * rn_nb(f.d) + rn_ms((a.n + 15) / 16, f.d)) {
+// ms: 16-sample groups a tile
+static int rn_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a, int ms) {
+  switch (4 * rn_nb(f.d) + ms) {
     case 5: return rn_launch_bwd<1, 1>(st, f, a);
     case 6: return rn_launch_bwd<1, 2>(st, f, a);
     case 7: return rn_launch_bwd<1, 3>(st, f, a);
@@ -1282,9 +1286,7 @@ static int rn_train_pass(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) 
   }
 }
 
-static int rn_wgrad(hipStream_t st, const RnvpDev& f, int l0, int nl, const float* part, int64_t tiles16, float* grad) {
-  const int ms = rn_ms(tiles16, f.d);
-  const int64_t tiles = (tiles16 + ms - 1) / ms;
+static int rn_wgrad(hipStream_t st, const RnvpDev& f, int l0, int nl, const float* part, int64_t tiles, float* grad) {
   const unsigned gx = (unsigned)((rn_part_row(f.d, f.h) / 4 + 63) / 64);
   hipLaunchKernelGGL(rnvp_wgrad_kernel, dim3(gx, (unsigned)nl), dim3(256), 0, st, f, l0, part, (int)tiles, grad);
   return check_launch("realnvp weight gradient");
@@ -1353,7 +1355,8 @@ extern "C" int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* r, int32_t 
   FMC_ARG(n_partial_tiles >= tiles, "partials hold %lld tiles, %lld needed", (long long)n_partial_tiles,
           (long long)tiles);
   if (n == 0) return FMC_OK;
-  return rn_bwd((hipStream_t)stream, f, RnBwdArgs{layer, layer + 1, x_in, n, g_logp, gy, gx, partials});
+  // one row of partials for every 16 samples, whatever n: a caller may sum the rows of several calls
+  return rn_bwd((hipStream_t)stream, f, RnBwdArgs{layer, layer + 1, x_in, n, g_logp, gy, gx, partials}, 1);
 }
 
 extern "C" int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* r, int32_t layer, float* partials,
@@ -1364,7 +1367,9 @@ extern "C" int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* r, int32_t lay
   FMC_ARG(layer >= 0 && layer < f.L, "layer %d out of range", layer);
   FMC_ARG(partials && grad, "NULL pointer");
   FMC_ARG(n_tiles >= 1 && n_tiles <= 0x7fffffffLL, "n_tiles must be >= 1");
-  FMC_ARG(partial_rows >= n_tiles, "partials hold %lld rows, %lld needed", (long long)partial_rows, (long long)n_tiles);
+  const int64_t c = n_tiles < 256 ? (n_tiles + 15) / 16 : 16;  // (spare rows that the interface asks for)
+  FMC_ARG(partial_rows >= n_tiles + c, "partials hold %lld rows, %lld needed (tiles + %lld more)",
+          (long long)partial_rows, (long long)(n_tiles + c), (long long)c);
   return rn_wgrad((hipStream_t)stream, f, layer, 1, partials, n_tiles, grad);
 }
 
@@ -1392,6 +1397,8 @@ extern "C" int fmc_rnvp_backward(void* stream, const fmc_rnvp* r, const float* s
   FMC_ARG(workspace_floats >= need, "workspace holds %lld floats, need %lld (fmc_rnvp_backward_ws_size)",
           (long long)workspace_floats, (long long)need);
   hipStream_t st = (hipStream_t)stream;
-  if ((rc = rn_bwd(st, f, RnBwdArgs{0, f.L, saved, n, g_logp, gy, gx, workspace}))) return rc;
-  return rn_wgrad(st, f, 0, f.L, workspace, (n + 15) / 16, grad);
+  const int64_t t16 = (n + 15) / 16;
+  const int ms = rn_ms(t16, f.d);
+  if ((rc = rn_bwd(st, f, RnBwdArgs{0, f.L, saved, n, g_logp, gy, gx, workspace}, ms))) return rc;
+  return rn_wgrad(st, f, 0, f.L, workspace, (t16 + ms - 1) / ms, grad);
 }

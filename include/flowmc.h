@@ -383,8 +383,10 @@ int fmc_rnvp_pass(void* stream, const fmc_rnvp* flow, int32_t dir, int32_t flags
 /* log_prob: replaces eqx.filter_value_and_grad in NFModel.train_step       */
 /* (nf_model/base.py:98-125) for RealNVP. gy [n, d] = dL/d(layer output)    */
 /* -> gx [n, d] (no aliasing); partials [rows, partial_per_tile] receive    */
-/* the weight gradients by tile, summed in a fixed order by                 */
-/* fmc_rnvp_weight_grad (n_tiles = ceil(n / tile); partial_rows >= n_tiles).*/
+/* the weight gradients of every tile (16 samples: rows 0 .. tiles-1).      */
+/* fmc_rnvp_weight_grad sums n_tiles rows in a fixed order, those of        */
+/* several calls one behind the other too; partial_rows >= n_tiles +        */
+/* min(16, ceil(n_tiles / 16)).                                             */
 int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* flow, int32_t layer, const float* x_in,
                             int64_t n, const float* g_logp, const float* gy, float* gx,
                             float* partials, int64_t n_partial_tiles);
