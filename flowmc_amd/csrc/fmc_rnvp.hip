@@ -848,7 +848,8 @@ __global__ void __launch_bounds__(512) rnvp_train_pass_kernel(RnvpDev f, RnPassA
 // Weight gradients of a tile go to memory in fragment order, per (layer,
 // tile) and p: dW1 [hb][kg][64] float4 (element i of lane l: feature 16 hb +
 // 4 (l / 16) + i, dim 16 kg + l % 16), dW2 [hb][r][64] (dim 16 r + 4 (l / 16)
-// + i, feature 16 hb + l % 16), db1 [16 HB], db2 [16 R].
+// + i, feature 16 hb + l % 16), db1 [16 HB], db2 [16 R]. A workgroup takes the
+// tiles b, b + grid, .. and adds their weight gradients up in its own row.
 struct RnBwdArgs {
   int l0, l1;
   const float* x;  // [l1 - l0, n, d] layer inputs, from layer l0
@@ -856,7 +857,7 @@ struct RnBwdArgs {
   const float* g_logp;
   const float* gy;  // [n, d] dL/d(output of layer l1 - 1)
   float* gx;        // [n, d] dL/d(input of layer l0)
-  float* part;      // [l1 - l0, tiles, rn_part_row]
+  float* part;      // [l1 - l0, workgroups, rn_part_row]
 };
 
 __host__ __device__ inline int64_t rn_part_mlp(int hb, int kc, int r) { return 256LL * hb * (kc + r) + 16 * hb + 16 * r; }
@@ -882,8 +883,8 @@ struct RnBwdFrag {
 };
 
 template <int NB, int MS>
-__global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
+__device__ __forceinline__ void rn_bwd_tile(const RnvpDev& f, const RnBwdArgs& a, int64_t m0, bool first,
+                                            unsigned char* smem) {
   constexpr int S = 16 * MS, NT = 512;
   const int d = f.d, h = f.h, ldx = d + 1, t = threadIdx.x;
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), col = lane & 15, q = lane >> 4;
@@ -895,8 +896,14 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
   // gradients of the scale and of the shift outputs: F with the product's k
   // over the dims, T with k over the samples
   float* cF = red + 8 * NB * MS * 256;
-  const int64_t m0 = (int64_t)blockIdx.x * S;
   const f32x4_t zero{0.f, 0.f, 0.f, 0.f};
+  // (every entry of the row is one lane's, tile after tile)
+  auto keep4 = [&](float* p, f32x4_t v) {
+    f32x4_a4_t* p4 = reinterpret_cast<f32x4_a4_t*>(p);
+    if (!first) v += *p4;
+    *p4 = v;
+  };
+  auto keep = [&](float* p, float v) { *p = first ? v : *p + v; };
 
   for (int o = t; o < S * d; o += NT) {
     const int m = o / d, j = o - m * d;
@@ -1088,13 +1095,13 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
         }
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
-          if (k0 + k < KC) *reinterpret_cast<f32x4_a4_t*>(pp + ((int64_t)hb * KC + k0 + k) * 256 + 4 * lane) = o1[k];
-          if (k0 + k < R) *reinterpret_cast<f32x4_a4_t*>(pw2 + ((int64_t)hb * R + k0 + k) * 256 + 4 * lane) = o2[k];
+          if (k0 + k < KC) keep4(pp + ((int64_t)hb * KC + k0 + k) * 256 + 4 * lane, o1[k]);
+          if (k0 + k < R) keep4(pw2 + ((int64_t)hb * R + k0 + k) * 256 + 4 * lane, o2[k]);
         }
         if (k0 == 0) {
           sb += __shfl_xor(sb, 16, 64);
           sb += __shfl_xor(sb, 32, 64);
-          if (lane < 16) pb1[16 * hb + lane] = sb;
+          if (lane < 16) keep(pb1 + 16 * hb + lane, sb);
         }
       }
 #pragma unroll
@@ -1128,7 +1135,7 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
         }
         s += __shfl_xor(s, 16, 64);
         s += __shfl_xor(s, 32, 64);
-        if (lane < 16) pb1[16 * HB + 16 * r + lane] = s;
+        if (lane < 16) keep(pb1 + 16 * HB + 16 * r + lane, s);
       }
     }
     __syncthreads();  // the fragments are rewritten by the next layer
@@ -1139,13 +1146,30 @@ __global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
   }
 }
 
-// Sum of the tiles' weight gradients, scattered to the reference-shaped
+// MORE: more tiles than workgroups (a kernel of its own: what the loop keeps
+// over the tiles takes 92 bytes of scratch a lane instead of 32 at one block and
+// three groups)
+template <int NB, int MS, bool MORE>
+__global__ void __launch_bounds__(512) rnvp_bwd_kernel(RnvpDev f, RnBwdArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int S = 16 * MS;
+  if constexpr (MORE) {
+    // (a tile starts where every thread has read what it overwrites: its own
+    // entries of the state gradient, the rest before the last barrier)
+    for (int64_t tile = blockIdx.x; tile * S < a.n; tile += gridDim.x)
+      rn_bwd_tile<NB, MS>(f, a, tile * S, tile == blockIdx.x, smem);
+  } else {
+    rn_bwd_tile<NB, MS>(f, a, (int64_t)blockIdx.x * S, true, smem);
+  }
+}
+
+// Sum of the rows of weight gradients, scattered to the reference-shaped
 // leaves of the gradient vector: a workgroup takes 64 float4 of one layer,
-// wave w the tiles w, w + 4, .. in four sums that take turns; the sixteen meet
-// in LDS pairwise (four sums over a quarter of the tiles each had twice the
-// error at 60,000 samples and 4.5 times at 400,000). Bound by reading the tiles'
+// wave w the rows w, w + 4, .. in four sums that take turns; the sixteen meet
+// in LDS pairwise (four sums over a quarter of all tiles each had twice the
+// error at 60,000 samples and 4.5 times at 400,000). Bound by reading the
 // rows (a wave reads 1 KB of one row at a time).
-__global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, const float* __restrict__ part, int tiles,
+__global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, const float* __restrict__ part, int rows,
                                                          float* __restrict__ grad) {
   __shared__ f32x4_t sh[4][64];
   const int d = f.d, h = f.h, l = l0 + blockIdx.y;
@@ -1157,15 +1181,15 @@ __global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, cons
   const bool in = 4 * e4 < 2 * pm;
   f32x4_t v{0.f, 0.f, 0.f, 0.f};
   if (in) {
-    const float* src = part + (int64_t)blockIdx.y * tiles * row + 4 * e4;
+    const float* src = part + (int64_t)blockIdx.y * rows * row + 4 * e4;
     auto at = [&](int t) -> f32x4_t { return *reinterpret_cast<const f32x4_a4_t*>(src + (int64_t)t * row); };
     f32x4_t u[4] = {v, v, v, v};
     int t = w;
-    for (; t + 12 < tiles; t += 16) {
+    for (; t + 12 < rows; t += 16) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) u[k] += at(t + 4 * k);
     }
-    for (int k = 0; t < tiles; t += 4, ++k) {
+    for (int k = 0; t < rows; t += 4, ++k) {
       const f32x4_t x = at(t);
       if (k == 0) u[0] += x;
       else if (k == 1) u[1] += x;
@@ -1241,6 +1265,25 @@ static int rn_ms(int64_t tiles16, int d) {
   return (int)ms;
 }
 
+// How a sweep over all layers is cut: rows of weight gradients (workgroups) and
+// layers a launch. The rows hold what a tile leaves, two workgroups a CU at
+// most (more tiles are added up in them: with a row a tile the workspace grew
+// with the batch and the rows' sum had chains of hundreds of terms), and as
+// many layers share a launch as keep the rows within 256 MB (10,000 samples
+// at d = 32, 8 layers, hidden 256 take 168 MB; d = 128, 10 layers would 1.5 GB).
+struct RnSweep {
+  int ms, layers;
+  int64_t rows;
+  RnSweep(const RnvpDev& f, int64_t n) {
+    const int64_t t16 = (n + 15) / 16;
+    ms = rn_ms(t16, f.d);
+    rows = (t16 + ms - 1) / ms;
+    if (rows > 512) rows = 512;
+    const int64_t fit = (64LL << 20) / (rows * rn_part_row(f.d, f.h));
+    layers = fit < 1 ? 1 : fit > f.L ? f.L : (int)fit;
+  }
+};
+
 template <int NB, int MS>
 static int rn_launch_train(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) {
   const size_t shm = (size_t)rn_rup16(16 * MS * (f.d + 1) * 4) + (8192 + 512 + 1024 * rn_b16(f.d)) * MS;
@@ -1252,25 +1295,25 @@ static int rn_launch_train(hipStream_t st, const RnvpDev& f, const RnPassArgs& a
 }
 
 template <int NB, int MS>
-static int rn_launch_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a) {
+static int rn_launch_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a, int64_t rows) {
   const size_t shm = (size_t)rn_bwd_lds(f.d, NB, MS);
-  if (const int rc = rn_set_lds(rnvp_bwd_kernel<NB, MS>, shm)) return rc;
-  const int64_t grid = (a.n + 16 * MS - 1) / (16 * MS);
-  FMC_ARG(grid <= 0x7fffffffLL, "too many samples for one launch");
-  hipLaunchKernelGGL((rnvp_bwd_kernel<NB, MS>), dim3((unsigned)grid), dim3(512), shm, st, f, a);
+  FMC_ARG(rows <= 0x7fffffffLL, "too many samples for one launch");
+  const auto k = rows * (16 * MS) < a.n ? rnvp_bwd_kernel<NB, MS, true> : rnvp_bwd_kernel<NB, MS, false>;
+  if (const int rc = rn_set_lds(k, shm)) return rc;
+  hipLaunchKernelGGL(k, dim3((unsigned)rows), dim3(512), shm, st, f, a);
   return check_launch("realnvp adjoint");
 }
 
-// ms: 16-sample groups a tile
-static int rn_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a, int ms) {
+// ms: 16-sample groups a tile; rows: workgroups, at most the tiles
+static int rn_bwd(hipStream_t st, const RnvpDev& f, const RnBwdArgs& a, int ms, int64_t rows) {
   switch (4 * rn_nb(f.d) + ms) {
-    case 5: return rn_launch_bwd<1, 1>(st, f, a);
-    case 6: return rn_launch_bwd<1, 2>(st, f, a);
-    case 7: return rn_launch_bwd<1, 3>(st, f, a);
-    case 9: return rn_launch_bwd<2, 1>(st, f, a);
-    case 10: return rn_launch_bwd<2, 2>(st, f, a);
-    case 11: return rn_launch_bwd<2, 3>(st, f, a);
-    default: return rn_launch_bwd<4, 1>(st, f, a);
+    case 5: return rn_launch_bwd<1, 1>(st, f, a, rows);
+    case 6: return rn_launch_bwd<1, 2>(st, f, a, rows);
+    case 7: return rn_launch_bwd<1, 3>(st, f, a, rows);
+    case 9: return rn_launch_bwd<2, 1>(st, f, a, rows);
+    case 10: return rn_launch_bwd<2, 2>(st, f, a, rows);
+    case 11: return rn_launch_bwd<2, 3>(st, f, a, rows);
+    default: return rn_launch_bwd<4, 1>(st, f, a, rows);
   }
 }
 
@@ -1286,9 +1329,9 @@ static int rn_train_pass(hipStream_t st, const RnvpDev& f, const RnPassArgs& a) 
   }
 }
 
-static int rn_wgrad(hipStream_t st, const RnvpDev& f, int l0, int nl, const float* part, int64_t tiles, float* grad) {
+static int rn_wgrad(hipStream_t st, const RnvpDev& f, int l0, int nl, const float* part, int64_t rows, float* grad) {
   const unsigned gx = (unsigned)((rn_part_row(f.d, f.h) / 4 + 63) / 64);
-  hipLaunchKernelGGL(rnvp_wgrad_kernel, dim3(gx, (unsigned)nl), dim3(256), 0, st, f, l0, part, (int)tiles, grad);
+  hipLaunchKernelGGL(rnvp_wgrad_kernel, dim3(gx, (unsigned)nl), dim3(256), 0, st, f, l0, part, (int)rows, grad);
   return check_launch("realnvp weight gradient");
 }
 
@@ -1356,7 +1399,7 @@ extern "C" int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* r, int32_t 
           (long long)tiles);
   if (n == 0) return FMC_OK;
   // one row of partials for every 16 samples, whatever n: a caller may sum the rows of several calls
-  return rn_bwd((hipStream_t)stream, f, RnBwdArgs{layer, layer + 1, x_in, n, g_logp, gy, gx, partials}, 1);
+  return rn_bwd((hipStream_t)stream, f, RnBwdArgs{layer, layer + 1, x_in, n, g_logp, gy, gx, partials}, 1, tiles);
 }
 
 extern "C" int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* r, int32_t layer, float* partials,
@@ -1378,9 +1421,8 @@ extern "C" int fmc_rnvp_backward_ws_size(const fmc_rnvp* r, int64_t n, int64_t* 
   int rc = check_rnvp(r, f, false);
   if (rc) return rc;
   FMC_ARG(n >= 1 && floats != nullptr, "n must be >= 1 and floats not NULL");
-  const int64_t t16 = (n + 15) / 16;
-  const int ms = rn_ms(t16, f.d);
-  *floats = (int64_t)f.L * ((t16 + ms - 1) / ms) * rn_part_row(f.d, f.h);
+  const RnSweep sw(f, n);
+  *floats = sw.layers * sw.rows * rn_part_row(f.d, f.h);
   return FMC_OK;
 }
 
@@ -1392,13 +1434,17 @@ extern "C" int fmc_rnvp_backward(void* stream, const fmc_rnvp* r, const float* s
   FMC_ARG(n >= 1, "n must be >= 1");
   FMC_ARG(saved && g_logp && gy && gx && grad && workspace, "NULL pointer");
   FMC_ARG((uintptr_t)workspace % 16 == 0, "workspace must be 16-byte aligned");
-  int64_t need = 0;
-  if ((rc = fmc_rnvp_backward_ws_size(r, n, &need))) return rc;
+  const RnSweep sw(f, n);
+  const int64_t need = sw.layers * sw.rows * rn_part_row(f.d, f.h);
   FMC_ARG(workspace_floats >= need, "workspace holds %lld floats, need %lld (fmc_rnvp_backward_ws_size)",
           (long long)workspace_floats, (long long)need);
   hipStream_t st = (hipStream_t)stream;
-  const int64_t t16 = (n + 15) / 16;
-  const int ms = rn_ms(t16, f.d);
-  if ((rc = rn_bwd(st, f, RnBwdArgs{0, f.L, saved, n, g_logp, gy, gx, workspace}, ms))) return rc;
-  return rn_wgrad(st, f, 0, f.L, workspace, (t16 + ms - 1) / ms, grad);
+  for (int l1 = f.L; l1 > 0; l1 -= sw.layers) {
+    const int l0 = l1 > sw.layers ? l1 - sw.layers : 0;
+    // (a tile reads its gradient rows before it writes them: gx in place)
+    const RnBwdArgs a{l0, l1, saved + (int64_t)l0 * n * f.d, n, g_logp, l1 == f.L ? gy : gx, gx, workspace};
+    if ((rc = rn_bwd(st, f, a, sw.ms, sw.rows))) return rc;
+    if ((rc = rn_wgrad(st, f, l0, l1 - l0, workspace, sw.rows, grad))) return rc;
+  }
+  return FMC_OK;
 }

@@ -393,7 +393,9 @@ int fmc_rnvp_backward_layer(void* stream, const fmc_rnvp* flow, int32_t layer, c
 int fmc_rnvp_weight_grad(void* stream, const fmc_rnvp* flow, int32_t layer, float* partials,
                          int64_t n_tiles, int64_t partial_rows, float* grad);
 /* The whole backward sweep in two launches: the adjoint of every layer and */
-/* tile, then the weight gradients of all layers (every parameter entry of  */
+/* tile, then the weight gradients of all layers (two launches for a few    */
+/* layers at a time where the workspace of all would exceed 256 MB; it does */
+/* not grow with n past some ten thousand samples; every parameter entry of */
 /* grad that can be non-zero is written; masked weights and the statistics  */
 /* are left alone: clear grad once). saved [L, n, d] and gy as              */
 /* fmc_rnvp_pass wrote them; gx [n, d] = dL/d(standardised input) (no       */
