@@ -47,6 +47,7 @@ chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg, int lpc_rt, int dp, NoiseRi
   const int lpc = LPC ? LPC : lpc_rt;
   const TargetDev t{tg.kind, tg.n_dim, tg.n_modes, (gparam_t)tg.params, dp};
   if (PARAMS && dp > 0) stage_target<TK>(t);
+  if (PARAMS && LPC == 0 && dp == STAGE_RAW) stage_raw(t, (int)target_param_count(TK, t.d, t.K));
   const int lane = threadIdx.x & 63;
   const int r = lane & (lpc - 1);
   const int gbase = lane - r;
@@ -69,28 +70,30 @@ chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg, int lpc_rt, int dp, NoiseRi
   }
   if (c >= io.C) return;  // whole group leaves together
   auto run = [&](auto staged) {
-    constexpr bool LDSP = decltype(staged)::value;
+    constexpr int PAR = decltype(staged)::value;
     using RG = std::conditional_t<TK == FMC_TARGET_GAUSS_DENSE && LPC == 1 && NV <= 2, DenseRegs<NV>, NoRegs>;
     if constexpr (KIND == KK_MALA)
-      mala_group<NV, TK, LDSP, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+      mala_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
     else if constexpr (KIND == KK_GRW)
-      grw_group<NV, TK, LDSP, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+      grw_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
     else if constexpr (KIND == KK_HMC_DENSE)
-      hmc_group<NV, MK_DENSE, TK, LDSP, NoRegs>(t, io, cfg, c, r, lpc, gbase);
+      hmc_group<NV, MK_DENSE, TK, PAR, NoRegs>(t, io, cfg, c, r, lpc, gbase);
     else if (io.metric)
-      hmc_group<NV, MK_DIAG, TK, LDSP, RG>(t, io, cfg, c, r, lpc, gbase);
+      hmc_group<NV, MK_DIAG, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
     else
-      hmc_group<NV, MK_UNIT, TK, LDSP, RG>(t, io, cfg, c, r, lpc, gbase);
+      hmc_group<NV, MK_UNIT, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
   };
   if constexpr (!PARAMS) {
-    run(std::false_type{});
+    run(std::integral_constant<int, PAR_MEM>{});
   } else if constexpr (LPC > 0) {
-    run(std::true_type{});
+    run(std::integral_constant<int, PAR_ROWS>{});
   } else {
     if (dp > 0)
-      run(std::true_type{});
+      run(std::integral_constant<int, PAR_ROWS>{});
+    else if (dp == STAGE_RAW)
+      run(std::integral_constant<int, PAR_RAW>{});
     else
-      run(std::false_type{});
+      run(std::integral_constant<int, PAR_MEM>{});
   }
 }
 
@@ -155,14 +158,23 @@ static inline int check_layout(const Layout& L, int d) {
   return FMC_OK;
 }
 
-// Row stride of the staged parameters for a layout (0: not staged).
+// How a layout stages the parameters: the stride of rows padded to the lanes'
+// dims where they fit the 64 KB of LDS that need no attribute, STAGE_RAW where
+// only the unpadded block fits 48 KB (the rows are up to twice as long: d = 65
+// takes 128 dims a row), else STAGE_NONE. 32 MALA steps of 4096 chains, us,
+// padded / unpadded / from memory: dense d = 100 1652 / 4883 / 9359, mixture d =
+// 65 with 60 modes 542 / 715 / 1012, with 93 modes - / 1088 / 1563.
 static inline int staged_stride(const fmc_target* t, const Layout& L) {
   const int dp = 4 * L.nv * L.lpc;
   const int64_t n = target_staged_count(t->kind, t->n_dim, t->n_modes, dp);
-  return (n > 0 && n * 4 <= 48 * 1024) ? dp : 0;
+  if (n == 0) return STAGE_NONE;
+  if (((n + 3) & ~3LL) * 4 <= 64 * 1024) return dp;
+  return target_param_count(t->kind, t->n_dim, t->n_modes) * 4 <= 48 * 1024 ? STAGE_RAW : STAGE_NONE;
 }
 static inline int staged_floats(const fmc_target* t, int dp) {
-  return dp ? (int)((target_staged_count(t->kind, t->n_dim, t->n_modes, dp) + 3) & ~3LL) : 0;
+  if (dp == STAGE_NONE) return 0;
+  return (int)(((dp > 0 ? target_staged_count(t->kind, t->n_dim, t->n_modes, dp)
+                        : target_param_count(t->kind, t->n_dim, t->n_modes)) + 3) & ~3LL);
 }
 
 // Whether a workgroup is one chain wavefront and three that draw its random

@@ -223,7 +223,7 @@ __device__ __forceinline__ float temper(const ChainIO& io, float beta, float lp,
 // MALA.py:26-89). The gradient at the current point is carried from the
 // previous step instead of being re-evaluated: MALA.py:59 recomputes it at the
 // same point, which for a deterministic target is the same value.
-template <int NV, int TK, bool LDSP, bool RING, class RG>
+template <int NV, int TK, int PAR, bool RING, class RG>
 __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg,
                                            const NoiseRing& nr, int64_t c, int r, int lpc, int gbase) {
   const int d = t.d;
@@ -231,7 +231,7 @@ __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io
   float4 x[NV], g[NV];
   load_row<NV>(io.x + c * d, d, r, lpc, x);
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, true>(t, rg, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, PAR, true>(t, rg, x, g, r, lpc, gbase), g);
   const float dt = cfg.dt;
   const float h = 0.5f * dt * dt;
   const float inv2dt2 = 1.f / (2.f * dt * dt);
@@ -251,7 +251,7 @@ __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io
         f4(prop[v], e) = fmaf(dt, f4c(xi[v], e), fmaf(h, f4c(g[v], e), f4c(x[v], e)));
         s1 = fmaf(n, n, s1);
       }
-    float lp1 = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, prop, g1, r, lpc, gbase), g1);
+    float lp1 = temper<NV>(io, beta, target_vg<NV, TK, PAR, false>(t, rg, prop, g1, r, lpc, gbase), g1);
     float s2 = 0.f;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
@@ -285,7 +285,7 @@ __device__ __forceinline__ void mala_group(const TargetDev& t, const ChainIO& io
 // log u < logp(x') - logp(x). The log-density of the entry state is evaluated
 // once (take_steps.py:177) and carried; the target's gradient output is dead
 // and removed by the compiler.
-template <int NV, int TK, bool LDSP, bool RING, class RG>
+template <int NV, int TK, int PAR, bool RING, class RG>
 __device__ __forceinline__ void grw_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg,
                                           const NoiseRing& nr, int64_t c, int r, int lpc, int gbase) {
   const int d = t.d;
@@ -293,7 +293,7 @@ __device__ __forceinline__ void grw_group(const TargetDev& t, const ChainIO& io,
   float4 x[NV], g[NV];
   load_row<NV>(io.x + c * d, d, r, lpc, x);
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, true>(t, rg, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, PAR, true>(t, rg, x, g, r, lpc, gbase), g);
   const float dt = cfg.dt;
   RowWriter rows(io, cfg, d, c);
   float lu_keep = 0.f;
@@ -306,7 +306,7 @@ __device__ __forceinline__ void grw_group(const TargetDev& t, const ChainIO& io,
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) f4(prop[v], e) = fmaf(dt, f4c(xi[v], e), f4c(x[v], e));
-    const float lp1 = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, prop, g, r, lpc, gbase), g);
+    const float lp1 = temper<NV>(io, beta, target_vg<NV, TK, PAR, false>(t, rg, prop, g, r, lpc, gbase), g);
     const bool acc = lu < lp1 - lp;
     if (acc) {
 #pragma unroll
@@ -371,7 +371,7 @@ __device__ __forceinline__ void dense_momentum(const float* __restrict__ Lc, int
   }
 }
 
-template <int NV, int MK, int TK, bool LDSP = false, class RG = NoRegs>
+template <int NV, int MK, int TK, int PAR = PAR_MEM, class RG = NoRegs>
 __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg, int64_t c,
                           int r, int lpc, int gbase) {
   constexpr bool UNIT_M = MK == MK_UNIT;
@@ -386,7 +386,7 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
     for (int v = 0; v < NV; ++v) m[v] = make_float4(1.f, 1.f, 1.f, 1.f);
   }
   const float beta = row_beta(io, c);
-  float lp = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, x, g, r, lpc, gbase), g);
+  float lp = temper<NV>(io, beta, target_vg<NV, TK, PAR, false>(t, rg, x, g, r, lpc, gbase), g);
   const float eps = cfg.dt;
   const int L = cfg.n_leapfrog;
   RowWriter rows(io, cfg, d, c);
@@ -439,7 +439,7 @@ __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io,
       for (int v = 0; v < NV; ++v)
 #pragma unroll
         for (int e = 0; e < 4; ++e) f4(xl[v], e) = fmaf(eps, UNIT_M ? f4c(p[v], e) : f4c(m[v], e) * f4c(p[v], e), f4c(xl[v], e));
-      lpl = temper<NV>(io, beta, target_vg<NV, TK, LDSP, false>(t, rg, xl, gl, r, lpc, gbase), gl);
+      lpl = temper<NV>(io, beta, target_vg<NV, TK, PAR, false>(t, rg, xl, gl, r, lpc, gbase), gl);
 #pragma unroll
       for (int v = 0; v < NV; ++v)
 #pragma unroll

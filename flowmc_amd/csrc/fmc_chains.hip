@@ -18,6 +18,7 @@ __global__ void __launch_bounds__(256) target_eval_kernel(fmc_target tg, const f
                                                           int lpc, int dp) {
   const TargetDev t{tg.kind, tg.n_dim, tg.n_modes, (gparam_t)tg.params, dp};
   if (dp > 0) stage_target<TK>(t);
+  if (dp == STAGE_RAW) stage_raw(t, (int)target_param_count(TK, t.d, t.K));
   const int lane = threadIdx.x & 63;
   const int r = lane & (lpc - 1);
   const int gbase = lane - r;
@@ -26,8 +27,9 @@ __global__ void __launch_bounds__(256) target_eval_kernel(fmc_target tg, const f
   const int d = t.d;
   float4 xv[NV], g[NV];
   load_row<NV>(x + c * d, d, r, lpc, xv);
-  const float lp = dp > 0 ? target_vg<NV, TK, true, false>(t, NoRegs(t), xv, g, r, lpc, gbase)
-                          : target_vg<NV, TK, false, false>(t, NoRegs(t), xv, g, r, lpc, gbase);
+  const float lp = dp > 0            ? target_vg<NV, TK, PAR_ROWS, false>(t, NoRegs(t), xv, g, r, lpc, gbase)
+                   : dp == STAGE_RAW ? target_vg<NV, TK, PAR_RAW, false>(t, NoRegs(t), xv, g, r, lpc, gbase)
+                                     : target_vg<NV, TK, PAR_MEM, false>(t, NoRegs(t), xv, g, r, lpc, gbase);
   if (grad) store_row<NV>(grad + c * d, d, r, lpc, g);
   if (r == 0 && logp) logp[c] = lp;
 }

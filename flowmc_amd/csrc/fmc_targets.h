@@ -32,22 +32,33 @@ struct TargetDev {
   int d;
   int K;           // modes (GMM)
   gparam_t p;      // parameter block
-  int dp;          // row stride of the staged copy: the dims the lanes of a group hold, zero-padded
+  int dp;          // row stride of the padded staged copy (the dims the lanes of a group hold), or STAGE_*
 };
 
 __device__ __forceinline__ int dim_of(int v, int e, int r, int lpc) { return (v * lpc + r) * 4 + e; }
 
+// Where a kernel reads the parameters: memory, LDS rows padded to the lanes'
+// dims, or an unpadded LDS copy, for parameters that fit the LDS only so.
+enum { PAR_MEM = 0, PAR_ROWS = 1, PAR_RAW = 2 };
+constexpr int STAGE_NONE = 0, STAGE_RAW = -1;
+
+// Parameter i of the block (not of padded rows)
+template <int PAR>
+__device__ __forceinline__ float param(const TargetDev& t, int64_t i) {
+  return PAR == PAR_RAW ? fmc_chain_lds[i] : t.p[i];
+}
+
 // Four consecutive parameters of a staged row (LDS; zero past the dims)
 __device__ __forceinline__ float4 staged4(int off) { return *reinterpret_cast<const float4*>(fmc_chain_lds + off); }
 
-template <int NV, bool LDSP>
+template <int NV, int PAR>
 __device__ __forceinline__ float tgt_gauss_diag(const TargetDev& t, const float4 (&x)[NV],
                                                 float4 (&g)[NV], int r, int lpc) {
   float acc = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     float4 m4, p4;
-    if (LDSP) {
+    if (PAR == PAR_ROWS) {
       m4 = staged4(dim_of(v, 0, r, lpc));
       p4 = staged4(t.dp + dim_of(v, 0, r, lpc));
     }
@@ -55,9 +66,9 @@ __device__ __forceinline__ float tgt_gauss_diag(const TargetDev& t, const float4
     for (int e = 0; e < 4; ++e) {
       int j = dim_of(v, e, r, lpc);
       float gj = 0.f;
-      if (LDSP || j < t.d) {
-        float y = f4c(x[v], e) - (LDSP ? f4c(m4, e) : t.p[j]);
-        float pr = LDSP ? f4c(p4, e) : t.p[t.d + j];
+      if (PAR == PAR_ROWS || j < t.d) {
+        float y = f4c(x[v], e) - (PAR == PAR_ROWS ? f4c(m4, e) : param<PAR>(t, j));
+        float pr = PAR == PAR_ROWS ? f4c(p4, e) : param<PAR>(t, t.d + j);
         gj = -pr * y;
         acc = fmaf(0.5f * gj, y, acc);
       }
@@ -89,7 +100,7 @@ struct NoRegs {
   __device__ __forceinline__ explicit NoRegs(const TargetDev&) {}
 };
 
-template <int NV, bool LDSP, class RG>
+template <int NV, int PAR, class RG>
 __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                                  float4 (&g)[NV], int r, int lpc, int gbase) {
   constexpr bool REG = !std::is_same<RG, NoRegs>::value;
@@ -99,14 +110,14 @@ __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& r
   for (int v = 0; v < NV; ++v) {
     float4 m4;
     if constexpr (REG) m4 = rg.m[v];
-    else if (LDSP) m4 = staged4(dim_of(v, 0, r, lpc));
+    else if (PAR == PAR_ROWS) m4 = staged4(dim_of(v, 0, r, lpc));
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       int j = dim_of(v, e, r, lpc);
-      if (LDSP)
+      if (PAR == PAR_ROWS)
         f4(y[v], e) = f4c(x[v], e) - f4c(m4, e);
       else
-        f4(y[v], e) = (j < d) ? f4c(x[v], e) - t.p[j] : 0.f;
+        f4(y[v], e) = (j < d) ? f4c(x[v], e) - param<PAR>(t, j) : 0.f;
       f4(g[v], e) = 0.f;
     }
   }
@@ -124,14 +135,14 @@ __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& r
           for (int v = 0; v < NV; ++v) {
             float4 p4;
             if constexpr (REG) p4 = rg.P[4 * v2 + e2][v];
-            else if (LDSP) p4 = staged4(t.dp * (j2 + 1) + dim_of(v, 0, r, lpc));
+            else if (PAR == PAR_ROWS) p4 = staged4(t.dp * (j2 + 1) + dim_of(v, 0, r, lpc));
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               int j = dim_of(v, e, r, lpc);
-              if (LDSP)
+              if (PAR == PAR_ROWS)
                 f4(g[v], e) = fmaf(-f4c(p4, e), ys, f4c(g[v], e));
               else if (j < d)
-                f4(g[v], e) = fmaf(-t.p[d + (int64_t)j * d + j2], ys, f4c(g[v], e));
+                f4(g[v], e) = fmaf(-param<PAR>(t, d + (int64_t)j * d + j2), ys, f4c(g[v], e));
             }
           }
         }
@@ -246,7 +257,7 @@ __device__ __forceinline__ float tgt_funnel(const TargetDev& t, const float4 (&x
 // together: their loads and lane sums overlap (20480 tempered rows, 100 steps:
 // 442 -> 420 us, 500 chains 2.1 -> 1.84 us a step; four together take the
 // registers of the fifth wavefront on a SIMD, 487 us).
-template <int NV, bool LDSP>
+template <int NV, int PAR>
 __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (&x)[NV],
                                               float4 (&g)[NV], int r, int lpc) {
   const int d = t.d, K = t.K;
@@ -255,7 +266,7 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
 #pragma unroll
   for (int v = 0; v < NV; ++v) g[v] = make_float4(0.f, 0.f, 0.f, 0.f);
   // U modes' quadratic forms at once: their loads and sums over the lanes overlap
-  constexpr int U = LDSP && NV <= 2 ? 2 : 1;
+  constexpr int U = PAR != PAR_MEM && NV <= 2 ? 2 : 1;
   for (int k0 = 0; k0 < K; k0 += U) {
     float4 z[U][NV], i4[U][NV];
     float qs[U];
@@ -266,15 +277,15 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         float4 m4;
-        if (LDSP) {
+        if (PAR == PAR_ROWS) {
           m4 = staged4(k * t.dp + dim_of(v, 0, r, lpc));
           i4[u][v] = staged4(o_is + k * t.dp + dim_of(v, 0, r, lpc));
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int j = dim_of(v, e, r, lpc);
-            f4(m4, e) = j < d ? t.p[(int64_t)k * d + j] : 0.f;
-            f4(i4[u][v], e) = j < d ? t.p[(int64_t)(K + k) * d + j] : 0.f;
+            f4(m4, e) = j < d ? param<PAR>(t, (int64_t)k * d + j) : 0.f;
+            f4(i4[u][v], e) = j < d ? param<PAR>(t, (int64_t)(K + k) * d + j) : 0.f;
           }
         }
 #pragma unroll
@@ -288,7 +299,7 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = k0 + u < K ? k0 + u : k0;
-      qs[u] = fmaf(-0.5f, group_sum(qs[u], lpc), LDSP ? fmc_chain_lds[o_c + k] : t.p[2 * (int64_t)K * d + k]);
+      qs[u] = fmaf(-0.5f, group_sum(qs[u], lpc), PAR == PAR_ROWS ? fmc_chain_lds[o_c + k] : param<PAR>(t, 2 * (int64_t)K * d + k));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -332,18 +343,18 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
 // Dual moon (docs/tutorials/dualmoon.ipynb, test/integration/test_MALA.py:11-20):
 // log p = -50 (|x - center| - 2)^2 + LSE_a(-(x0 + a)^2 / (2*0.8^2)) + LSE_a(-(x1 + a)^2 / (2*0.6^2)),
 // a in {-3, +3}. Requires d >= 2.
-template <int NV, bool LDSP>
+template <int NV, int PAR>
 __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 (&x)[NV],
                                                float4 (&g)[NV], int r, int lpc, int gbase) {
   const int d = t.d;
   float4 ctr[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    if (LDSP) {
+    if (PAR == PAR_ROWS) {
       ctr[v] = staged4(dim_of(v, 0, r, lpc));
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) f4(ctr[v], e) = dim_of(v, e, r, lpc) < d ? t.p[dim_of(v, e, r, lpc)] : 0.f;
+      for (int e = 0; e < 4; ++e) f4(ctr[v], e) = dim_of(v, e, r, lpc) < d ? param<PAR>(t, dim_of(v, e, r, lpc)) : 0.f;
     }
   }
   float n2 = 0.f;
@@ -393,26 +404,26 @@ __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 
 }
 
 // TK >= 0: the kind is fixed at compile time (one target per kernel);
-// TK = -1: dispatch on t.kind at run time. LDSP: the parameters are staged in
-// LDS (stage_target).
+// TK = -1: dispatch on t.kind at run time. PAR: where the parameters are
+// (stage_target, stage_raw).
 // RG: parameters held in registers (DenseRegs), or NoRegs.
-template <int NV, int TK, bool LDSP, bool ENTRY, class RG>
+template <int NV, int TK, int PAR, bool ENTRY, class RG>
 __device__ __forceinline__ float target_vg(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                            float4 (&g)[NV], int r, int lpc, int gbase) {
   switch (TK >= 0 ? TK : t.kind) {
     case FMC_TARGET_GAUSS_DIAG:
-      return tgt_gauss_diag<NV, LDSP>(t, x, g, r, lpc);
+      return tgt_gauss_diag<NV, PAR>(t, x, g, r, lpc);
     case FMC_TARGET_GAUSS_DENSE:
-      return tgt_gauss_dense<NV, LDSP>(t, rg, x, g, r, lpc, gbase);
+      return tgt_gauss_dense<NV, PAR>(t, rg, x, g, r, lpc, gbase);
     case FMC_TARGET_ROSENBROCK:
       return tgt_rosenbrock<NV>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_FUNNEL:
       return tgt_funnel<NV, ENTRY>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_GMM_DIAG:
-      return tgt_gmm_diag<NV, LDSP>(t, x, g, r, lpc);
+      return tgt_gmm_diag<NV, PAR>(t, x, g, r, lpc);
     case FMC_TARGET_DUAL_MOON:
     default:
-      return tgt_dual_moon<NV, LDSP>(t, x, g, r, lpc, gbase);
+      return tgt_dual_moon<NV, PAR>(t, x, g, r, lpc, gbase);
   }
 }
 
@@ -444,8 +455,14 @@ __device__ __forceinline__ void stage_target(const TargetDev& t) {
   __syncthreads();
 }
 
+// Copies the n parameters to LDS as they are (the whole workgroup).
+__device__ __forceinline__ void stage_raw(const TargetDev& t, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) fmc_chain_lds[i] = t.p[i];
+  __syncthreads();
+}
+
 // Number of floats of the parameter block of each kind (host check).
-inline int64_t target_param_count(int kind, int d, int K) {
+__host__ __device__ inline int64_t target_param_count(int kind, int d, int K) {
   switch (kind) {
     case FMC_TARGET_GAUSS_DIAG: return 2LL * d;
     case FMC_TARGET_GAUSS_DENSE: return (int64_t)d + (int64_t)d * d;
