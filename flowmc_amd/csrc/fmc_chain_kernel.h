@@ -238,7 +238,10 @@ static void launch_chain_kind(hipStream_t st, const fmc_target* t, const ChainIO
         if (L.lpc == 1) {
           switch (L.nv) {
             case 1: launch_chain_lpc<1, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
-            case 2: launch_chain_lpc<2, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
+            case 2:
+              if (t->n_dim <= 4) break;  // (registers: no chunk of padding only)
+              launch_chain_lpc<2, KIND, TK, 1>(st, t, io, cfg, L, dp);
+              return;
             case 4: launch_chain_lpc<4, KIND, TK, 1>(st, t, io, cfg, L, dp); return;
             default: break;
           }

@@ -152,7 +152,12 @@ __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& r
 #pragma unroll
   for (int v = 0; v < NV; ++v)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc = fmaf(0.5f * f4c(y[v], e), f4c(g[v], e), acc);
+    for (int e = 0; e < 4; ++e) {
+      // (a padding row's zeros make a NaN of an infinite y; parameters in
+      // registers have padding in their last chunk only)
+      if (PAR == PAR_ROWS && (!REG || (v == NV - 1 && e > 0)) && dim_of(v, e, r, lpc) >= d) f4(g[v], e) = 0.f;
+      acc = fmaf(0.5f * f4c(y[v], e), f4c(g[v], e), acc);
+    }
   return group_sum(acc, lpc);
 }
 

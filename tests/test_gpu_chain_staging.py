@@ -55,3 +55,24 @@ def test_parameters_that_fit_unpadded(gpu, name, d, k):
         moved = acc.any(1)
         assert int(moved.sum()) > 65
         assert torch.equal(end[moved], lp[moved])
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 7, 9, 18, 33, 110])
+def test_dense_gaussian_at_infinity(gpu, d):
+    """Every entry of the precision and of x - mean positive: the log-density is
+    -inf, and so is every entry of the gradient."""
+    p = torch.eye(d, dtype=torch.float64) + 0.5
+    t = TG.GaussianDense(torch.zeros(d, dtype=torch.float64), p)
+    x = torch.ones(d, d) + torch.diag(torch.full((d,), float("inf")))
+    lp, gr = torch.empty(d, device="cuda"), torch.empty(d, d, device="cuda")
+    desc, xg = t.descriptor(), x.cuda()
+    N.call("fmc_target_eval", N.stream_ptr(), C.byref(desc), xg.data_ptr(), d, lp.data_ptr(), gr.data_ptr(), None)
+    assert torch.equal(lp.cpu(), torch.full((d,), -float("inf")))
+    assert torch.equal(gr.cpu(), torch.full((d, d), -float("inf")))
+    for cfg in (None, N.fmc_launch_cfg(1, 2, 256, 0)):  # two chunks a lane: also with padding in both
+        if cfg is not None and d > 8:
+            continue
+        y, end = xg.clone(), torch.empty(d, device="cuda")  # a chain that starts there keeps its state
+        N.call("fmc_mala_run", N.stream_ptr(), C.byref(desc), y.data_ptr(), end.data_ptr(), d, 3, 0, 0.05, 1, 2, None, None,
+               None, None, None, 0, 0, 1, None if cfg is None else C.byref(cfg))
+        assert torch.equal(y, xg) and torch.equal(end.cpu(), lp.cpu())
