@@ -188,6 +188,19 @@ struct FlowDims {
     return (int64_t)(l / 2) * (pk_size(0) + pk_size(1)) + ((l & 1) ? pk_size(0) : 0);
   }
   FMC_HD int64_t pk_total() const { return pk_layer(L); }
+  // where reads end that run through the 32-row blocks of the hidden layers and
+  // of w3r in whole groups of `ahead` k-steps of 16 (512 elements each)
+  int64_t pk_read_end(int ahead) const {
+    int64_t end = 0;
+    for (int l = L > 2 ? L - 2 : 0; l < L; ++l)  // (the layers before lie two whole layers ahead of the end)
+      for (int i = 0; i <= nh; ++i) {
+        const int rows = i < nh ? hp(i) : n3r(l), K = i < nh ? wh_k(l, i) : hlp();
+        const int64_t e = pk_layer(l) + (i < nh ? pk_wh(l, i) : pk_w3r(l)) + (int64_t)(rows - 32) * K +
+                          (int64_t)rup(K / 16, ahead) * 512;
+        if (rows > 0 && e > end) end = e;
+      }
+    return end;
+  }
   // packed biases (FP32)
   FMC_HD int64_t pb_b(int i) const { return hsp[i]; }  // hidden layer i
   FMC_HD int64_t pb_b3(int) const { return pb_b(nh); }  // chunked output-layer bias

@@ -6,6 +6,7 @@
 namespace fmc {
 
 constexpr int WIDE_MT = 64;  // samples a workgroup
+constexpr int WD_P = 4;      // k-steps of weight fragments in flight
 
 struct WideSmem {
   int xs, ldw, h, b, total;  // byte offsets: tile, the wavefronts' partial log-dets, activations, a layer's biases
@@ -31,7 +32,7 @@ struct WideSmem {
 // Whether a pass goes the wide way. It takes a BF16 conditioner of up to 256
 // units a layer (a wavefront holds a whole layer's share of a tile across the
 // barrier), register splines, a diagonal base and no saved layer inputs; two
-// workgroups a CU have to fit the LDS. More samples than the small-grid
+// workgroups a CU have to fit the LDS, and the ring's reads the packed buffer. More samples than the small-grid
 // passes (whose eight wavefronts sum the log-dets in another order), and
 // enough for its half as many workgroups to fill the chip: general / wide, us,
 // n = 20000 | 33000 | 50000 | 100000:
@@ -42,6 +43,7 @@ struct WideSmem {
 inline bool flow_wide(const FlowDims& dm, const PassArgs& a, int cus) {
   if (!dm.reg_spline() || dm.base_dense || dm.hmaxp() > 256 || a.saved || a.gy_out) return false;
   if (dm.pk_total() * 2 >= (1LL << 31) || WideSmem(dm).total > 80 * 1024) return false;
+  if (dm.pk_read_end(WD_P) > dm.pk_total()) return false;  // (no layout so far: w3rt is at least as long as w3r's last steps)
   bool broad = true;
   for (int i = 0; i < dm.nh; ++i) broad = broad && dm.hp(i) > 128;
   return a.n > (broad ? 64 : 160) * (int64_t)cus;

@@ -6,8 +6,6 @@
 
 namespace fmc {
 
-// k-steps of weight fragments in flight
-constexpr int WD_P = 4;
 constexpr int WD_MB = WIDE_MT / 32;  // 32-sample blocks of the tile
 struct WdRing {
   bf16x8_t r[WD_P][2];
@@ -19,8 +17,11 @@ struct WdPanel {
   int KB;
 };
 // Fragments come by buffer loads: the block and k-step as a scalar offset, the
-// lane's place as the vector offset (no address arithmetic on the lanes), and
-// the ring may read past a panel of few k-steps (past the buffer: zeros).
+// lane's place as the vector offset (no address arithmetic on the lanes). The
+// ring reads up to WD_P - 1 k-steps past a panel and uses none of them: what
+// follows a panel in the packed buffer is another image, after the last w3r
+// panel the transposed one (flow_wide checks it; a bounds check of the load
+// would not count the scalar offset).
 struct WdSrc {
   __amdgpu_buffer_rsrc_t rs;
   int voff;
