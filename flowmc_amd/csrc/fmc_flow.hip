@@ -967,14 +967,6 @@ extern "C" int fmc_adamw_clip_dev(void* stream, float* theta, const float* grad,
                     workspace_len, grad_norm);
 }
 
-// The whole backward sweep of a training step (nf_model/base.py:98-125, the
-// gradient of NFModel.loss_fn): per layer, last to first, the adjoint on
-// `stream`, then that layer's weight gradient. With a side stream the weight
-// gradient of layer l runs there beside the adjoint of layer l-1: the two
-// stores / affine-partial buffers alternate between layers, an adjoint waits
-// for the weight gradient that last read its store, and `stream` joins the
-// side stream before returning. The events are the call's own (created and
-// released here), so overlapping calls on other streams do not interfere.
 // p[0:n) = 0 (a kernel rather than a memset, so that a caller may record the
 // sweep into a HIP graph); float4 stores when p is 16-byte aligned
 __global__ void __launch_bounds__(256) zero_kernel(float* __restrict__ p, int64_t n, int vec) {
@@ -989,13 +981,58 @@ __global__ void __launch_bounds__(256) zero_kernel(float* __restrict__ p, int64_
   for (int64_t i = i0; i < n; i += stride) p[i] = 0.f;
 }
 
+// The events of a backward sweep on two streams: the calling thread's own, kept
+// from call to call. A call may be recorded into a HIP graph, and an event must
+// not be released while the capture that recorded it is open: the runtime visits
+// a capture's events when it ends. A wait takes the event's last record at the
+// time of the call, so overlapping calls on other streams do not interfere.
+struct SweepEvents {
+  static constexpr int MAX_DEV = 16;
+  int n = 0, dev[MAX_DEV];
+  hipEvent_t ev[MAX_DEV][3];  // adjoint done; weight gradient of store 0 / 1 done
+  ~SweepEvents() {
+    for (int i = 0; i < n; ++i)
+      for (hipEvent_t e : ev[i]) (void)hipEventDestroy(e);
+  }
+  // the current device's three events, or NULL with the error set
+  const hipEvent_t* get() {
+    int d = 0;
+    if (hipGetDevice(&d) != hipSuccess) {
+      set_error(FMC_ERR_HIP, "hipGetDevice failed");
+      return nullptr;
+    }
+    for (int i = 0; i < n; ++i)
+      if (dev[i] == d) return ev[i];
+    if (n == MAX_DEV) {
+      set_error(FMC_ERR_HIP, "a thread runs backward sweeps on at most %d devices", MAX_DEV);
+      return nullptr;
+    }
+    for (int k = 0; k < 3; ++k)
+      if (hipEventCreateWithFlags(&ev[n][k], hipEventDisableTiming) != hipSuccess) {
+        while (k-- > 0) (void)hipEventDestroy(ev[n][k]);
+        set_error(FMC_ERR_HIP, "hipEventCreateWithFlags failed");
+        return nullptr;
+      }
+    dev[n] = d;
+    return ev[n++];
+  }
+};
+static thread_local SweepEvents g_sweep_events;
+
+// The whole backward sweep of a training step (nf_model/base.py:98-125, the
+// gradient of NFModel.loss_fn): per layer, last to first, the adjoint on
+// `stream`, then that layer's weight gradient. With a side stream the weight
+// gradient of layer l runs there beside the adjoint of layer l-1: the two
+// stores / affine-partial buffers alternate between layers, an adjoint waits
+// for the weight gradient that last read its store, and `stream` joins the
+// side stream before returning.
 extern "C" int fmc_flow_backward(void* stream, void* side_stream, const fmc_flow* fl, const float* saved, int64_t n,
                                  const float* g_logp, float* gy, float* gx, void* store0, void* store1,
                                  int64_t store_ld, float* aff0, float* aff1, int32_t n_partials, float* grad,
                                  int32_t split, float* wg_workspace, int64_t wg_workspace_bytes) {
   FMC_ARG(fl != nullptr && saved && g_logp && gy && gx && store0 && aff0 && grad, "NULL pointer");
-  const bool two = side_stream != nullptr;
-  FMC_ARG(!two || (store1 != nullptr && aff1 != nullptr), "the side-stream schedule needs store1 and aff1");
+  const bool two = side_stream != nullptr && side_stream != stream;  // (one stream twice: nothing to overlap)
+  FMC_ARG(side_stream == nullptr || (store1 != nullptr && aff1 != nullptr), "the side-stream schedule needs store1 and aff1");
   FMC_ARG(!split || wg_workspace != nullptr, "the split weight gradient needs its workspace");
   FMC_ARG(fl->n_layers >= 1 && n >= 1, "bad n_layers / n");
   FlowDev fd;
@@ -1005,16 +1042,9 @@ extern "C" int fmc_flow_backward(void* stream, void* side_stream, const fmc_flow
     set_error(FMC_ERR_HIP, "%s failed", what);
     return (int)FMC_ERR_HIP;
   };
-  hipEvent_t ev_adj = nullptr, ev_wg[2] = {nullptr, nullptr};
-  if (two) {
-    for (hipEvent_t* e : {&ev_adj, &ev_wg[0], &ev_wg[1]}) {
-      if (hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) {
-        for (hipEvent_t x : {ev_adj, ev_wg[0], ev_wg[1]})
-          if (x) (void)hipEventDestroy(x);
-        return hip_fail("hipEventCreateWithFlags");
-      }
-    }
-  }
+  const hipEvent_t* ev = two ? g_sweep_events.get() : nullptr;
+  if (two && ev == nullptr) return FMC_ERR_HIP;
+  const hipEvent_t ev_adj = two ? ev[0] : nullptr, ev_wg[2] = {two ? ev[1] : nullptr, two ? ev[2] : nullptr};
   bool pending[2] = {false, false};
   int rc = FMC_OK;
   const int L = fl->n_layers;
@@ -1070,7 +1100,6 @@ extern "C" int fmc_flow_backward(void* stream, void* side_stream, const fmc_flow
     for (int b = 0; b < 2; ++b)
       if (pending[b] && hipStreamWaitEvent(main_st, ev_wg[b], 0) != hipSuccess && rc == FMC_OK)
         rc = hip_fail("hipStreamWaitEvent");
-    for (hipEvent_t x : {ev_adj, ev_wg[0], ev_wg[1]}) (void)hipEventDestroy(x);
   }
   return rc;
 }

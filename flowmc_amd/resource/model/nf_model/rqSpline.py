@@ -11,6 +11,7 @@ operand image packed from it in ``precision`` ("bfloat16" default, or
 from __future__ import annotations
 
 import ctypes as C
+import gc
 import json
 import math
 from typing import Optional
@@ -526,17 +527,30 @@ class MaskedCouplingRQSpline(NFModel):
                state.nu.data_ptr(), float(optim.learning_rate), float(optim.b1), float(optim.b2), float(optim.eps),
                float(optim.weight_decay), optim.max_norm, self._base_dense)
         if getattr(ws, "graph_key", None) != key:
-            ws.graph = None
+            if getattr(ws, "graph", None) is not None:
+                torch.cuda.synchronize(self.device)  # its last replay may still run
+            ws.graph = ws.graph_key = None
             ws.x_static = torch.empty((B, self._n_features), dtype=torch.float32, device=self.device)
             ws.step_dev = torch.zeros(1, dtype=torch.int32, device=self.device)
             ws.step_next = None  # the count step_dev holds for the next replay
             self._ensure_packed()  # (recording runs nothing: theta stays as it is)
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                s = self._struct()
-                _native.call("fmc_flow_pack", _native.stream_ptr(), C.byref(s))
-                self._train_body(ws.x_static, ws, optim, state, ws.step_dev, want_loss=False)
-                ws.step_dev.add_(1)  # the next replay's count, without a launch outside the graph
+            # no garbage collection while recording: a dropped flow that is part of
+            # a reference cycle would have its own recording destroyed, which
+            # waits for the device, in the middle of this one
+            collecting = gc.isenabled()
+            gc.disable()
+            try:
+                with torch.cuda.graph(g):
+                    s = self._struct()
+                    _native.call("fmc_flow_pack", _native.stream_ptr(), C.byref(s))
+                    self._train_body(ws.x_static, ws, optim, state, ws.step_dev, want_loss=False)
+                    ws.step_dev.add_(1)  # the next replay's count, without a launch outside the graph
+            finally:
+                if collecting:
+                    gc.enable()
+            # the buffers behind the recorded addresses live as long as the recording
+            ws.graph_uses = (self.theta, self.packed, self.packed_bias, state.mu, state.nu)
             ws.graph, ws.graph_key = g, key
         ws.x_static.copy_(xb)
         state.count += 1
