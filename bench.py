@@ -331,7 +331,7 @@ def bench_nfmcmc(args):
     fl = flow_flops_per_sample(d, L, K, H) * C_ * S
     achieved = fl / (ms * 1e-3) / 1e12
     traffic = None  # HBM bytes per launch from the counter runs of the same pass (flow_pass workload)
-    tf = os.path.join(ROOT, "profiles", "flow_pass_kernel_traffic.json")
+    tf = os.path.join(ROOT, "profiles", "flow_wide_kernel_traffic.json")
     if os.path.exists(tf) and C_ * S == 409600:
         with open(tf) as f:
             traffic = json.load(f).get("bytes_per_launch")
@@ -345,7 +345,7 @@ def bench_nfmcmc(args):
         # weight gradients (the next two) beside it
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / BF16_PEAK_TFLOPS, "traffic": traffic,
-                     "kernel": "flow_pass_kernel (exact inverse over the 409,600 proposals of a global step, BF16)",
+                     "kernel": "flow_wide_kernel (exact inverse over the 409,600 proposals of a global step, BF16)",
                      "kernel_ms": ms, "flops_per_launch": fl},
         "extra": {"wall_s": wall, **an, "local_acceptance": local_acc, "global_acceptance": global_acc,
                   "mode_occupancy": occupancy,
@@ -696,7 +696,7 @@ def bench_flow_pass(args):
     bins, [256, 256]), ``--steps`` launches. It also runs one 256 MiB
     device-to-device copy (a kernel of known traffic) so that counter runs
     (FETCH_SIZE / WRITE_SIZE) can be scaled to bytes. Traffic measured that
-    way is read from profiles/flow_pass_kernel_traffic.json when present."""
+    way is read from profiles/flow_wide_kernel_traffic.json when present."""
     import torch
 
     from flowmc_amd import random as fr
@@ -713,8 +713,10 @@ def bench_flow_pass(args):
     ms = time_kernel(lambda: m.sample(fr.PRNGKey(1), n), reps=args.steps)
     fl = flow_flops_per_sample(d, L, K, H) * n
     achieved = fl / (ms * 1e-3) / 1e12
+    # (an FP32 conditioner takes the general pass, whose traffic is not counted)
+    kernel = "flow_wide_kernel" if args.precision == "bfloat16" else "flow_pass_kernel"
     traffic = None
-    tf = os.path.join(ROOT, "profiles", "flow_pass_kernel_traffic.json")
+    tf = os.path.join(ROOT, "profiles", kernel + "_traffic.json")
     if os.path.exists(tf):
         with open(tf) as f:
             traffic = json.load(f).get("bytes_per_launch")
@@ -724,7 +726,7 @@ def bench_flow_pass(args):
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_PEAK_TFLOPS if args.precision == "bfloat16"
                      else FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / (BF16_PEAK_TFLOPS if args.precision == "bfloat16" else FP32_PEAK_TFLOPS),
-                     "traffic": traffic, "kernel": "flow_pass_kernel (exact inverse)", "kernel_ms": ms,
+                     "traffic": traffic, "kernel": kernel + " (exact inverse)", "kernel_ms": ms,
                      "flops_per_launch": fl, "algorithmic_bytes_per_launch": n * (d * 4 * 2)},
         "config": {"workload": "flow_pass", "samples": n, "dim": d, "layers": L, "bins": K, "hidden": H,
                    "precision": args.precision},
@@ -775,9 +777,9 @@ def bench_realnvp_train(args):
     out = {
         "value": args.steps * B / wall,
         "ms_per_step": wall * 1e3 / args.steps,
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP32_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "train step (fused forward + per-layer adjoint + partial reduction + AdamW), FP32",
+                     "kernel": "train step (fused forward + adjoint of all layers + weight-gradient sums + AdamW), FP32",
                      "flops_per_step": fl_step},
         "extra": {"loss_before": l0, "loss_after": l1, "sample_ms_409600": ms_s,
                   "sample_tflops": fl_fwd * n_s / (ms_s * 1e-3) / 1e12},

@@ -22,7 +22,7 @@ enum KernelKind { KK_MALA = 0, KK_HMC = 1, KK_GRW = 2, KK_HMC_DENSE = 3 };
 // the 128-D Rosenbrock 350, of the 8-mode 64-D mixture 469) and, with few
 // chains, the wait of a lone wavefront between them. us, the same calls with
 // one kernel for all targets, parameters read from memory and runtime lane
-// counts -> now: 1000 MALA steps of 1000 5-D dense-Gaussian chains 3133 -> 712;
+// counts -> now: 1000 MALA steps of 1000 5-D dense-Gaussian chains 3133 -> 714;
 // 64 of 16384 128-D Rosenbrock chains 237 -> 164; 100 tempered steps of 20480
 // 64-D mixture rows 660 -> 370; 128 HMC steps of 2301 27-D Rosenbrock chains
 // 9.6 -> 4.5 a step.

@@ -13,8 +13,10 @@
 //            92 TFLOP/s (FMA register tiles over LDS: 4.05 ms)
 //   training one step of 10,000 samples, same flow: 0.32 ms (1.10 ms with FMA
 //            tiles, one adjoint launch a layer and a partial weight gradient
-//            for every 16 samples): forward 72 us, adjoint of all layers 200,
+//            for every 16 samples): forward 72 us, adjoint of all layers 205,
 //            weight-gradient sums 19
+// Sums keep short chains that are added pairwise (rn_mlp, RnOrder, the adjoint):
+// the matrix cores would as well add everything in one.
 #include "fmc_common.h"
 
 namespace fmc {
@@ -1229,20 +1231,6 @@ __global__ void __launch_bounds__(256) rnvp_wgrad_kernel(RnvpDev f, int l0, cons
 }
 
 // ---------------------------------------------------------------- host ---
-static int check_rnvp(const fmc_rnvp* r, RnvpDev& f, bool need_packed) {
-  FMC_ARG(r != nullptr, "RealNVP description is NULL");
-  FMC_ARG(r->n_dim >= 1 && r->n_layers >= 1 && r->n_hidden >= 1, "n_dim, n_layers and n_hidden must be >= 1");
-  FMC_ARG(r->theta != nullptr && r->layout != nullptr, "theta or layout is NULL");
-  FMC_ARG(!need_packed || r->packed != nullptr, "packed buffer is NULL");
-  // the sizes these kernels take: 16 samples' state, gradient and hidden rows in 160 KB
-  const int64_t d4 = (r->n_dim + 3) & ~3, h4 = (r->n_hidden + 3) & ~3;
-  const int64_t need = 2 * ((64LL * (r->n_dim + 1) + 15) & ~15LL) + 64 * (4 * d4 + 2 * h4) + 128;
-  FMC_ARG(need <= 160 * 1024, "n_dim %d / n_hidden %d exceed the LDS budget of the RealNVP kernels", r->n_dim,
-          r->n_hidden);
-  f = RnvpDev{r->n_dim, r->n_layers, r->n_hidden, r->dt, r->theta, r->packed, r->layout};
-  return FMC_OK;
-}
-
 // blocks of 16 dims held in registers: a mask that halves the dims fits (up
 // to 128 dims; past 256, two, for the adjoint's LDS)
 static inline int rn_nb(int d) {
@@ -1253,6 +1241,25 @@ static inline int64_t rn_bwd_lds(int d, int nb, int ms) {
   // fragments: 2 KC + 4 R blocks of 1 KB, KC + R <= ceil(d / 16) + 1
   return (int64_t)rn_rup16(16 * ms * (d + 1) * 4) + 64 * ms + 8192LL * nb * ms + 1024LL * ms * (4 * rn_b16(d) + 2);
 }
+static int check_rnvp(const fmc_rnvp* r, RnvpDev& f, bool need_packed) {
+  FMC_ARG(r != nullptr, "RealNVP description is NULL");
+  FMC_ARG(r->n_dim >= 1 && r->n_layers >= 1 && r->n_hidden >= 1, "n_dim, n_layers and n_hidden must be >= 1");
+  FMC_ARG(r->theta != nullptr && r->layout != nullptr, "theta or layout is NULL");
+  FMC_ARG(!need_packed || r->packed != nullptr, "packed buffer is NULL");
+  // the sizes taken: a bound from kernels that kept hidden rows in LDS, kept so
+  // that what is refused stays refused. It admits d <= 424 and hidden <= 1268,
+  // and the tiles of these kernels (a 16-sample adjoint the largest) fit 160 KB
+  // for all of them (checked below).
+  const int64_t d4 = (r->n_dim + 3) & ~3, h4 = (r->n_hidden + 3) & ~3;
+  const int64_t need = 2 * ((64LL * (r->n_dim + 1) + 15) & ~15LL) + 64 * (4 * d4 + 2 * h4) + 128;
+  FMC_ARG(need <= 160 * 1024, "n_dim %d / n_hidden %d exceed the LDS budget of the RealNVP kernels", r->n_dim,
+          r->n_hidden);
+  FMC_ARG(rn_bwd_lds(r->n_dim, rn_nb(r->n_dim), 1) <= 160 * 1024, "n_dim %d exceeds the LDS of the RealNVP adjoint",
+          r->n_dim);
+  f = RnvpDev{r->n_dim, r->n_layers, r->n_hidden, r->dt, r->theta, r->packed, r->layout};
+  return FMC_OK;
+}
+
 // 16-sample groups per workgroup of the training kernels: as many as leave one
 // workgroup a CU, up to three (four spill; measured at d = 32, 8 layers,
 // hidden 256, adjoint + forward, n = 10,000: one group 433 + 120 us, two 353 +

@@ -8,7 +8,9 @@
 // every lane of the group and writes the lane's gradient chunks.
 //
 // Sums of products are written as the FMAs they run as, so that every kernel
-// that inlines a target (fused, batched, per-step evaluation) rounds alike.
+// that inlines a target (fused, batched, per-step evaluation) rounds alike,
+// with one exception: the funnel's evaluation at the entry of a MALA or
+// random-walk launch (ENTRY) adds two squares in the other order.
 //
 // These replace jax.value_and_grad(logpdf) of the user target at
 // src/flowMC/resource/kernel/MALA.py:59 and jax.grad(potential) at
