@@ -65,3 +65,42 @@ def test_hidden_sums(gpu, d, h, n):
         return float(np.sqrt(np.mean((v - exact) ** 2)))
 
     assert rms(got) <= 1.1 * rms(acc[0].astype(np.float64))
+
+
+def _close(a, b):
+    return float(((a.detach().cpu().double() - b).abs() / (1 + b.abs())).max()) <= 2e-4
+
+
+# the batches around which the pass changes (hidden 20, two blocks: 512 tiles of
+# 16 samples shared by a workgroup each, then a wavefront each), against the
+# FP64 oracle: FP32 products of up to a few hundred terms a layer, errors
+# growing a few-fold over the layers
+@pytest.mark.parametrize("n", [8192, 8193, 20000])
+@pytest.mark.parametrize("d", [5, 33, 70, 150])
+def test_passes_around_the_rule(gpu, d, n):
+    from oracle import realnvp as R
+
+    p = R.init_params(d, 2, 20, seed=d, scale=0.5, out_scale=1.0 / 20 ** 0.5)
+    p["data_mean"] = torch.linspace(-0.5, 0.5, d, dtype=torch.float64)
+    p["data_cov"] = torch.diag(torch.linspace(0.5, 1.5, d, dtype=torch.float64))
+    theta = R.to_flat(p).float()
+    m, p = RealNVP(d, 2, 20, fr.PRNGKey(0), _theta=theta), R.from_flat(theta.double(), d, 2, 20)
+    x = torch.randn(n, d, generator=torch.Generator().manual_seed(n + d))
+    for got, want in ((m.forward(x.cuda()), R.forward(p, x.double())), (m.inverse(x.cuda()), R.inverse(p, x.double()))):
+        assert _close(got[0], want[0]) and _close(got[1], want[1])
+    assert _close(m.log_prob(x.cuda()), R.log_prob(p, x.double()))
+
+
+@pytest.mark.parametrize("d,trans", [(40, 1), (40, 39), (40, 40), (40, 0), (130, 120), (130, 5)])
+def test_uneven_masks_a_wavefront_each(gpu, d, trans):
+    from flowmc_amd.resource.model.nf_model.realNVP import AffineCoupling
+    from oracle import realnvp as R
+
+    mask = torch.zeros(d)
+    mask[torch.randperm(d, generator=torch.Generator().manual_seed(trans))[:trans]] = 1.0  # 1 = transformed
+    layer = AffineCoupling(d, 20, mask, fr.PRNGKey(3), 0.5, scale=0.5)
+    x = torch.randn(9001, d, generator=torch.Generator().manual_seed(d))
+    y, ld = layer.forward(x.cuda())
+    lp = R.from_flat(layer.theta.cpu().double(), d, 1, 20)["layers"][0]
+    ry, rld = R.affine_coupling(lp, x.double(), 1 - mask.double(), dt=0.5)
+    assert _close(y, ry) and _close(ld, rld)
