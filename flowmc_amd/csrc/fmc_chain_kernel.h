@@ -31,23 +31,30 @@ enum KernelKind { KK_MALA = 0, KK_HMC = 1, KK_GRW = 2, KK_HMC_DENSE = 3 };
 // LPC): the target's value and gradient are inlined without a run-time
 // dispatch, and with LPC > 0 (the default layouts, workgroups of at most 256
 // threads) the group sums and broadcasts are straight-line DPP code and
-// parameters are always staged. LPC = 0 takes the lane count at run time, any
-// workgroup up to 1024 threads (HMC keeps position, momentum, gradient, metric
-// and the leapfrog copies in registers: bounded at 512 threads, which gives it
-// 256 VGPRs instead of 128, where NV >= 2 spilled) and parameters too large
-// for LDS.
+// parameters are always staged in rows. LPC_RUN takes the lane count at run time
+// and any workgroup up to 1024 threads (HMC keeps position, momentum, gradient,
+// metric and the leapfrog copies in registers: bounded at 512 threads, which gives
+// it 256 VGPRs instead of 128, where NV >= 2 spilled); four and more chunks a lane
+// in workgroups of at most 256 threads have a kernel of their own (LPC_RUN256),
+// which does not spill: 16 MALA steps of 2000
+// 1500-D Rosenbrock chains 425 -> 182 us, of 5000 600-D diagonal Gaussian ones
+// 204 -> 112.
+//
+// PAR: where the parameters are (a kernel for each: two or three copies of the
+// step loop in one kernel shared its registers, and the largest layouts spilled
+// more: MALA of a 600-D diagonal Gaussian took 1.5 times as long).
 //
 // RING: wavefront 0 advances the workgroup's 64 / lpc chains and the others
 // draw its random numbers, a block of steps ahead, into LDS (use_ring has
 // the rule).
-template <int NV, int KIND, int TK, int LPC, bool RING>
-__global__ void __launch_bounds__(LPC ? 256 : (KIND == KK_HMC || KIND == KK_HMC_DENSE) ? 512 : 1024)
+enum { LPC_RUN = 0, LPC_RUN256 = -1 };
+template <int NV, int KIND, int TK, int LPC, bool RING, int PAR>
+__global__ void __launch_bounds__(LPC != LPC_RUN ? 256 : (KIND == KK_HMC || KIND == KK_HMC_DENSE) ? 512 : 1024)
 chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg, int lpc_rt, int dp, NoiseRing nr) {
-  constexpr bool PARAMS = TK != FMC_TARGET_ROSENBROCK && TK != FMC_TARGET_FUNNEL;
-  const int lpc = LPC ? LPC : lpc_rt;
+  const int lpc = LPC > 0 ? LPC : lpc_rt;
   const TargetDev t{tg.kind, tg.n_dim, tg.n_modes, (gparam_t)tg.params, dp};
-  if (PARAMS && dp > 0) stage_target<TK>(t);
-  if (PARAMS && LPC == 0 && dp == STAGE_RAW) stage_raw(t, (int)target_param_count(TK, t.d, t.K));
+  if (PAR == PAR_ROWS) stage_target<TK>(t);
+  if (PAR == PAR_RAW) stage_raw(t, (int)target_param_count(TK, t.d, t.K));
   const int lane = threadIdx.x & 63;
   const int r = lane & (lpc - 1);
   const int gbase = lane - r;
@@ -69,32 +76,18 @@ chain_kernel(fmc_target tg, ChainIO io, StepCfg cfg, int lpc_rt, int dp, NoiseRi
     c = c0 + lane / lpc;
   }
   if (c >= io.C) return;  // whole group leaves together
-  auto run = [&](auto staged) {
-    constexpr int PAR = decltype(staged)::value;
-    using RG = std::conditional_t<TK == FMC_TARGET_GAUSS_DENSE && LPC == 1 && NV <= 2, DenseRegs<NV>, NoRegs>;
-    if constexpr (KIND == KK_MALA)
-      mala_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
-    else if constexpr (KIND == KK_GRW)
-      grw_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
-    else if constexpr (KIND == KK_HMC_DENSE)
-      hmc_group<NV, MK_DENSE, TK, PAR, NoRegs>(t, io, cfg, c, r, lpc, gbase);
-    else if (io.metric)
-      hmc_group<NV, MK_DIAG, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
-    else
-      hmc_group<NV, MK_UNIT, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
-  };
-  if constexpr (!PARAMS) {
-    run(std::integral_constant<int, PAR_MEM>{});
-  } else if constexpr (LPC > 0) {
-    run(std::integral_constant<int, PAR_ROWS>{});
-  } else {
-    if (dp > 0)
-      run(std::integral_constant<int, PAR_ROWS>{});
-    else if (dp == STAGE_RAW)
-      run(std::integral_constant<int, PAR_RAW>{});
-    else
-      run(std::integral_constant<int, PAR_MEM>{});
-  }
+  using RG = std::conditional_t<LPC <= 0, RunLanes,
+                                std::conditional_t<TK == FMC_TARGET_GAUSS_DENSE && LPC == 1 && NV <= 2, DenseRegs<NV>, NoRegs>>;
+  if constexpr (KIND == KK_MALA)
+    mala_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+  else if constexpr (KIND == KK_GRW)
+    grw_group<NV, TK, PAR, RING, RG>(t, io, cfg, nr, c, r, lpc, gbase);
+  else if constexpr (KIND == KK_HMC_DENSE)
+    hmc_group<NV, MK_DENSE, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
+  else if (io.metric)
+    hmc_group<NV, MK_DIAG, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
+  else
+    hmc_group<NV, MK_UNIT, TK, PAR, RG>(t, io, cfg, c, r, lpc, gbase);
 }
 
 // ----------------------------------------------------------- host side ----
@@ -158,6 +151,9 @@ static inline int check_layout(const Layout& L, int d) {
   return FMC_OK;
 }
 
+static inline bool raw_fits(const fmc_target* t) {
+  return target_param_count(t->kind, t->n_dim, t->n_modes) * 4 <= 48 * 1024;
+}
 // How a layout stages the parameters: the stride of rows padded to the lanes'
 // dims where they fit the 64 KB of LDS that need no attribute, STAGE_RAW where
 // only the unpadded block fits 48 KB (the rows are up to twice as long: d = 65
@@ -169,7 +165,24 @@ static inline int staged_stride(const fmc_target* t, const Layout& L) {
   const int64_t n = target_staged_count(t->kind, t->n_dim, t->n_modes, dp);
   if (n == 0) return STAGE_NONE;
   if (((n + 3) & ~3LL) * 4 <= 64 * 1024) return dp;
-  return target_param_count(t->kind, t->n_dim, t->n_modes) * 4 <= 48 * 1024 ? STAGE_RAW : STAGE_NONE;
+  return raw_fits(t) ? STAGE_RAW : STAGE_NONE;
+}
+// Where rows that are partly padding lose to the unpadded block: an explicit
+// layout of mostly idle lanes, or more workgroups than the rows leave room for on
+// the CUs (16 random-walk steps of 10,000 chains of a 300-D 8-mode mixture, 512
+// dims a row: 329 / 285 us; of 1000 chains 70 / 82). Never for a few hundred
+// floats (9 / 15 us a launch of a 100-D diagonal Gaussian over 256 dims) or, in
+// the explicit layout, few wavefronts (64-D 8-mode mixture over 256 dims, random
+// walks of 7 chains 35 / 58, of 1000 72 / 59).
+static inline bool idle_lanes(const fmc_target* t, const Layout& L, int dp, int64_t n) {
+  return t->kind != FMC_TARGET_GAUSS_DENSE && dp > 2 * t->n_dim + 8 && n * L.lpc > 64 * 256 &&
+         target_staged_count(t->kind, t->n_dim, t->n_modes, dp) > 1024;
+}
+static inline bool rows_cost_more(const fmc_target* t, const Layout& L, int dp, int64_t n) {
+  if (t->kind == FMC_TARGET_GAUSS_DENSE || 4 * dp <= 5 * t->n_dim) return false;
+  if (idle_lanes(t, L, dp, n)) return true;
+  const int64_t bytes = 4 * target_staged_count(t->kind, t->n_dim, t->n_modes, dp), per = L.block / L.lpc;
+  return bytes > 4096 && (n + per - 1) / per > 256 * (160 * 1024 / bytes);
 }
 static inline int staged_floats(const fmc_target* t, int dp) {
   if (dp == STAGE_NONE) return 0;
@@ -202,22 +215,69 @@ static bool use_ring(const ChainIO& io, const StepCfg& cfg, const Layout& L, int
          (io.C * L.lpc + 63) / 64 <= RING_MAX_WAVES && 4 * (size_t)staged + ring_bytes<NV>(L.lpc) <= RING_MAX_LDS;
 }
 
-template <int NV, int KIND, int TK, int LPC>
-static void launch_chain_lpc(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
+template <int NV, int KIND, int TK, int LPC, int PAR>
+static void launch_chain_par(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
                              const Layout& L, int dp) {
   const int nf = staged_floats(t, dp);
   const NoiseRing nr{nf, cfg.n_steps};
   if constexpr (LPC > 0 && (KIND == KK_MALA || KIND == KK_GRW)) {
     if (use_ring<NV>(io, cfg, L, nf)) {
       const int per_block = 64 / LPC;
-      hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, true>), dim3((unsigned)((io.C + per_block - 1) / per_block)),
-                         dim3(256), 4 * (size_t)nf + ring_bytes<NV>(LPC), st, *t, io, cfg, L.lpc, dp, nr);
+      hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, true, PAR>),
+                         dim3((unsigned)((io.C + per_block - 1) / per_block)), dim3(256),
+                         4 * (size_t)nf + ring_bytes<NV>(LPC), st, *t, io, cfg, L.lpc, dp, nr);
       return;
     }
   }
   const int per_block = L.block / L.lpc;
-  hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, false>), dim3((unsigned)((io.C + per_block - 1) / per_block)),
+  hipLaunchKernelGGL((chain_kernel<NV, KIND, TK, LPC, false, PAR>), dim3((unsigned)((io.C + per_block - 1) / per_block)),
                      dim3((unsigned)L.block), 4 * (size_t)nf, st, *t, io, cfg, L.lpc, dp, nr);
+}
+
+// (LPC > 0: parameters are staged in rows, if the target has any)
+template <int NV, int KIND, int TK, int LPC>
+static void launch_chain_lpc(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
+                             const Layout& L, int dp) {
+  if constexpr (TK == FMC_TARGET_ROSENBROCK || TK == FMC_TARGET_FUNNEL) {
+    launch_chain_par<NV, KIND, TK, LPC, PAR_MEM>(st, t, io, cfg, L, dp);
+  } else if constexpr (LPC > 0) {
+    launch_chain_par<NV, KIND, TK, LPC, PAR_ROWS>(st, t, io, cfg, L, dp);
+  } else {
+    // (the rows' loads move out of the step loop, and the 1024-thread kernels
+    // that hold most else have no registers for them: MALA of a 600-D diagonal
+    // Gaussian, four chunks, 201 us, unpadded 117; random-walk steps of a 1500-D
+    // one, eight, 149 / 95)
+    constexpr bool ROWS = LPC == LPC_RUN256 || TK == FMC_TARGET_GAUSS_DENSE || KIND == KK_HMC || KIND == KK_HMC_DENSE ||
+                          NV < 4 || (NV == 4) == (KIND == KK_GRW);
+    if (dp > 0 && (!ROWS || rows_cost_more(t, L, dp, io.C))) dp = raw_fits(t) ? STAGE_RAW : ROWS ? dp : STAGE_NONE;
+    if constexpr (ROWS) {
+      if (dp > 0) {
+        launch_chain_par<NV, KIND, TK, LPC, PAR_ROWS>(st, t, io, cfg, L, dp);
+        return;
+      }
+    }
+    if (dp == STAGE_RAW)
+      launch_chain_par<NV, KIND, TK, LPC, PAR_RAW>(st, t, io, cfg, L, dp);
+    else
+      launch_chain_par<NV, KIND, TK, LPC, PAR_MEM>(st, t, io, cfg, L, dp);
+  }
+}
+
+// Four and eight chunks a lane: workgroups of at most 256 threads without spills
+// where that pays, MALA and, at eight, random-walk steps (random-walk steps of
+// 5000 600-D diagonal Gaussian chains, four chunks, 75 -> 82 us; HMC and a dense
+// precision need the second wavefront on a SIMD more: HMC of 2000 1500-D Rosenbrock
+// chains 107 -> 158 us).
+template <int NV, int KIND, int TK>
+static void launch_chain_wide(hipStream_t st, const fmc_target* t, const ChainIO& io, const StepCfg& cfg,
+                              const Layout& L, int dp) {
+  if constexpr ((KIND == KK_MALA || (KIND == KK_GRW && NV == 8)) && TK != FMC_TARGET_GAUSS_DENSE) {
+    if (L.block <= 256) {
+      launch_chain_lpc<NV, KIND, TK, LPC_RUN256>(st, t, io, cfg, L, dp);
+      return;
+    }
+  }
+  launch_chain_lpc<NV, KIND, TK, LPC_RUN>(st, t, io, cfg, L, dp);
 }
 
 // The kernels specialised on their lane count: the layouts choose_layout gives
@@ -227,7 +287,8 @@ static void launch_chain_kind(hipStream_t st, const fmc_target* t, const ChainIO
                               const Layout& L) {
   const int dp = staged_stride(t, L);
   if constexpr (KIND != KK_HMC_DENSE) {
-    const bool staged = dp > 0 || TK == FMC_TARGET_ROSENBROCK || TK == FMC_TARGET_FUNNEL;
+    // (an explicit layout of mostly idle lanes stages its parameters unpadded)
+    const bool staged = TK == FMC_TARGET_ROSENBROCK || TK == FMC_TARGET_FUNNEL || (dp > 0 && !idle_lanes(t, L, dp, io.C));
     if (staged && L.block <= 256) {
 #define FMC_LPC(NV_, LPC_)                                                      \
   case LPC_:                                                                    \
@@ -268,10 +329,10 @@ static void launch_chain_kind(hipStream_t st, const fmc_target* t, const ChainIO
     }
   }
   switch (L.nv) {
-    case 1: launch_chain_lpc<1, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
-    case 2: launch_chain_lpc<2, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
-    case 4: launch_chain_lpc<4, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
-    default: launch_chain_lpc<8, KIND, TK, 0>(st, t, io, cfg, L, dp); break;
+    case 1: launch_chain_lpc<1, KIND, TK, LPC_RUN>(st, t, io, cfg, L, dp); break;
+    case 2: launch_chain_lpc<2, KIND, TK, LPC_RUN>(st, t, io, cfg, L, dp); break;
+    case 4: launch_chain_wide<4, KIND, TK>(st, t, io, cfg, L, dp); break;
+    default: launch_chain_wide<8, KIND, TK>(st, t, io, cfg, L, dp); break;
   }
 }
 

@@ -371,7 +371,7 @@ __device__ __forceinline__ void dense_momentum(const float* __restrict__ Lc, int
   }
 }
 
-template <int NV, int MK, int TK, int PAR = PAR_MEM, class RG = NoRegs>
+template <int NV, int MK, int TK, int PAR, class RG>
 __device__ __forceinline__ void hmc_group(const TargetDev& t, const ChainIO& io, const StepCfg& cfg, int64_t c,
                           int r, int lpc, int gbase) {
   constexpr bool UNIT_M = MK == MK_UNIT;

@@ -38,11 +38,11 @@ __global__ void __launch_bounds__(512) hmc_batched_kernel(const fmc_hmc_slot* __
              sl.out_acc,  sl.n_chains, sl.buf_len, sl.cursor, sl.key0,   sl.key1};
   io.chol = sl.momentum_chol;
   if (io.chol)
-    hmc_group<NV, MK_DENSE, -1>(t, io, cfg, c, r, lpc, gbase);
+    hmc_group<NV, MK_DENSE, -1, PAR_MEM, RunLanes>(t, io, cfg, c, r, lpc, gbase);
   else if (io.metric)
-    hmc_group<NV, MK_DIAG, -1>(t, io, cfg, c, r, lpc, gbase);
+    hmc_group<NV, MK_DIAG, -1, PAR_MEM, RunLanes>(t, io, cfg, c, r, lpc, gbase);
   else
-    hmc_group<NV, MK_UNIT, -1>(t, io, cfg, c, r, lpc, gbase);
+    hmc_group<NV, MK_UNIT, -1, PAR_MEM, RunLanes>(t, io, cfg, c, r, lpc, gbase);
 }
 
 // Homogeneous unit-metric batches (every slot holds the same target kind TK
@@ -65,7 +65,7 @@ __device__ __forceinline__ void hmc_unit_fixed(const fmc_work_item& it, const fm
   TargetDev t{TK, sl.target.n_dim, sl.target.n_modes, (gparam_t)sl.target.params, 0};
   ChainIO io{sl.x,        sl.logp,     nullptr,    sl.noise,  sl.log_u,  sl.out_pos, sl.out_logp,
              sl.out_acc,  sl.n_chains, sl.buf_len, sl.cursor, sl.key0,   sl.key1};
-  hmc_group<NV, MK_UNIT, TK>(t, io, cfg, c, r, LPC, gbase);
+  hmc_group<NV, MK_UNIT, TK, PAR_MEM, NoRegs>(t, io, cfg, c, r, LPC, gbase);
 }
 
 template <int NV, int TK>

@@ -101,11 +101,15 @@ struct DenseRegs {
 struct NoRegs {
   __device__ __forceinline__ explicit NoRegs(const TargetDev&) {}
 };
+// ... and a lane count that is known at run time only
+struct RunLanes {
+  __device__ __forceinline__ explicit RunLanes(const TargetDev&) {}
+};
 
 template <int NV, int PAR, class RG>
 __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                                  float4 (&g)[NV], int r, int lpc, int gbase) {
-  constexpr bool REG = !std::is_same<RG, NoRegs>::value;
+  constexpr bool REG = std::is_same<RG, DenseRegs<NV>>::value;
   const int d = t.d;
   float4 y[NV];
 #pragma unroll
@@ -131,8 +135,10 @@ __device__ __forceinline__ float tgt_gauss_dense(const TargetDev& t, const RG& r
       for (int e2 = 0; e2 < 4; ++e2) {
         const int j2 = REG ? 4 * v2 + e2 : dim_of(v2, e2, s, lpc);
         // (in registers by two columns: a zero column costs less than its test)
+        float ys = 0.f;  // (from memory the shuffle ahead of the test: HMC, d = 200, 13.2 / 12.6 ms)
+        if (PAR == PAR_MEM) ys = __shfl(f4c(y[v2], e2), gbase + s, 64);
         if ((REG ? j2 & ~1 : j2) < d) {
-          const float ys = (REG || lpc == 1) ? f4c(y[v2], e2) : __shfl(f4c(y[v2], e2), gbase + s, 64);
+          if (PAR != PAR_MEM) ys = (REG || lpc == 1) ? f4c(y[v2], e2) : __shfl(f4c(y[v2], e2), gbase + s, 64);
 #pragma unroll
           for (int v = 0; v < NV; ++v) {
             float4 p4;
@@ -187,7 +193,9 @@ __device__ __forceinline__ float group_last_to_first(float v, int lpc) {
 }
 
 // log p = -scale * sum_{i<d-1} [100 (x_{i+1} - x_i^2)^2 + (1 - x_i)^2]
-template <int NV>
+// RUN: a run-time lane count reads its neighbours by shuffles (a branch on it
+// for each read made HMC of d = 700 up to 1.2 times slower)
+template <int NV, bool RUN>
 __device__ __forceinline__ float tgt_rosenbrock(const TargetDev& t, const float4 (&x)[NV],
                                                 float4 (&g)[NV], int r, int lpc, int gbase) {
   const float scale = t.p[0];
@@ -196,10 +204,11 @@ __device__ __forceinline__ float tgt_rosenbrock(const TargetDev& t, const float4
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     // x_{j+1} for element 3 and x_{j-1} for element 0 live in neighbouring lanes.
-    float nx_same = lane_next(x[v].x, lpc);
+    float nx_same = RUN ? __shfl(x[v].x, gbase + ((r + 1) & (lpc - 1)), 64) : lane_next(x[v].x, lpc);
     float nx_next = group_bcast0(x[(v + 1 < NV) ? v + 1 : v].x, lpc);
-    float pw_same = lane_prev(x[v].w, lpc);
-    float pw_prev = group_last_to_first(x[(v > 0) ? v - 1 : 0].w, lpc);
+    float pw_same = RUN ? __shfl(x[v].w, gbase + ((r - 1) & (lpc - 1)), 64) : lane_prev(x[v].w, lpc);
+    const float last = x[(v > 0) ? v - 1 : 0].w;
+    float pw_prev = RUN ? __shfl(last, gbase + lpc - 1, 64) : group_last_to_first(last, lpc);
     float nxt3 = (r < lpc - 1) ? nx_same : nx_next;
     float prv0 = (r > 0) ? pw_same : pw_prev;
 #pragma unroll
@@ -274,68 +283,110 @@ __device__ __forceinline__ float tgt_gmm_diag(const TargetDev& t, const float4 (
   for (int v = 0; v < NV; ++v) g[v] = make_float4(0.f, 0.f, 0.f, 0.f);
   // U modes' quadratic forms at once: their loads and sums over the lanes overlap
   constexpr int U = PAR != PAR_MEM && NV <= 2 ? 2 : 1;
-  for (int k0 = 0; k0 < K; k0 += U) {
-    float4 z[U][NV], i4[U][NV];
-    float qs[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u < K ? k0 + u : k0;
+  if constexpr (U == 1) {
+    // many chunks a lane, or parameters in memory: one mode at a time, its
+    // gradient the only copy of it (the form above took twice the registers and
+    // spilled: MALA of a 1100-D mixture 2.0 times as long), a branch on the chain
+    for (int k = 0; k < K; ++k) {
+      float4 gk[NV];
       float q = 0.f;
 #pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        float4 m4;
-        if (PAR == PAR_ROWS) {
-          m4 = staged4(k * t.dp + dim_of(v, 0, r, lpc));
-          i4[u][v] = staged4(o_is + k * t.dp + dim_of(v, 0, r, lpc));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int j = dim_of(v, e, r, lpc);
-            f4(m4, e) = j < d ? param<PAR>(t, (int64_t)k * d + j) : 0.f;
-            f4(i4[u][v], e) = j < d ? param<PAR>(t, (int64_t)(K + k) * d + j) : 0.f;
-          }
-        }
+      for (int v = 0; v < NV; ++v)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          f4(z[u][v], e) = (f4c(x[v], e) - f4c(m4, e)) * f4c(i4[u][v], e);
-          q = fmaf(f4c(z[u][v], e), f4c(z[u][v], e), q);
+          const int j = dim_of(v, e, r, lpc);
+          float gj = 0.f;
+          if (PAR == PAR_ROWS || j < d) {
+            const float is = PAR == PAR_ROWS ? fmc_chain_lds[o_is + k * t.dp + j] : param<PAR>(t, (int64_t)(K + k) * d + j);
+            const float mu = PAR == PAR_ROWS ? fmc_chain_lds[k * t.dp + j] : param<PAR>(t, (int64_t)k * d + j);
+            const float z = (f4c(x[v], e) - mu) * is;
+            q = fmaf(z, z, q);
+            gj = -z * is;
+          }
+          f4(gk[v], e) = gj;
         }
-      }
-      qs[u] = q;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u < K ? k0 + u : k0;
-      qs[u] = fmaf(-0.5f, group_sum(qs[u], lpc), PAR == PAR_ROWS ? fmc_chain_lds[o_c + k] : param<PAR>(t, 2 * (int64_t)K * d + k));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (k0 + u >= K) break;
-      const float q = qs[u];
-      const bool top = q > m;
-      const float a = fabsf(q - m);
-      // (expf gives 0 below -103.97; not for a NaN)
-      if (__builtin_amdgcn_ballot_w64(!(a > 104.f)) == 0) {
-        if (__builtin_amdgcn_ballot_w64(top) != 0) {
-          sw = top ? 1.f : sw;
-#pragma unroll
-          for (int v = 0; v < NV; ++v)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              f4(g[v], e) = top ? -f4c(z[u][v], e) * f4c(i4[u][v], e) : f4c(g[v], e);
-          m = top ? q : m;
-        }
-      } else {
-        const float w = expf(-a);
-        sw = fmaf(top ? sw : 1.f, w, top ? 1.f : sw);
+      q = fmaf(-0.5f, group_sum(q, lpc), PAR == PAR_ROWS ? fmc_chain_lds[o_c + k] : param<PAR>(t, 2 * (int64_t)K * d + k));
+      if (q > m) {  // (q is bitwise equal across the group)
+        const float sc = expf(m - q);
+        sw = fmaf(sw, sc, 1.f);
 #pragma unroll
         for (int v = 0; v < NV; ++v)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float gk = -f4c(z[u][v], e) * f4c(i4[u][v], e);
-            f4(g[v], e) = fmaf(top ? f4c(g[v], e) : gk, w, top ? gk : f4c(g[v], e));
+          for (int e = 0; e < 4; ++e) f4(g[v], e) = fmaf(f4c(g[v], e), sc, f4c(gk[v], e));
+        m = q;
+      } else {
+        const float w = expf(q - m);
+        sw += w;
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f4(g[v], e) = fmaf(w, f4c(gk[v], e), f4c(g[v], e));
+      }
+    }
+  } else {
+    for (int k0 = 0; k0 < K; k0 += U) {
+      float4 z[U][NV], i4[U][NV];
+      float qs[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u < K ? k0 + u : k0;
+        float q = 0.f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          float4 m4;
+          if (PAR == PAR_ROWS) {
+            m4 = staged4(k * t.dp + dim_of(v, 0, r, lpc));
+            i4[u][v] = staged4(o_is + k * t.dp + dim_of(v, 0, r, lpc));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int j = dim_of(v, e, r, lpc);
+              f4(m4, e) = j < d ? param<PAR>(t, (int64_t)k * d + j) : 0.f;
+              f4(i4[u][v], e) = j < d ? param<PAR>(t, (int64_t)(K + k) * d + j) : 0.f;
+            }
           }
-        m = top ? q : m;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            f4(z[u][v], e) = (f4c(x[v], e) - f4c(m4, e)) * f4c(i4[u][v], e);
+            q = fmaf(f4c(z[u][v], e), f4c(z[u][v], e), q);
+          }
+        }
+        qs[u] = q;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u < K ? k0 + u : k0;
+        qs[u] = fmaf(-0.5f, group_sum(qs[u], lpc), PAR == PAR_ROWS ? fmc_chain_lds[o_c + k] : param<PAR>(t, 2 * (int64_t)K * d + k));
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (k0 + u >= K) break;
+        const float q = qs[u];
+        const bool top = q > m;
+        const float a = fabsf(q - m);
+        // (expf gives 0 below -103.97; not for a NaN)
+        if (__builtin_amdgcn_ballot_w64(!(a > 104.f)) == 0) {
+          if (__builtin_amdgcn_ballot_w64(top) != 0) {
+            sw = top ? 1.f : sw;
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                f4(g[v], e) = top ? -f4c(z[u][v], e) * f4c(i4[u][v], e) : f4c(g[v], e);
+            m = top ? q : m;
+          }
+        } else {
+          const float w = expf(-a);
+          sw = fmaf(top ? sw : 1.f, w, top ? 1.f : sw);
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float gk = -f4c(z[u][v], e) * f4c(i4[u][v], e);
+              f4(g[v], e) = fmaf(top ? f4c(g[v], e) : gk, w, top ? gk : f4c(g[v], e));
+            }
+          m = top ? q : m;
+        }
       }
     }
   }
@@ -413,7 +464,8 @@ __device__ __forceinline__ float tgt_dual_moon(const TargetDev& t, const float4 
 // TK >= 0: the kind is fixed at compile time (one target per kernel);
 // TK = -1: dispatch on t.kind at run time. PAR: where the parameters are
 // (stage_target, stage_raw).
-// RG: parameters held in registers (DenseRegs), or NoRegs.
+// RG: parameters held in registers (DenseRegs), or NoRegs; RunLanes where lpc
+// is no compile-time constant.
 template <int NV, int TK, int PAR, bool ENTRY, class RG>
 __device__ __forceinline__ float target_vg(const TargetDev& t, const RG& rg, const float4 (&x)[NV],
                                            float4 (&g)[NV], int r, int lpc, int gbase) {
@@ -423,7 +475,7 @@ __device__ __forceinline__ float target_vg(const TargetDev& t, const RG& rg, con
     case FMC_TARGET_GAUSS_DENSE:
       return tgt_gauss_dense<NV, PAR>(t, rg, x, g, r, lpc, gbase);
     case FMC_TARGET_ROSENBROCK:
-      return tgt_rosenbrock<NV>(t, x, g, r, lpc, gbase);
+      return tgt_rosenbrock<NV, std::is_same<RG, RunLanes>::value>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_FUNNEL:
       return tgt_funnel<NV, ENTRY>(t, x, g, r, lpc, gbase);
     case FMC_TARGET_GMM_DIAG:
@@ -451,8 +503,9 @@ __device__ __forceinline__ void stage_target(const TargetDev& t) {
   const int d = t.d, dp = t.dp;
   const int rows = TK == FMC_TARGET_GAUSS_DIAG ? 2 : TK == FMC_TARGET_GAUSS_DENSE ? d + 1
                    : TK == FMC_TARGET_GMM_DIAG ? 2 * t.K : TK == FMC_TARGET_DUAL_MOON ? 1 : 0;
+  const int sh = __builtin_ctz(dp);  // (a power of two)
   for (int i = threadIdx.x; i < rows * dp; i += blockDim.x) {
-    const int w = i / dp, j = i - w * dp;
+    const int w = i >> sh, j = i & (dp - 1);
     float v = 0.f;
     if (j < d) v = (TK == FMC_TARGET_GAUSS_DENSE && w > 0) ? t.p[d + (int64_t)j * d + (w - 1)] : t.p[(int64_t)w * d + j];
     fmc_chain_lds[i] = v;
