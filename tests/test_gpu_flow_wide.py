@@ -56,3 +56,20 @@ def test_wide_pass_rows_match_the_general_pass(gpu, direction, flags, draws, d, 
         ys, ls = _pass(m, direction, flags, None if draws else x[a:a + SMALL].contiguous(), SMALL, d, a)
         assert torch.equal(y[a:a + SMALL], ys)
         assert ((ld[a:a + SMALL] - ls).abs() <= 2.0 ** -24 * 10 * d * (layers + 1)).all()
+
+
+# n at the rounds in which 256 CUs take a call (96 samples a CU in the general
+# pass, 128 in the wide one), for conditioners on either side of each rule
+@pytest.mark.parametrize("n", [24576, 24577, 32768, 32769, 49153, 73729])
+@pytest.mark.parametrize("d,layers,hidden,bins", [
+    (2, 2, [32, 32], 8), (33, 2, [128, 256, 64, 32], 8), (7, 2, [64], 10), (16, 2, [100, 70], 5), (8, 2, [256], 8),
+])
+@pytest.mark.parametrize("direction,flags,draws", [(0, 3, False), (2, 7, True)])
+def test_rows_around_the_rounds_match_small_calls(gpu, direction, flags, draws, d, layers, hidden, bins, n):
+    m = _model(d, layers, hidden, bins)
+    x = None if draws else 3 * torch.randn(n, d, generator=torch.Generator().manual_seed(n)).cuda()
+    y, ld = _pass(m, direction, flags, x, n, d)
+    for a in (0, n // 2, n - SMALL):
+        ys, ls = _pass(m, direction, flags, None if draws else x[a:a + SMALL].contiguous(), SMALL, d, a)
+        assert torch.equal(y[a:a + SMALL], ys)
+        assert ((ld[a:a + SMALL] - ls).abs() <= 2.0 ** -24 * 10 * d * (layers + 1)).all()
