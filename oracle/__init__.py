@@ -4,7 +4,7 @@ This package restates, in FP64 on the CPU (torch for autograd, numpy for
 integer RNG arithmetic), the reference algorithms that the HIP kernels of
 ``flowmc_amd`` replace. Each function cites the flowMC v0.4.5 file:line it
 follows. It is imported only by ``tests/``, ``__graft_entry__.smoke()`` and
-the ``cpu_baseline`` leg of ``bench.py`` — as the checker / CPU baseline,
+the ``cpu_baseline`` leg of ``bench.py`` — as the oracle and the CPU baseline,
 never as a product code path.
 
 Pinning (what independently checks each function; see tests/test_oracle_*.py):
